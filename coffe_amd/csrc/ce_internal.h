@@ -168,7 +168,7 @@ int ce_launch_divergent(void *stream, const double *d_k, const double *d_pk, int
 size_t ce_cov_lds_bytes(int N);
 int ce_launch_cov_ahat(void *stream, int nl, int N, const ce_radix_plan *rp, const double *d_tw, const double *d_A,
                        double *d_ahat);
-int ce_launch_cov_diag(void *stream, int nspec, int N, const int64_t *d_in_off, const int32_t *d_n_in,
+int ce_launch_cov_diag(void *stream, int nspec, int N, int ld, int frag, const int64_t *d_in_off, const int32_t *d_n_in,
                        const double *d_k, const double *d_pk, const double *d_kg, const double *d_k3,
                        const double *d_kn1, const double *d_kn2, double step, double *d_d, int *d_status);
 int ce_launch_cov_rows(void *stream, int nblk, int N, const ce_radix_plan *rpN, const ce_radix_plan *rpM,
@@ -176,17 +176,35 @@ int ce_launch_cov_rows(void *stream, int nblk, int N, const ce_radix_plan *rpN, 
                        const int *d_pl1, const int *d_pl2, int nrows, const int *d_rows, const double *d_prn1,
                        const double *d_prn2, int R, const int *d_flo, const int *d_fcnt, const int *d_foff,
                        const double *d_fw, double *d_W);
-/* the adjoint of coffe_cov_integrals: d_gint -> d_gpk (zeroed here), workspaces
-   d_Wbar [2 nspec][npair][nrows][R] and d_dbar [nspec][2][N] */
-int ce_launch_cov_vjp(void *stream, int nspec, int N, const ce_radix_plan *rpN, const ce_radix_plan *rpM,
-                      const double *d_tw, const double *d_ahat, const double *d_B, int npair, const int *d_pl1,
-                      const int *d_pl2, int nrows, const int *d_rows, const double *d_prn1, int R, const int *d_flo,
-                      const int *d_fcnt, const int *d_foff, const double *d_fws, const int *d_upos,
-                      const int *d_uelo, const int *d_uehi,
-                      const double *d_fw, const double *d_fac, const double *d_gint, double *d_Wbar, double *d_dbar,
-                      const int64_t *d_in_off, const int32_t *d_n_in, const double *d_k, const double *d_pk,
-                      const double *d_kg, const double *d_k3, const double *d_kn1, const double *d_kn2, double step,
-                      double *d_gpk, int64_t n_total);
+/* the adjoint of coffe_cov_integrals' transforms, gint -> dbar [nspec][2][N] (workspace d_Wbar
+   [2 nspec][npair][nrows][R]), and of its diagonals, dbar -> d_gpk (zeroed here) */
+int ce_launch_cov_rows_vjp(void *stream, int nspec, int N, const ce_radix_plan *rpN, const ce_radix_plan *rpM,
+                           const double *d_tw, const double *d_ahat, const double *d_B, int npair, const int *d_pl1,
+                           const int *d_pl2, int nrows, const int *d_rows, const double *d_prn1, int R,
+                           const int *d_flo, const int *d_fcnt, const int *d_foff, const double *d_fws,
+                           const int *d_upos, const int *d_uelo, const int *d_uehi, const double *d_fw,
+                           const double *d_fac, const double *d_gint, double *d_Wbar, double *d_dbar);
+int ce_launch_cov_diag_vjp(void *stream, int nspec, int N, const double *d_dbar, const int64_t *d_in_off,
+                           const int32_t *d_n_in, const double *d_k, const double *d_pk, const double *d_kg,
+                           const double *d_k3, const double *d_kn1, const double *d_kn2, double step, double *d_gpk,
+                           int64_t n_total);
+/* the integrals as contractions over k (cov_contract.hip): tables of nl 4 Rp Np doubles (Rp, Np: R
+   and N rounded up to 16) and diagonals, nblk = 2 nspec rounded up to 16 of Np each, in
+   fragments; the adjoint reads the tables as plain rows (cov_unfold).  Splits of the
+   contracted range: d_part holds that many times the output (unused with one split), the
+   adjoint's [splits][nblk][Np] */
+int ce_launch_cov_fold(void *stream, int nl, int N, int Np, int R, int Rp, const double *d_ahat, const double *d_bhat,
+                       const int *d_lo, const int *d_cnt, const int *d_off, const double *d_uw, const double *d_fws,
+                       const double *d_prn, double *d_tab);
+int ce_launch_cov_unfold(void *stream, int nl, int Np, int Rp, const double *d_tab, double *d_rows);
+int ce_cov_contract_splits(int nblk, int npair, int R, int Np);
+int ce_cov_contract_splits_T(int nblk, int npair, int R, int Np);
+int ce_launch_cov_contract(void *stream, int nblk, int Np, int R, int npair, const int *d_pl1, const int *d_pl2,
+                           const double *d_tab, const double *d_d, const double *d_fac, int nsplit, double *d_part,
+                           double *d_out);
+int ce_launch_cov_contract_T(void *stream, int nblk, int N, int Np, int R, int npair, const int *d_pl1,
+                             const int *d_pl2, const double *d_tab, const double *d_gint, const double *d_fac,
+                             int nsplit, double *d_part, double *d_dbar);
 int ce_launch_cov_cols(void *stream, int nspec, int npair, int nrows, int R, const int *d_upos, const int *d_ucnt,
                        const int *d_uoff, const double *d_uw, const double *d_fac, const double *d_W, double *d_out);
 int ce_launch_cov_assemble(void *stream, int nspec, int nz, int nl, int R, int npair, const int *d_ls,

@@ -54,7 +54,8 @@ __global__ void __launch_bounds__(1024) k_cov_ahat(int N, ce_radix_plan rp, cons
 }
 
 struct diag_args {
-    int N;
+    int N, ld;               // ld: stride of the diagonals, zeros above N
+    int frag;                // store fragments (cov_contract.hip) of 16 diagonals x 16 t
     const int64_t *in_off;   // [nspec]
     const int32_t *n_in;     // [nspec]
     const double *k, *p;     // concatenated spectra
@@ -62,7 +63,7 @@ struct diag_args {
     const double *k3;        // k_t^3
     const double *kn1, *kn2; // k_t^nu1, k_t^nu2
     double step;
-    double *d;               // [nspec][2][N]
+    double *d;               // [nspec][2][ld]
     int *status;
 };
 
@@ -70,15 +71,25 @@ __global__ void __launch_bounds__(256) k_cov_diag(diag_args a)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int s = blockIdx.y;
-    if (t >= a.N) return;
+    if (t >= a.ld) return;
+    double *o = a.d + (int64_t)s * 2 * a.ld + t;   // and the second power's, o2 elements on
+    int64_t o2 = a.ld;
+    if (a.frag) {
+        o = a.d + ((int64_t)(s >> 3) * (a.ld / 16) + (t >> 4)) * 256 + ((t >> 1) & 1) * 128 +
+            (((t >> 2) & 3) * 16 + 2 * (s & 7)) * 2 + (t & 1);
+        o2 = 2;
+    }
+    if (t >= a.N) {
+        o[0] = o[o2] = 0.0;
+        return;
+    }
     const int64_t off = a.in_off[s];
     const double P = ce::akima_general(a.k + off, a.p + off, a.n_in[s], a.kg[t]);
     // fk = k^3 P^power / dlnk, then / k^nu1 / k^nu2 (covariance.c:391-403, twobessel.c:49-55)
     const double d1 = a.k3[t] * P / a.step / a.kn1[t] / a.kn2[t];
     const double d2 = a.k3[t] * (P * P) / a.step / a.kn1[t] / a.kn2[t];
-    double *o = a.d + (int64_t)s * 2 * a.N;
-    o[t] = d1;
-    o[a.N + t] = d2;
+    o[0] = d1;
+    o[o2] = d2;
     if (!isfinite(d1) || !isfinite(d2)) a.status[0] = 1;
 }
 
@@ -644,15 +655,15 @@ extern "C" int ce_launch_cov_ahat(void *stream, int nl, int N, const ce_radix_pl
     return (int)hipGetLastError();
 }
 
-extern "C" int ce_launch_cov_diag(void *stream, int nspec, int N, const int64_t *d_in_off, const int32_t *d_n_in,
-                                  const double *d_k, const double *d_pk, const double *d_kg, const double *d_k3,
+extern "C" int ce_launch_cov_diag(void *stream, int nspec, int N, int ld, int frag, const int64_t *d_in_off,
+                                  const int32_t *d_n_in, const double *d_k, const double *d_pk, const double *d_kg, const double *d_k3,
                                   const double *d_kn1, const double *d_kn2, double step, double *d_d, int *d_status)
 {
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, (hipStream_t)stream, d_status, 1, 0);
     diag_args a;
-    a.N = N; a.in_off = d_in_off; a.n_in = d_n_in; a.k = d_k; a.p = d_pk; a.kg = d_kg; a.k3 = d_k3;
+    a.N = N; a.ld = ld; a.frag = frag; a.in_off = d_in_off; a.n_in = d_n_in; a.k = d_k; a.p = d_pk; a.kg = d_kg; a.k3 = d_k3;
     a.kn1 = d_kn1; a.kn2 = d_kn2; a.step = step; a.d = d_d; a.status = d_status;
-    hipLaunchKernelGGL(k_cov_diag, dim3((N + 255) / 256, nspec), dim3(256), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(k_cov_diag, dim3((ld + 255) / 256, nspec), dim3(256), 0, (hipStream_t)stream, a);
     return (int)hipGetLastError();
 }
 
@@ -809,16 +820,14 @@ extern "C" int ce_launch_cov_assemble_vjp(void *stream, int nspec, int nz, int n
     return (int)hipGetLastError();
 }
 
-extern "C" int ce_launch_cov_vjp(void *stream, int nspec, int N, const ce_radix_plan *rpN, const ce_radix_plan *rpM,
-                                 const double *d_tw, const double *d_ahat, const double *d_B, int npair,
-                                 const int *d_pl1, const int *d_pl2, int nrows, const int *d_rows,
-                                 const double *d_prn1, int R, const int *d_flo, const int *d_fcnt, const int *d_foff,
-                                 const double *d_fws, const int *d_upos, const int *d_uelo, const int *d_uehi,
-                                 const double *d_fw, const double *d_fac,
-                                 const double *d_gint, double *d_Wbar, double *d_dbar, const int64_t *d_in_off,
-                                 const int32_t *d_n_in, const double *d_k, const double *d_pk, const double *d_kg,
-                                 const double *d_k3, const double *d_kn1, const double *d_kn2, double step,
-                                 double *d_gpk, int64_t n_total)
+/* dbar of the transforms (rows path): gint -> dbar */
+extern "C" int ce_launch_cov_rows_vjp(void *stream, int nspec, int N, const ce_radix_plan *rpN,
+                                      const ce_radix_plan *rpM, const double *d_tw, const double *d_ahat,
+                                      const double *d_B, int npair, const int *d_pl1, const int *d_pl2, int nrows,
+                                      const int *d_rows, const double *d_prn1, int R, const int *d_flo,
+                                      const int *d_fcnt, const int *d_foff, const double *d_fws, const int *d_upos,
+                                      const int *d_uelo, const int *d_uehi, const double *d_fw, const double *d_fac,
+                                      const double *d_gint, double *d_Wbar, double *d_dbar)
 {
     if (N > CE_ROWS_T_ACC * 1024) return (int)hipErrorInvalidValue;
     hipStream_t s = (hipStream_t)stream;
@@ -830,7 +839,6 @@ extern "C" int ce_launch_cov_vjp(void *stream, int nspec, int N, const ce_radix_
                        s, c);
     const int64_t nd = (int64_t)2 * nspec * N;
     hipLaunchKernelGGL(k_fill_double, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, s, d_dbar, nd, 0.0);
-    hipLaunchKernelGGL(k_fill_double, dim3((unsigned)((n_total + 255) / 256)), dim3(256), 0, s, d_gpk, n_total, 0.0);
     const size_t lds = ce_cov_lds_bytes(N);
     int st = set_lds((const void *)k_cov_rows_T, lds);
     if (st) return st;
@@ -847,6 +855,17 @@ extern "C" int ce_launch_cov_vjp(void *stream, int nspec, int N, const ce_radix_
     a.chunk = (nrows + nchunk - 1) / nchunk;
     const int grid_x = (nrows + a.chunk - 1) / a.chunk;
     hipLaunchKernelGGL(k_cov_rows_T, dim3(grid_x, npair, 2 * nspec), dim3(1024), lds, s, a);
+    return (int)hipGetLastError();
+}
+
+/* dbar -> d_gpk (zeroed here) through the diagonals and the Akima spline */
+extern "C" int ce_launch_cov_diag_vjp(void *stream, int nspec, int N, const double *d_dbar, const int64_t *d_in_off,
+                                      const int32_t *d_n_in, const double *d_k, const double *d_pk,
+                                      const double *d_kg, const double *d_k3, const double *d_kn1,
+                                      const double *d_kn2, double step, double *d_gpk, int64_t n_total)
+{
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(k_fill_double, dim3((unsigned)((n_total + 255) / 256)), dim3(256), 0, s, d_gpk, n_total, 0.0);
     diagT_args d;
     d.N = N; d.in_off = d_in_off; d.n_in = d_n_in; d.k = d_k; d.p = d_pk; d.kg = d_kg; d.k3 = d_k3;
     d.kn1 = d_kn1; d.kn2 = d_kn2; d.step = step; d.dbar = d_dbar; d.gpk = d_gpk;

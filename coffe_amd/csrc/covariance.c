@@ -271,22 +271,61 @@ struct coffe_cov_plan {
     double *d_fws;     /* the column weights times pi / (16 N^2 r_j^nu2) (the row transform's scale) */
     int *d_rows, *d_pl1, *d_pl2, *d_flo, *d_fcnt, *d_foff, *d_upos, *d_status, *d_ls, *d_pair_of;
     int *d_uelo, *d_uehi;   /* monotone envelopes of the windows in row order (adjoint) */
-    /* per call, grown on demand */
+    /* the contraction's tables (cov_contract.hip); NULL: the integrals go row by row */
+    int Np;            /* N rounded up to 16: the stride of the diagonals and of the tables' rows */
+    double *d_tab;
+    double *d_tabT;    /* the same as plain rows, made at the first adjoint call */
+    /* per call, grown on demand; d_W: the rows' column functionals, or the contraction's splits */
     int spec_cap;
+    size_t w_cap;
     int64_t *d_in_off;
     int32_t *d_n_in;
     double *d_d, *d_W;
-    /* adjoint workspaces (coffe_cov_integrals_vjp), allocated on first use */
+    /* adjoint workspaces (coffe_cov_integrals_vjp), allocated on first use; d_Wbar: the rows'
+       cotangents, or the contraction's splits */
     int adj_cap;
+    size_t wbar_cap;
     double *d_Wbar, *d_dbar;
 };
+
+/* the contraction's tables take 32 bytes per multipole, separation and k; at most 16 of the 288 GB */
+#define TAB_CONTRACT ((size_t)16 << 30)
+static size_t contract_bytes(int nl, int N, int R)
+{
+    return sizeof(double) * 4 * (size_t)nl * (size_t)((R + 15) / 16 * 16) * (size_t)((N + 15) / 16 * 16);
+}
+
+/*
+ * Whether nblk diagonals go through the contraction (cov_contract.hip) rather than the row
+ * transforms: the lesser of two times per pair and diagonal, fitted to both on the card
+ * (10-200 Mpc/h, k over six decades).  Contraction: R^2 N of 4 flops at 51 TFLOP/s (few) or 2 at
+ * 62 (many; 53 in the adjoint).  Rows: a row costs its transforms and, per separation, its
+ * functionals, 142 ns forward and 265 ns adjoint at N = 8000, R = 700, 177 and 361 at R = 1000;
+ * lengths outside the LDS kernels 44 times that transform.  Measured at N = 8000: one spectrum
+ * 3.6 against 3.0 ms at R = 700 (adjoint 3.6 against 5.6), 16 spectra 50.8 against 55.5 ms at
+ * R = 1000 and 97.9 against 76.4 at R = 1400.
+ */
+static int contract_faster(const coffe_cov_plan *p, int nblk, int adjoint)
+{
+    const double N = p->N, R = p->R, pad = 16.0 * ((nblk + 15) / 16) / nblk;
+    const double con = R * R * N * (pad < 2.0 ? (adjoint ? 3.8e-14 : 3.2e-14) * pad : 7.8e-14);
+    const double row = p->nrows * ((p->fft ? 44.0 : 1.0) * 6e-13 * N * log2(N) + (adjoint ? 3.3e-10 : 1.2e-10) * R);
+    return con < row;
+}
+
+/* whether any call of a plan would take the contraction: the tables are made then */
+static int contract_ok(const coffe_cov_plan *p)
+{
+    return contract_bytes(p->nl, p->N, p->R) <= TAB_CONTRACT &&
+           (contract_faster(p, 2, 0) || contract_faster(p, 2, 1) || contract_faster(p, 16, 0) || contract_faster(p, 16, 1));
+}
 
 void coffe_cov_plan_destroy(coffe_cov_plan *p)
 {
     if (!p) return;
     free(p->h_sep);
     double *dd[] = {p->d_tw, p->d_A, p->d_ahat, p->d_B, p->d_kg, p->d_k3, p->d_kn1, p->d_kn2, p->d_prn1,
-                    p->d_prn2, p->d_fac, p->d_fw, p->d_fws, p->d_sep, p->d_d, p->d_W};
+                    p->d_prn2, p->d_fac, p->d_fw, p->d_fws, p->d_sep, p->d_d, p->d_W, p->d_tab, p->d_tabT};
     for (size_t i = 0; i < sizeof(dd) / sizeof(dd[0]); ++i) hipFree(dd[i]);
     int *di[] = {p->d_rows, p->d_pl1, p->d_pl2, p->d_flo, p->d_fcnt, p->d_foff, p->d_upos, p->d_uelo, p->d_uehi, p->d_status,
                  p->d_ls, p->d_pair_of};
@@ -440,7 +479,34 @@ int coffe_cov_plan_create(coffe_engine *e, int N, double kmin, double kmax, int 
         if (p->fft) st = ce_general_cov_ahat(p->fft, s, nl, N, p->d_A, p->d_ahat);
         else if (ce_launch_cov_ahat(s, nl, N, &p->rpN, p->d_tw, p->d_A, p->d_ahat)) st = COFFE_EDEVICE;
     }
+    p->Np = N;
+    double *d_Bf = NULL, *d_bhat = NULL;
+    if (st == COFFE_OK && contract_ok(p)) {
+        /* the column axis' array with the c2r's weights, zero above N/2, transformed as A is */
+        p->Np = (N + 15) / 16 * 16;
+        double *Bf = (double *)calloc(2 * (size_t)N * (size_t)nl, sizeof(double));
+        if (!Bf) st = COFFE_ENOMEM;
+        for (int i = 0; i < nl && st == COFFE_OK; ++i)
+            for (int q = 0; q <= N / 2; ++q)
+                for (int c = 0; c < 2; ++c)
+                    Bf[2 * ((size_t)N * i + q) + c] = B[2 * ((size_t)(N / 2 + 1) * i + q) + c] *
+                                                      (q == 0 || q == N / 2 ? 1.0 : 2.0);
+        if (st == COFFE_OK) st = upload((void **)&d_Bf, Bf, 2 * nb * (size_t)nl, s);
+        if (st == COFFE_OK) st = ce_dev_alloc((void **)&d_bhat, 2 * nb * (size_t)nl);
+        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_tab, contract_bytes(nl, N, R));
+        if (st == COFFE_OK) {
+            if (p->fft) st = ce_general_cov_ahat(p->fft, s, nl, N, d_Bf, d_bhat);
+            else if (ce_launch_cov_ahat(s, nl, N, &p->rpN, p->d_tw, d_Bf, d_bhat)) st = COFFE_EDEVICE;
+        }
+        if (st == COFFE_OK && ce_launch_cov_fold(s, nl, N, p->Np, R, (R + 15) / 16 * 16, p->d_ahat, d_bhat, p->d_flo,
+                                                 p->d_fcnt, p->d_foff, p->d_fw, p->d_fws, p->d_prn1, p->d_tab))
+            st = COFFE_EDEVICE;
+        const int sync = ce_hip_ok(hipStreamSynchronize(s));   /* Bf and the device arrays are released here */
+        if (st == COFFE_OK) st = sync;
+        free(Bf);
+    }
     if (st == COFFE_OK) st = ce_hip_ok(hipStreamSynchronize(s));
+    hipFree(d_Bf); hipFree(d_bhat);
     free(k); free(r); free(k3); free(kn); free(prn); free(tw); free(A); free(B);
     free(mark); free(pos); free(rows); free(upos);
     functionals_free(&f);
@@ -452,18 +518,31 @@ int coffe_cov_plan_create(coffe_engine *e, int N, double kmin, double kmax, int 
 int coffe_cov_plan_rows(const coffe_cov_plan *p) { return p ? p->nrows : 0; }
 int coffe_cov_plan_pairs(const coffe_cov_plan *p) { return p ? p->npair : 0; }
 
-static int grow(coffe_cov_plan *p, int nspec)
+static size_t wsize(const coffe_cov_plan *p, int nspec, int contract)
 {
-    if (nspec <= p->spec_cap) return COFFE_OK;
-    hipFree(p->d_in_off); hipFree(p->d_n_in); hipFree(p->d_d); hipFree(p->d_W);
-    p->d_in_off = NULL; p->d_n_in = NULL; p->d_d = NULL; p->d_W = NULL; p->spec_cap = 0;
-    int st = ce_dev_alloc((void **)&p->d_in_off, sizeof(int64_t) * (size_t)nspec);
-    if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_n_in, sizeof(int32_t) * (size_t)nspec);
-    if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_d, sizeof(double) * 2 * (size_t)p->N * (size_t)nspec);
-    if (st == COFFE_OK)
-        st = ce_dev_alloc((void **)&p->d_W, sizeof(double) * 2 * (size_t)nspec * (size_t)p->npair *
-                                                (size_t)p->nrows * (size_t)p->R);
-    if (st == COFFE_OK) p->spec_cap = nspec;
+    const size_t blk = 2 * (size_t)nspec * (size_t)p->npair * (size_t)p->R;
+    if (!contract) return blk * (size_t)p->nrows;
+    const int ns = ce_cov_contract_splits(2 * nspec, p->npair, p->R, p->Np);
+    return ns > 1 ? blk * (size_t)p->R * (size_t)ns : 0;
+}
+
+static int grow(coffe_cov_plan *p, int nspec, size_t w)
+{
+    int st = COFFE_OK;
+    if (nspec > p->spec_cap) {
+        hipFree(p->d_in_off); hipFree(p->d_n_in); hipFree(p->d_d);
+        p->d_in_off = NULL; p->d_n_in = NULL; p->d_d = NULL; p->spec_cap = 0;
+        st = ce_dev_alloc((void **)&p->d_in_off, sizeof(int64_t) * (size_t)nspec);
+        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_n_in, sizeof(int32_t) * (size_t)nspec);
+        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_d, sizeof(double) * 16 * (size_t)p->Np * (size_t)((nspec + 7) / 8));
+        if (st == COFFE_OK) p->spec_cap = nspec;
+    }
+    if (st == COFFE_OK && w > p->w_cap) {
+        hipFree(p->d_W);
+        p->d_W = NULL; p->w_cap = 0;
+        st = ce_dev_alloc((void **)&p->d_W, sizeof(double) * w);
+        if (st == COFFE_OK) p->w_cap = w;
+    }
     return st;
 }
 
@@ -484,15 +563,22 @@ int coffe_cov_integrals(coffe_cov_plan *p, int nspec, const int64_t *n_in, const
         cnt[i] = (int32_t)n_in[i];
         o += n_in[i];
     }
-    if (st == COFFE_OK) st = grow(p, nspec);
+    const int contract = p->d_tab && contract_faster(p, 2 * nspec, 0);
+    /* the splits shrink as spectra are added: the workspace is no multiple of nspec */
+    if (st == COFFE_OK) st = grow(p, nspec, wsize(p, nspec, contract));
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_in_off, off, sizeof(int64_t) * (size_t)nspec,
                                                       hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_n_in, cnt, sizeof(int32_t) * (size_t)nspec,
                                                       hipMemcpyHostToDevice, s));
-    if (st == COFFE_OK && ce_launch_cov_diag(s, nspec, p->N, p->d_in_off, p->d_n_in, d_k, d_pk, p->d_kg, p->d_k3,
-                                             p->d_kn1, p->d_kn2, p->step, p->d_d, p->d_status))
+    if (st == COFFE_OK && ce_launch_cov_diag(s, nspec, p->N, contract ? p->Np : p->N, contract, p->d_in_off, p->d_n_in,
+                                             d_k, d_pk, p->d_kg, p->d_k3, p->d_kn1, p->d_kn2, p->step, p->d_d,
+                                             p->d_status))
         st = COFFE_EDEVICE;
-    if (st == COFFE_OK && p->fft)
+    if (st == COFFE_OK && contract) {
+        if (ce_launch_cov_contract(s, 2 * nspec, p->Np, p->R, p->npair, p->d_pl1, p->d_pl2, p->d_tab, p->d_d, p->d_fac,
+                                   ce_cov_contract_splits(2 * nspec, p->npair, p->R, p->Np), p->d_W, d_out))
+            st = COFFE_EDEVICE;
+    } else if (st == COFFE_OK && p->fft)
         st = ce_general_cov_rows(p->fft, s, 2 * nspec, p->N, p->d_ahat, p->d_B, p->d_d, p->npair, p->d_pl1, p->d_pl2,
                                  p->nrows, p->d_rows, p->d_prn1, p->R, p->d_flo, p->d_fcnt, p->d_foff, p->d_fws,
                                  p->d_W);
@@ -501,7 +587,8 @@ int coffe_cov_integrals(coffe_cov_plan *p, int nspec, const int64_t *n_in, const
                                 p->d_pl1, p->d_pl2, p->nrows, p->d_rows, p->d_prn1, p->d_prn2, p->R, p->d_flo,
                                 p->d_fcnt, p->d_foff, p->d_fws, p->d_W))
         st = COFFE_EDEVICE;
-    if (st == COFFE_OK && ce_launch_cov_cols(s, nspec, p->npair, p->nrows, p->R, p->d_upos, p->d_fcnt, p->d_foff,
+    if (st == COFFE_OK && !contract &&
+        ce_launch_cov_cols(s, nspec, p->npair, p->nrows, p->R, p->d_upos, p->d_fcnt, p->d_foff,
                                              p->d_fw, p->d_fac, p->d_W, d_out))
         st = COFFE_EDEVICE;
     int h_status = 0;
@@ -532,24 +619,49 @@ int coffe_cov_integrals_vjp(coffe_cov_plan *p, int nspec, const int64_t *n_in, c
         cnt[i] = (int32_t)n_in[i];
         o += n_in[i];
     }
-    if (st == COFFE_OK) st = grow(p, nspec);
+    const int contract = p->d_tab && contract_faster(p, 2 * nspec, 1);
+    if (st == COFFE_OK) st = grow(p, nspec, 0);
+    const int nsplit = contract ? ce_cov_contract_splits_T(2 * nspec, p->npair, p->R, p->Np) : 0;
+    const size_t need = contract ? 2 * (size_t)nspec * (size_t)nsplit * (size_t)p->Np
+                                 : 2 * (size_t)nspec * (size_t)p->npair * (size_t)p->nrows * (size_t)p->R;
+    if (st == COFFE_OK && need > p->wbar_cap) {
+        hipFree(p->d_Wbar);
+        p->d_Wbar = NULL; p->wbar_cap = 0;
+        st = ce_dev_alloc((void **)&p->d_Wbar, sizeof(double) * need);
+        if (st == COFFE_OK) p->wbar_cap = need;
+    }
     if (st == COFFE_OK && nspec > p->adj_cap) {
-        hipFree(p->d_Wbar); hipFree(p->d_dbar);
-        p->d_Wbar = NULL; p->d_dbar = NULL; p->adj_cap = 0;
-        st = ce_dev_alloc((void **)&p->d_Wbar, sizeof(double) * 2 * (size_t)nspec * (size_t)p->npair *
-                                                   (size_t)p->nrows * (size_t)p->R);
-        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_dbar, sizeof(double) * 2 * (size_t)p->N * (size_t)nspec);
+        hipFree(p->d_dbar);
+        p->d_dbar = NULL; p->adj_cap = 0;
+        st = ce_dev_alloc((void **)&p->d_dbar, sizeof(double) * 2 * (size_t)p->N * (size_t)nspec);
         if (st == COFFE_OK) p->adj_cap = nspec;
     }
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_in_off, off, sizeof(int64_t) * (size_t)nspec,
                                                       hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_n_in, cnt, sizeof(int32_t) * (size_t)nspec,
                                                       hipMemcpyHostToDevice, s));
-    if (st == COFFE_OK &&
-        ce_launch_cov_vjp(s, nspec, p->N, &p->rpN, &p->rpM, p->d_tw, p->d_ahat, p->d_B, p->npair, p->d_pl1, p->d_pl2,
-                          p->nrows, p->d_rows, p->d_prn1, p->R, p->d_flo, p->d_fcnt, p->d_foff, p->d_fws, p->d_upos,
-                          p->d_uelo, p->d_uehi, p->d_fw, p->d_fac, d_gint, p->d_Wbar, p->d_dbar, p->d_in_off, p->d_n_in, d_k, d_pk,
-                          p->d_kg, p->d_k3, p->d_kn1, p->d_kn2, p->step, d_gpk, o))
+    if (st == COFFE_OK && contract && !p->d_tabT) {
+        double *rows = NULL;
+        st = ce_dev_alloc((void **)&rows, contract_bytes(p->nl, p->N, p->R));
+        if (st == COFFE_OK && ce_launch_cov_unfold(s, p->nl, p->Np, (p->R + 15) / 16 * 16, p->d_tab, rows)) {
+            st = COFFE_EDEVICE;
+            hipFree(rows);
+        } else {
+            p->d_tabT = rows;
+        }
+    }
+    if (st == COFFE_OK && contract) {
+        if (ce_launch_cov_contract_T(s, 2 * nspec, p->N, p->Np, p->R, p->npair, p->d_pl1, p->d_pl2, p->d_tabT, d_gint,
+                                     p->d_fac, nsplit, p->d_Wbar, p->d_dbar))
+            st = COFFE_EDEVICE;
+    } else if (st == COFFE_OK &&
+               ce_launch_cov_rows_vjp(s, nspec, p->N, &p->rpN, &p->rpM, p->d_tw, p->d_ahat, p->d_B, p->npair, p->d_pl1,
+                                      p->d_pl2, p->nrows, p->d_rows, p->d_prn1, p->R, p->d_flo, p->d_fcnt, p->d_foff,
+                                      p->d_fws, p->d_upos, p->d_uelo, p->d_uehi, p->d_fw, p->d_fac, d_gint, p->d_Wbar,
+                                      p->d_dbar))
+        st = COFFE_EDEVICE;
+    if (st == COFFE_OK && ce_launch_cov_diag_vjp(s, nspec, p->N, p->d_dbar, p->d_in_off, p->d_n_in, d_k, d_pk, p->d_kg,
+                                                 p->d_k3, p->d_kn1, p->d_kn2, p->step, d_gpk, o))
         st = COFFE_EDEVICE;
     if (st == COFFE_OK) st = ce_hip_ok(hipStreamSynchronize(s));
     free(off); free(cnt);
