@@ -154,9 +154,10 @@ int ce_launch_spline_adj(void *stream, int nchunk, const ce_chunk_dev *d_chunks,
                          const ce_grid_dev *d_grids, const double *d_k, const double *d_ws, double *d_gpk,
                          const int32_t *d_ranges);
 
-/* ---- small-separation table nodes (quad_kernels.hip): out/status [nspec][ntab][43] ---- */
+/* ---- small-separation table nodes (quad_kernels.hip): out/status [nspec][ntab][43]; max_n: the
+   longest spectrum ---- */
 int ce_launch_small_r(void *stream, int nspec, int ntab, const ce_spec_dev *d_spec, const ce_grid_dev *d_grids,
-                      const ce_table_desc *d_tabs, const double *d_k, const double *d_pk, double epsrel,
+                      const ce_table_desc *d_tabs, const double *d_k, const double *d_pk, int max_n, double epsrel,
                       double *d_out, int *d_status);
 /* the divergent I_0^4 table and its renormalisations (quad_kernels.hip): status
    and interval counts (may be null) [2 nsep + nchi^2] in the order i40, r0, ren */

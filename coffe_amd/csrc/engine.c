@@ -1395,7 +1395,10 @@ int coffe_batch_small_r(coffe_batch *b, const double *d_k, const double *d_pk, d
     const size_t n = (size_t)b->nspec * (size_t)b->ntab * (1 + CE_MIN_SEP_LEN);
     if (!b->d_srstat && dev_alloc((void **)&b->d_srstat, sizeof(int) * n) != COFFE_OK) return COFFE_ENOMEM;
     hipStream_t s = stream ? (hipStream_t)stream : b->e->stream;
-    if (ce_launch_small_r(s, b->nspec, b->ntab, b->d_spec, b->d_grids, b->d_tabs, d_k, d_pk, 1e-5, d_out,
+    int max_n = 0;
+    for (int i = 0; i < b->nspec; ++i)
+        if (b->h_spec[i].n_in > max_n) max_n = b->h_spec[i].n_in;
+    if (ce_launch_small_r(s, b->nspec, b->ntab, b->d_spec, b->d_grids, b->d_tabs, d_k, d_pk, max_n, 1e-5, d_out,
                           b->d_srstat))
         return COFFE_EDEVICE;
     int *h = (int *)malloc(sizeof(int) * n);
@@ -1578,7 +1581,7 @@ static int integral_table_any(double n, double l, size_t N, const double *k, con
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(d_grid, &hg, sizeof(hg), hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(d_tab, &td, sizeof(td), hipMemcpyHostToDevice, s));
     if (st == COFFE_OK &&
-        ce_launch_small_r(s, 1, 1, d_spec, d_grid, d_tab, base, base + nin, 1e-5, base + off_out, d_stat))
+        ce_launch_small_r(s, 1, 1, d_spec, d_grid, d_tab, base, base + nin, (int)nin, 1e-5, base + off_out, d_stat))
         st = COFFE_EDEVICE;
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(out_y, base + off_out, sizeof(double) * nodes, hipMemcpyDeviceToHost, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(h_stat, d_stat, sizeof(int) * nodes, hipMemcpyDeviceToHost, s));

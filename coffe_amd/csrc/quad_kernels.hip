@@ -9,11 +9,21 @@
 // over [kmin, kmax], P(k) the Akima spline of the input samples, by QUADPACK QAG
 // with the 61-point Gauss-Kronrod rule, epsabs 0, epsrel 1e-5 (common.c:1004-1040).
 //
-// One wavefront runs one adaptive integration: lane j evaluates Kronrod node j of
-// the interval being refined, the Gauss / Kronrod / |f| / |f - mean| sums are
-// reduced with lane shuffles, and the interval list (a, b, result, error) lives in
-// LDS.  Every lane holds the same reduced values, so the control flow of the
-// bisection loop is uniform across the wavefront.
+// One wavefront runs one adaptive integration: lane j evaluates Kronrod node j of both
+// halves of the interval being refined, the Gauss / Kronrod / |f| / |f - mean| sums are
+// reduced with DPP adds, and lane i holds interval i of the list (a, b, result, error)
+// in registers.  Every lane holds the same reduced values, so the control flow of the
+// bisection loop is uniform across the wavefront.  The few integrals that need more than
+// 64 intervals (the r = 0 renormalisation below 0.01 Mpc, of the divergent tables) are left to
+// a second kernel with the list in LDS (cap CE_QAG_CAP).
+//
+// What bounds it: the bisections are serial, and a step was a chain of a ten-step search of
+// the samples in L2, nine divisions for the Akima coefficients, series loops and shuffles,
+// twice, with five wavefronts a CU (32 KB of LDS list each).  The spline's coefficients
+// and an index of its nodes by their leading bits now sit in LDS, shared by a workgroup's
+// wavefronts, and sixteen wavefronts fit a CU: the FP64 units now bound it (two sines and a
+// division a node).  40,995 integrals of about 20 intervals, 600
+// samples: 1.12 against 8.2 ms.
 #include <float.h>
 #include <hip/hip_runtime.h>
 
@@ -26,64 +36,91 @@ namespace {
 __constant__ double c_min_sep[CE_MIN_SEP_LEN];
 __constant__ double c_xgk[31], c_wgk[31], c_wg[15];
 
-// spherical Bessel j_l(x), integer l >= 0: power series for |x| < 0.5, upward
-// recurrence from j_0, j_1 when x > l, otherwise Miller's downward recurrence
-// normalised with sum_k (2k+1) j_k^2 = 1 (GSL sf_bessel_jl is called at
-// integrals.c:309-316)
-__device__ double sph_jl(int l, double x)
+// lane i (uniform) of v
+__device__ __forceinline__ double read_lane(double v, int i)
 {
-    const double ax = fabs(x);
-    if (ax == 0.0) return l == 0 ? 1.0 : 0.0;
-    if (ax < 0.5) {
-        double pre = 1.0;
-        for (int k = 1; k <= l; ++k) pre *= x / (2.0 * k + 1.0);
-        const double y = -0.5 * x * x;
-        double term = 1.0, sum = 1.0;
-        for (int k = 1; k < 30; ++k) {
-            term *= y / (k * (2.0 * l + 2.0 * k + 1.0));
-            sum += term;
-            if (fabs(term) < 1e-18 * fabs(sum)) break;
-        }
-        return pre * sum;
-    }
-    double s, c;
-    sincos(x, &s, &c);
-    const double j0 = s / x;
-    if (l == 0) return j0;
-    const double j1 = (s / x - c) / x;
-    if (l == 1) return j1;
-    if (ax > (double)l) {
-        double jm = j0, jc = j1;
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), i),
+                            __builtin_amdgcn_readlane(__double2loint(v), i));
+}
+
+// v of the lane that DPP control C names; lanes without one keep `own`
+template <int C, int ROWS = 0xf>
+__device__ __forceinline__ double dpp(double own, double v)
+{
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(__double2hiint(own), __double2hiint(v), C, ROWS, 0xf, false),
+        __builtin_amdgcn_update_dpp(__double2loint(own), __double2loint(v), C, ROWS, 0xf, false));
+}
+
+// sum and maximum over the wavefront, in every lane: shifts by 1, 2, 4, 8 inside the rows of
+// 16, then the rows' last lanes broadcast on (0x142, 0x143), the total in lane 63
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += dpp<0x111>(0.0, v);
+    v += dpp<0x112>(0.0, v);
+    v += dpp<0x114>(0.0, v);
+    v += dpp<0x118>(0.0, v);
+    v += dpp<0x142, 0xa>(0.0, v);
+    v += dpp<0x143, 0xc>(0.0, v);
+    return read_lane(v, 63);
+}
+__device__ __forceinline__ double wave_max(double v)
+{
+    v = fmax(v, dpp<0x111>(v, v));
+    v = fmax(v, dpp<0x112>(v, v));
+    v = fmax(v, dpp<0x114>(v, v));
+    v = fmax(v, dpp<0x118>(v, v));
+    v = fmax(v, dpp<0x142, 0xa>(v, v));
+    v = fmax(v, dpp<0x143, 0xc>(v, v));
+    return read_lane(v, 63);
+}
+
+// x^n, integer n (a few products: pow() costs more than the rest of an integrand)
+__device__ __forceinline__ double ipow(double x, int n)
+{
+    const int m = n < 0 ? -n : n;
+    double p = 1.0;
+    for (int i = 0; i < m; ++i) p *= x;
+    return n < 0 ? 1.0 / p : p;
+}
+
+// j_0: sin(x) / x has no cancellation
+__device__ __forceinline__ double sph_j0(double x) { return x == 0.0 ? 1.0 : sin(x) / x; }
+
+// spherical Bessel j_l(x), integer 0 <= l <= 4, x >= 0 (GSL sf_bessel_jl is called at
+// integrals.c:309-316): upward recurrence from j_0, j_1 for x > l, else the power series, whose
+// alternating terms fall from the first on there (x^2 <= 2 (2 l + 3) for l <= 5).  rc: lane k
+// holds 1 / (k (2 l + 2 k + 1)).
+__device__ double sph_jl(int l, double x, double rc)
+{
+    if (l == 0) return sph_j0(x);
+    const bool ser = x <= (double)l;
+    double res = 0.0;
+    if (!ser) {
+        double s, c;
+        sincos(x, &s, &c);
+        const double ix = 1.0 / x;
+        double jm = s * ix, jc = (jm - c) * ix;
         for (int k = 1; k < l; ++k) {
-            const double jn = (2.0 * k + 1.0) / x * jc - jm;
+            const double jn = (2.0 * k + 1.0) * ix * jc - jm;
             jm = jc;
             jc = jn;
         }
-        return jc;
+        res = jc;
     }
-    const int L = l + 30 + (int)ax;
-    double fp = 0.0, fc = 1.0, fl = 0.0, norm = 0.0, f0 = 0.0, f1 = 0.0;
-    for (int k = L; k >= 0; --k) {
-        norm += (2.0 * k + 1.0) * fc * fc;
-        if (k == l) fl = fc;
-        if (k == 1) f1 = fc;
-        if (k == 0) {
-            f0 = fc;
-            break;
+    if (__ballot(ser) != 0) {   // every lane of the wavefront is here: read_lane's rc
+        double pre = 1.0;
+        for (int k = 1; k <= l; ++k) pre *= x / (2.0 * k + 1.0);
+        const double y = ser ? -0.5 * x * x : 0.0;
+        double term = 1.0, sum = 1.0;
+        for (int k = 1; k < 40; ++k) {
+            term *= y * read_lane(rc, k);
+            sum += term;
+            if (__ballot(fabs(term) >= 1e-18 * fabs(sum)) == 0) break;
         }
-        const double fm = (2.0 * k + 1.0) / x * fc - fp;
-        fp = fc;
-        fc = fm;
-        if (fabs(fc) > 1e250) {
-            fc *= 1e-250; fp *= 1e-250; fl *= 1e-250; f1 *= 1e-250;
-            norm *= 1e-250; norm *= 1e-250;
-        }
+        if (ser) res = pre * sum;
     }
-    double scale = 1.0 / sqrt(norm);
-    const double ref = fabs(j0) > fabs(j1) ? j0 : j1;
-    const double fref = fabs(j0) > fabs(j1) ? f0 : f1;
-    if ((ref < 0) != (fref * scale < 0)) scale = -scale;
-    return fl * scale;
+    return res;
 }
 
 // cylindrical Bessel J_m(x), integer m >= 0, x >= 0 (the half-integer tables' small-r
@@ -143,13 +180,6 @@ __device__ double cyl_jn(int m, double x)
     return fm / norm;
 }
 
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // integrands over k of the Akima spline P(k) of the input samples
 enum {
     SR_BESSEL = 0,    // k^2 P j_l(k r) / (k r)^n              (integrals.c:280-325)
@@ -159,8 +189,6 @@ enum {
 };
 
 struct sr_unit {
-    const double *k, *p;   // input samples of the spectrum
-    int n_in;
     int n, l;
     double r, r2;
     int kind;
@@ -170,9 +198,93 @@ struct sr_unit {
     double nd, ld;
 };
 
-__device__ __forceinline__ double integrand(const sr_unit &u, double k)
+// The Akima spline of the samples as a workgroup's wavefronts read it: coefficients and an index
+// of the intervals in LDS (LDS = true), or the samples themselves where they do not fit
+// (LDS = false: a bisection in L2 and the coefficients anew at every value).
+#define CE_SPL_BUCKETS 1024
+#define CE_SPL_MAX 3000     // samples in LDS: 40 bytes each of the CU's 160 KB
+struct lds_spline {
+    const double *x;        // [n]
+    const double2 *yb, *cd; // [n]: value and coefficients of the interval from node j
+    const unsigned short *idx;   // [CE_SPL_BUCKETS + 1]: interval of each bucket's lower edge
+    int base, shift, nb;
+};
+template <bool LDS>
+struct spline {
+    const double *k, *p;
+    int n;
+    double x0, x1;
+    lds_spline s;
+};
+
+// a bucket is a step of the leading bits of a (positive) double: 2^-s octave
+__device__ __forceinline__ int key_of(double v, int shift) { return __double2hiint(v) >> shift; }
+
+__host__ __device__ inline size_t spline_bytes(int n)
 {
-    const double pk = ce::akima_general(u.k, u.p, u.n_in, k);
+    return (size_t)n * 40 + (CE_SPL_BUCKETS + 8) * sizeof(unsigned short);
+}
+
+// the workgroup fills sp.s for values in [lo, hi], lo > 0; ends with a barrier
+template <bool LDS>
+__device__ void spline_load(spline<LDS> &sp, const double *k, const double *p, int n, double lo, double hi, char *mem)
+{
+    sp.k = k;
+    sp.p = p;
+    sp.n = n;
+    sp.x0 = k[0];
+    sp.x1 = k[n - 1];
+    if (!LDS) return;
+    double2 *yb = (double2 *)mem, *cd = yb + n;
+    double *x = (double *)(cd + n);
+    unsigned short *idx = (unsigned short *)(x + n);
+    int shift = 14;   // 64 buckets an octave, or as many as there is room for
+    while (key_of(hi, shift) - key_of(lo, shift) + 1 > CE_SPL_BUCKETS) ++shift;
+    sp.s.shift = shift;
+    sp.s.base = key_of(lo, shift);
+    sp.s.nb = key_of(hi, shift) - sp.s.base + 1;
+    sp.s.x = x;
+    sp.s.yb = yb;
+    sp.s.cd = cd;
+    sp.s.idx = idx;
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        x[j] = k[j];
+        const ce::akima_cf<double> c = ce::akima_coefs<double>(k, nullptr, p, nullptr, n, j < n - 1 ? j : n - 2);
+        yb[j] = make_double2(c.y0, c.b);
+        cd[j] = make_double2(c.c, c.d);
+    }
+    for (int b = threadIdx.x; b <= sp.s.nb; b += blockDim.x) {
+        const double edge = __hiloint2double((sp.s.base + b) << shift, 0);
+        int j = 0;
+        if (edge >= k[n - 1]) j = n - 2;
+        else if (edge > k[0]) j = ce::interval_bisect(k, 0, n - 1, edge);
+        idx[b] = (unsigned short)j;
+    }
+    __syncthreads();
+}
+
+// the spline at v; NaN outside the samples (as ce::akima_general)
+template <bool LDS>
+__device__ __forceinline__ double spline_at(const spline<LDS> &sp, double v)
+{
+    if (!LDS) return ce::akima_general(sp.k, sp.p, sp.n, v);
+    const int b = min(max(key_of(v, sp.s.shift) - sp.s.base, 0), sp.s.nb - 1);
+    int lo = sp.s.idx[b], hi = min((int)sp.s.idx[b + 1] + 1, sp.n - 1);
+    while (hi > lo + 1) {
+        const int m = (lo + hi) >> 1;
+        if (sp.s.x[m] > v) hi = m;
+        else lo = m;
+    }
+    const double t = v - sp.s.x[lo];
+    const double2 yb = sp.s.yb[lo], cd = sp.s.cd[lo];
+    const double r = yb.x + t * (yb.y + t * (cd.x + cd.y * t));
+    return v >= sp.x0 && v <= sp.x1 ? r : __builtin_nan("");
+}
+
+template <bool LDS>
+__device__ __forceinline__ double integrand(const sr_unit &u, const spline<LDS> &sp, double k, double rc)
+{
+    const double pk = spline_at(sp, k);
     const double sqrt_pi_2 = 1.25331413731550025121;
     if (u.half && u.kind == SR_PREFACTOR) return sqrt_pi_2 * pow(k, 2.0 + u.ld - u.nd) * pk;
     if (u.half && u.kind == SR_BESSEL) {
@@ -180,19 +292,29 @@ __device__ __forceinline__ double integrand(const sr_unit &u, double k)
         return k * k * pk * sqrt_pi_2 * cyl_jn((int)(u.ld + 0.5), x) / pow(x, u.nd + 0.5);
     }
     switch (u.kind) {
-    case SR_PREFACTOR: return pow(k, (double)(2 + u.l - u.n)) * pk;
+    case SR_PREFACTOR: return ipow(k, 2 + u.l - u.n) * pk;
     case SR_RENORM0: {
-        const double j0 = sph_jl(0, k * u.r);
-        return pk * (1. - j0 * j0) / k / k;
+        const double x = k * u.r;
+        // 1 - j0^2 ~ x^2 / 3 keeps what the rounding of j0 leaves: the series is the closer
+        // one below 0.5 (at most half a unit off)
+        double j0 = sph_j0(x), term = 1.0, sum = 1.0;
+        const double y = x < 0.5 ? -0.5 * x * x : 0.0;
+        for (int i = 1; i < 20 && __ballot(term != 0.0 && fabs(term) >= 1e-18 * fabs(sum)) != 0; ++i) {
+            term *= y * read_lane(rc, i);
+            sum += term;
+        }
+        if (x < 0.5) j0 = sum;
+        return pk * (1. - j0 * j0) / (k * k);
     }
     case SR_RENORM: {
         // the product of the two Bessel factors first: symmetric in (r, r2) bit for bit
-        const double jj = sph_jl(0, k * u.r) * sph_jl(0, k * u.r2);
-        return pk * jj / k / k;
+        const double xa = k * u.r, xb = k * u.r2;
+        const double ss = (xa == 0.0 ? 1.0 : sin(xa)) * (xb == 0.0 ? 1.0 : sin(xb));
+        return pk * ss / ((xa == 0.0 ? 1.0 : xa) * (xb == 0.0 ? 1.0 : xb) * (k * k));
     }
     default: {
         const double x = k * u.r;
-        return k * k * pk * sph_jl(u.l, x) / pow(x, (double)u.n);
+        return k * k * pk * sph_jl(u.l, x, rc) * ipow(x, -u.n);
     }
     }
 }
@@ -201,31 +323,32 @@ struct qk_out {
     double result, abserr, resabs, resasc;
 };
 
-// QUADPACK qk61 on [a, b]: lane j < 61 evaluates node j of the rule (j < 30: the left
-// half, j = 30: the centre, j > 30: the right half)
-__device__ qk_out qk61(const sr_unit &u, double a, double b, int lane)
+// a lane's node of the 61-point rule: lane j < 61 evaluates node j (j < 30: the left half,
+// j = 30: the centre, j > 30: the right half) at centre + half x; the other lanes repeat the
+// last one with weight 0
+struct qk_lane {
+    double x, wk, wg, rc;
+};
+__device__ __forceinline__ qk_lane qk_node(int lane, int l)
 {
-    const double center = 0.5 * (a + b), half = 0.5 * (b - a);
-    double f = 0.0, wk = 0.0, wg = 0.0;
-    if (lane < 61) {
-        const int j = lane <= 30 ? lane : 60 - lane;   // QUADPACK index of the node
-        const double x = lane < 30 ? center - half * c_xgk[j] : (lane == 30 ? center : center + half * c_xgk[j]);
-        f = integrand(u, x);
-        wk = c_wgk[j];
-        wg = (j & 1) ? c_wg[j >> 1] : 0.0;
-    }
-    const double rk = wave_sum(wk * f);
-    const double rg = wave_sum(wg * f);
-    const double rabs = wave_sum(wk * fabs(f));
-    const double mean = 0.5 * rk;
-    const double rasc = wave_sum(wk * fabs(f - mean));
+    qk_lane q;
+    const int i = min(lane, 60), j = i <= 30 ? i : 60 - i;   // QUADPACK index of the node
+    q.x = i < 30 ? -c_xgk[j] : (i == 30 ? 0.0 : c_xgk[j]);
+    q.wk = lane < 61 ? c_wgk[j] : 0.0;
+    q.wg = lane < 61 && (j & 1) ? c_wg[j >> 1] : 0.0;
+    q.rc = lane ? 1.0 / (lane * (2.0 * l + 2.0 * lane + 1.0)) : 0.0;
+    return q;
+}
+
+__device__ __forceinline__ qk_out qk_finish(double rk, double rg, double rabs, double rasc, double half)
+{
     qk_out o;
     double err = fabs((rk - rg) * half);
     o.result = rk * half;
     o.resabs = rabs * fabs(half);
     o.resasc = rasc * fabs(half);
     if (o.resasc != 0.0 && err != 0.0) {
-        const double scale = pow(200.0 * err / o.resasc, 1.5);
+        const double t = 200.0 * err / o.resasc, scale = t * sqrt(t);
         err = scale < 1.0 ? o.resasc * scale : o.resasc;
     }
     if (o.resabs > DBL_MIN / (50.0 * DBL_EPSILON)) {
@@ -236,25 +359,134 @@ __device__ qk_out qk61(const sr_unit &u, double a, double b, int lane)
     return o;
 }
 
-struct sr_args {
-    int nspec, ntab;
-    const ce_spec_dev *spec;
-    const ce_grid_dev *grids;
-    const ce_table_desc *tabs;
-    const double *k, *p;
-    double epsrel;
-    double *out;      // [nspec][ntab][1 + CE_MIN_SEP_LEN]
-    int *status;      // same layout: 0 converged, 1 interval limit, 2 roundoff, 3 bad integrand
+// QUADPACK qk61 on [a, b]
+template <bool LDS>
+__device__ __forceinline__ qk_out qk61(const sr_unit &u, const spline<LDS> &sp, const qk_lane &q, double a, double b)
+{
+    const double half = 0.5 * (b - a);
+    const double f = integrand(u, sp, 0.5 * (a + b) + half * q.x, q.rc);
+    // a node with weight 0 adds 0, not a NaN
+    const double fw = q.wk != 0.0 ? f : 0.0;
+    const double rk = wave_sum(q.wk * fw), rg = wave_sum(q.wg * fw), rabs = wave_sum(q.wk * fabs(fw));
+    const double rasc = wave_sum(q.wk * fabs(fw - 0.5 * rk));
+    return qk_finish(rk, rg, rabs, rasc, half);
+}
+
+// the two halves of an interval, their sums side by side
+template <bool LDS>
+__device__ __forceinline__ void qk61_pair(const sr_unit &u, const spline<LDS> &sp, const qk_lane &q, double a, double m,
+                                          double b, qk_out &o1, qk_out &o2)
+{
+    const double h1 = 0.5 * (m - a), h2 = 0.5 * (b - m);
+    const double e1 = integrand(u, sp, 0.5 * (a + m) + h1 * q.x, q.rc);
+    const double e2 = integrand(u, sp, 0.5 * (m + b) + h2 * q.x, q.rc);
+    const double f1 = q.wk != 0.0 ? e1 : 0.0, f2 = q.wk != 0.0 ? e2 : 0.0;
+    const double k1 = wave_sum(q.wk * f1), k2 = wave_sum(q.wk * f2);
+    const double g1 = wave_sum(q.wg * f1), g2 = wave_sum(q.wg * f2);
+    const double a1 = wave_sum(q.wk * fabs(f1)), a2 = wave_sum(q.wk * fabs(f2));
+    const double s1 = wave_sum(q.wk * fabs(f1 - 0.5 * k1)), s2 = wave_sum(q.wk * fabs(f2 - 0.5 * k2));
+    o1 = qk_finish(k1, g1, a1, s1, h1);
+    o2 = qk_finish(k2, g2, a2, s2, h2);
+}
+
+// the interval list of one integral: lane i's registers hold interval i (up to 64), or LDS holds
+// them (up to CE_QAG_CAP).  largest(): the interval with the largest error, the first on ties.
+struct list_regs {
+    static constexpr int cap = 64;
+    int lane;
+    double a, b, r, e;
+    __device__ void init(int l, double *)
+    {
+        lane = l;
+        a = b = r = 0.0;
+        e = -1.0;
+    }
+    __device__ void get(int i, double &ia, double &ib, double &ir, double &ie) const
+    {
+        ia = read_lane(a, i);
+        ib = read_lane(b, i);
+        ir = read_lane(r, i);
+        ie = read_lane(e, i);
+    }
+    __device__ void put(int i, double ia, double ib, double ir, double ie)
+    {
+        if (lane == i) {
+            a = ia;
+            b = ib;
+            r = ir;
+            e = ie;
+        }
+    }
+    __device__ int largest(int size) const
+    {
+        const double m = wave_max(lane < size ? e : -1.0);
+        const unsigned long long hit = __ballot(lane < size && e == m);
+        return hit ? __builtin_ctzll(hit) : 0;
+    }
+    __device__ double sum(int) const { return wave_sum(r); }
+};
+struct list_lds {
+    static constexpr int cap = CE_QAG_CAP;
+    int lane;
+    double *ia, *ib, *ir, *ie;
+    __device__ void init(int l, double *mem)
+    {
+        lane = l;
+        ia = mem;
+        ib = ia + cap;
+        ir = ib + cap;
+        ie = ir + cap;
+    }
+    __device__ void get(int i, double &a, double &b, double &r, double &e) const
+    {
+        a = ia[i];
+        b = ib[i];
+        r = ir[i];
+        e = ie[i];
+    }
+    __device__ void put(int i, double a, double b, double r, double e)
+    {
+        __syncthreads();   // one wavefront per workgroup: the list's earlier reads are done
+        if (lane == 0) {
+            ia[i] = a;
+            ib[i] = b;
+            ir[i] = r;
+            ie[i] = e;
+        }
+        __syncthreads();
+    }
+    __device__ int largest(int size) const
+    {
+        double be = -1.0;
+        int bi = 0x7fffffff;
+        for (int k = lane; k < size; k += 64)
+            if (ie[k] > be) { be = ie[k]; bi = k; }
+        const double m = wave_max(be);
+        int best = be == m ? bi : 0x7fffffff;   // the first of the lanes' firsts
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) best = min(best, __shfl_xor(best, off, 64));
+        return best < size ? best : 0;
+    }
+    __device__ double sum(int size) const
+    {
+        double part = 0.0;
+        for (int k = lane; k < size; k += 64) part += ir[k];
+        return wave_sum(part);
+    }
 };
 
-// QUADPACK QAG (epsabs 0, the 61-point rule) of u over [lo, hi] by one wavefront, the
-// interval list in LDS (cap CE_QAG_CAP); every lane returns the same sum.  Status: 0
-// converged, 1 interval limit, 2 roundoff, 3 bad integrand behaviour.
-__device__ int qag_wave(const sr_unit &u, double lo, double hi, double epsrel, int lane, double *ia, double *ib,
-                        double *ir, double *ie, double &result, int *nint = nullptr)
+#define QAG_MORE (-1)   // more intervals than the list holds: the integral is left to the next kernel
+
+// QUADPACK QAG (epsabs 0, the 61-point rule) of u over [lo, hi] by one wavefront; every lane
+// returns the same sum.  Status: 0 converged, 1 interval limit (CE_QAG_CAP), 2 roundoff,
+// 3 bad integrand behaviour, QAG_MORE.
+template <class List, bool LDS>
+__device__ int qag_wave(const sr_unit &u, const spline<LDS> &sp, double lo, double hi, double epsrel, int lane,
+                        double *mem, double &result, int &nint)
 {
-    if (nint) *nint = 1;
-    qk_out q0 = qk61(u, lo, hi, lane);
+    const qk_lane q = qk_node(lane, u.l);
+    nint = 1;
+    const qk_out q0 = qk61(u, sp, q, lo, hi);
     int st = 0;
     result = q0.result;
     double tol = epsrel * fabs(q0.result);
@@ -263,18 +495,17 @@ __device__ int qag_wave(const sr_unit &u, double lo, double hi, double epsrel, i
                        (q0.abserr <= tol && q0.abserr != q0.resasc) || q0.abserr == 0.0;
     if (q0.abserr <= round_off && q0.abserr > tol) st = 2;
     if (done0) return st;
-    if (lane == 0) {
-        ia[0] = lo; ib[0] = hi; ir[0] = q0.result; ie[0] = q0.abserr;
-    }
-    __syncthreads();
+    List list;
+    list.init(lane, mem);
+    list.put(0, lo, hi, q0.result, q0.abserr);
     int size = 1, imax = 0, iter = 1, rt1 = 0, rt2 = 0;
     double area = q0.result, errsum = q0.abserr;
     do {
-        const double a1 = ia[imax], b2 = ib[imax];
+        double a1, b2, ri, ei;
+        list.get(imax, a1, b2, ri, ei);
         const double b1 = 0.5 * (a1 + b2), a2 = b1;
-        const double ri = ir[imax], ei = ie[imax];
-        const qk_out q1 = qk61(u, a1, b1, lane);
-        const qk_out q2 = qk61(u, a2, b2, lane);
+        qk_out q1, q2;
+        qk61_pair(u, sp, q, a1, b1, b2, q1, q2);
         const double area12 = q1.result + q2.result, err12 = q1.abserr + q2.abserr;
         errsum += err12 - ei;
         area += area12 - ri;
@@ -289,56 +520,39 @@ __device__ int qag_wave(const sr_unit &u, double lo, double hi, double epsrel, i
             const double tmp = (1 + 100 * DBL_EPSILON) * (fabs(a2) + 1000 * DBL_MIN);
             if (fabs(a1) <= tmp && fabs(b2) <= tmp) st = 3;
         }
-        __syncthreads();   // every lane has read the interval being replaced
-        if (lane == 0) {
-            // the refined interval keeps the half with the larger error
-            const bool right = q2.abserr > q1.abserr;
-            ia[imax] = right ? a2 : a1; ib[imax] = right ? b2 : b1;
-            ir[imax] = right ? q2.result : q1.result; ie[imax] = right ? q2.abserr : q1.abserr;
-            ia[size] = right ? a1 : a2; ib[size] = right ? b1 : b2;
-            ir[size] = right ? q1.result : q2.result; ie[size] = right ? q1.abserr : q2.abserr;
-        }
-        __syncthreads();
+        // the refined interval keeps the half with the larger error
+        const bool right = q2.abserr > q1.abserr;
+        list.put(imax, right ? a2 : a1, right ? b2 : b1, right ? q2.result : q1.result, right ? q2.abserr : q1.abserr);
+        list.put(size, right ? a1 : a2, right ? b1 : b2, right ? q1.result : q2.result, right ? q1.abserr : q2.abserr);
         size++;
-        // the interval with the largest error, first one on ties
-        double be = -1.0;
-        int bi = 0x7fffffff;
-        for (int kk = lane; kk < size; kk += 64) {
-            if (ie[kk] > be) { be = ie[kk]; bi = kk; }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double oe = __shfl_xor(be, off, 64);
-            const int oi = __shfl_xor(bi, off, 64);
-            if (oe > be || (oe == be && oi < bi)) { be = oe; bi = oi; }
-        }
-        imax = bi < size ? bi : 0;
         iter++;
         if (iter >= CE_QAG_CAP && errsum > tol && !st) st = 1;
-    } while (iter < CE_QAG_CAP && !st && errsum > tol);
-    double part = 0.0;
-    for (int kk = lane; kk < size; kk += 64) part += ir[kk];
-    result = wave_sum(part);
-    if (nint) *nint = size;
+        if (iter >= CE_QAG_CAP || st || !(errsum > tol)) break;
+        if (size >= List::cap) return QAG_MORE;
+        imax = list.largest(size);
+    } while (true);
+    result = list.sum(size);
+    nint = size;
     return st;
 }
 
-// one wavefront (block of 64) per (spectrum, table, node)
-__global__ void __launch_bounds__(64) k_small_r(sr_args a)
+struct sr_args {
+    int nspec, ntab;
+    const ce_spec_dev *spec;
+    const ce_grid_dev *grids;
+    const ce_table_desc *tabs;
+    const double *k, *p;
+    double epsrel;
+    double *out;      // [nspec][ntab][1 + CE_MIN_SEP_LEN]
+    int *status;      // same layout: 0 converged, 1 interval limit, 2 roundoff, 3 bad integrand
+};
+
+// the integral of `unit` = (spectrum, table, node); false: its value is 0
+__device__ __forceinline__ bool small_r_unit(const sr_args &a, int unit, sr_unit &u)
 {
-    __shared__ double ia[CE_QAG_CAP], ib[CE_QAG_CAP], ir[CE_QAG_CAP], ie[CE_QAG_CAP];
     constexpr int NODES = 1 + CE_MIN_SEP_LEN;
-    const int unit = blockIdx.x;
-    const int lane = threadIdx.x;
     const int node = unit % NODES;
     const int t = (unit / NODES) % a.ntab;
-    const int s = unit / (NODES * a.ntab);
-    const ce_spec_dev sp = a.spec[s];
-    const ce_grid_dev &g = a.grids[sp.grid];
-    sr_unit u;
-    u.k = a.k + sp.in_off;
-    u.p = a.p + sp.in_off;
-    u.n_in = sp.n_in;
     u.n = (int)a.tabs[t].n;
     u.l = (int)a.tabs[t].l;
     u.nd = a.tabs[t].n;
@@ -347,35 +561,69 @@ __global__ void __launch_bounds__(64) k_small_r(sr_args a)
     u.kind = node == 0 ? SR_PREFACTOR : SR_BESSEL;
     u.r = node == 0 ? 0.0 : c_min_sep[node - 1];
     u.r2 = 0.0;
-    const int64_t o = (int64_t)unit;
-    if (node == 0 && (u.half ? u.nd < u.ld : u.n < u.l)) {   // I_l^n(0) = 0 for n < l
-        if (lane == 0) {
-            a.out[o] = 0.0;
-            a.status[o] = 0;
-        }
-        return;
+    return !(node == 0 && (u.half ? u.nd < u.ld : u.n < u.l));   // I_l^n(0) = 0 for n < l
+}
+
+__device__ void small_r_store(const sr_args &a, int unit, const sr_unit &u, double result, int st)
+{
+    const double pi = 3.14159265358979323846;
+    double v = result / 2. / pi / pi;
+    if (u.kind == SR_PREFACTOR && u.half) {
+        // 2^(l+1/2) Gamma(l+3/2) = 2^m m!, m = l + 1/2 (integrals.c:215-231)
+        const int m = (int)(u.ld + 0.5);
+        double c = 1.0;
+        for (int i = 1; i <= m; ++i) c *= 2.0 * i;
+        v /= c;
+    } else if (u.kind == SR_PREFACTOR) {
+        double df = 1.0;   // (2l+1)!! = 2^(l+1/2) Gamma(l+3/2) / sqrt(pi/2)
+        for (int i = 3; i <= 2 * u.l + 1; i += 2) df *= i;
+        v /= df;
+    } else if (u.half ? u.nd >= u.ld : u.n >= u.l) {
+        v *= u.half ? pow(u.r, u.nd - u.ld) : pow(u.r, (double)(u.n - u.l));
     }
-    double result;
-    int st = qag_wave(u, g.kmin, g.kmax, a.epsrel, lane, ia, ib, ir, ie, result);
-    if (lane == 0) {
-        const double pi = 3.14159265358979323846;
-        double v = result / 2. / pi / pi;
-        if (node == 0 && u.half) {
-            // 2^(l+1/2) Gamma(l+3/2) = 2^m m!, m = l + 1/2 (integrals.c:215-231)
-            const int m = (int)(u.ld + 0.5);
-            double c = 1.0;
-            for (int i = 1; i <= m; ++i) c *= 2.0 * i;
-            v /= c;
-        } else if (node == 0) {
-            double df = 1.0;   // (2l+1)!! = 2^(l+1/2) Gamma(l+3/2) / sqrt(pi/2)
-            for (int i = 3; i <= 2 * u.l + 1; i += 2) df *= i;
-            v /= df;
-        } else if (u.half ? u.nd >= u.ld : u.n >= u.l) {
-            v *= u.half ? pow(u.r, u.nd - u.ld) : pow(u.r, (double)(u.n - u.l));
+    if (!isfinite(v) && st == 0) st = 3;
+    a.out[unit] = v;
+    a.status[unit] = st;
+}
+
+// one wavefront per (spectrum, table, node); a workgroup's wavefronts share a spectrum
+// (blockIdx.y) and its spline
+template <class List, bool LDS>
+__global__ void __launch_bounds__(512) k_small_r(sr_args a, size_t list_bytes)
+{
+    extern __shared__ double2 quad_lds[];
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int per = a.ntab * (1 + CE_MIN_SEP_LEN);
+    const int s = blockIdx.y;
+    const ce_spec_dev spec = a.spec[s];
+    const ce_grid_dev &g = a.grids[spec.grid];
+    const bool again = List::cap != 64;   // only what the first kernel left
+    spline<LDS> sp;
+    if (again) {
+        int any = 0;
+        for (int e = lane; e * (int)gridDim.x + (int)blockIdx.x < per; e += 64)
+            any |= a.status[(int64_t)s * per + e * (int)gridDim.x + (int)blockIdx.x] == QAG_MORE;
+        if (!__ballot(any)) return;
+    }
+    spline_load(sp, a.k + spec.in_off, a.p + spec.in_off, spec.n_in, g.kmin, g.kmax, (char *)quad_lds + list_bytes);
+    for (int e = blockIdx.x * nw + (threadIdx.x >> 6); e < per; e += gridDim.x * nw) {
+        const int unit = s * per + e;
+        if (again && a.status[unit] != QAG_MORE) continue;
+        sr_unit u;
+        if (!small_r_unit(a, unit, u)) {
+            if (lane == 0) {
+                a.out[unit] = 0.0;
+                a.status[unit] = 0;
+            }
+            continue;
         }
-        if (!isfinite(v) && st == 0) st = 3;
-        a.out[o] = v;
-        a.status[o] = st;
+        double result;
+        int nint;
+        const int st = qag_wave<List>(u, sp, g.kmin, g.kmax, a.epsrel, lane, (double *)quad_lds, result, nint);
+        if (lane == 0) {
+            if (st == QAG_MORE) a.status[unit] = st;
+            else small_r_store(a, unit, u, result, st);
+        }
     }
 }
 
@@ -396,35 +644,50 @@ struct div_args {
 // the divergent table I_0^4 and its renormalisations (integrals.c:772-909), one
 // wavefront per integral: units [0, nsep) I_0^4(sep) sep^4, [nsep, 2 nsep) the r = 0
 // renormalisation at sep (times sep^4 as well, integrals.c:351-356, n = 4, l = 0), then
-// the nchi^2 grid of int P j_0 j_0 / k^2; all divided by 2 pi^2
-__global__ void __launch_bounds__(64) k_divergent(div_args a)
+// the nchi^2 grid of int P j_0 j_0 / k^2; all divided by 2 pi^2.  The wavefronts stride over
+// the units, so that neighbours (which cost alike) go to different workgroups.
+template <class List, bool LDS>
+__global__ void __launch_bounds__(256, 4) k_divergent(div_args a, size_t list_bytes)
 {
-    __shared__ double ia[CE_QAG_CAP], ib[CE_QAG_CAP], ir[CE_QAG_CAP], ie[CE_QAG_CAP];
-    const int unit = blockIdx.x;
-    const int lane = threadIdx.x;
+    extern __shared__ double2 quad_lds[];
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int units = 2 * a.nsep + a.nchi * a.nchi;
+    const int stride = gridDim.x * nw;
+    const bool again = List::cap != 64;   // only what the first kernel left
+    if (again) {
+        int any = 0;
+        for (int64_t e = (int64_t)lane * stride + blockIdx.x; e < units; e += (int64_t)64 * stride)
+            any |= a.status[e] == QAG_MORE;
+        if (!__ballot(any)) return;
+    }
+    spline<LDS> sp;
+    spline_load(sp, a.k, a.p, a.n_in, a.kmin, a.kmax, (char *)quad_lds + list_bytes);
     sr_unit u;
-    u.k = a.k;
-    u.p = a.p;
-    u.n_in = a.n_in;
     u.n = 4;
     u.l = 0;
     u.half = 0;
     u.nd = 4.0;
     u.ld = 0.0;
-    u.r2 = 0.0;
-    if (unit < 2 * a.nsep) {
-        u.kind = unit < a.nsep ? SR_BESSEL : SR_RENORM0;
-        u.r = a.sep[unit < a.nsep ? unit : unit - a.nsep];
-    } else {
-        const int q = unit - 2 * a.nsep;
-        u.kind = SR_RENORM;
-        u.r = a.chi[q % a.nchi];
-        u.r2 = a.chi[q / a.nchi];
-    }
-    double result;
-    int nint;
-    int st = qag_wave(u, a.kmin, a.kmax, a.epsrel, lane, ia, ib, ir, ie, result, &nint);
-    if (lane == 0) {
+    for (int unit = (threadIdx.x >> 6) * gridDim.x + blockIdx.x; unit < units; unit += stride) {
+        if (again && a.status[unit] != QAG_MORE) continue;
+        u.r2 = 0.0;
+        if (unit < 2 * a.nsep) {
+            u.kind = unit < a.nsep ? SR_BESSEL : SR_RENORM0;
+            u.r = a.sep[unit < a.nsep ? unit : unit - a.nsep];
+        } else {
+            const int q = unit - 2 * a.nsep;
+            u.kind = SR_RENORM;
+            u.r = a.chi[q % a.nchi];
+            u.r2 = a.chi[q / a.nchi];
+        }
+        double result;
+        int nint;
+        int st = qag_wave<List>(u, sp, a.kmin, a.kmax, a.epsrel, lane, (double *)quad_lds, result, nint);
+        if (lane != 0) continue;
+        if (st == QAG_MORE) {
+            a.status[unit] = st;
+            continue;
+        }
         const double pi = 3.14159265358979323846;
         if (a.nint) a.nint[unit] = nint;
         double v = result;
@@ -438,11 +701,62 @@ __global__ void __launch_bounds__(64) k_divergent(div_args a)
     }
 }
 
+constexpr size_t LIST_BYTES = 4 * CE_QAG_CAP * sizeof(double);
+
+template <class F>
+hipError_t lds_limit(F *fn, size_t bytes)
+{
+    return hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+// first the kernel with the list in registers, then the one with the list in LDS for what it left
+template <bool LDS>
+hipError_t launch_small_r(const sr_args &all, size_t sbytes, hipStream_t s)
+{
+    const int per = all.ntab * (1 + CE_MIN_SEP_LEN);
+    // wavefronts per workgroup: one while the integrals do not fill the chip (each then makes
+    // its own spline in a microsecond or two), eight beyond
+    const int nw = (int64_t)all.nspec * per <= 2048 ? 1 : 8;
+    hipError_t e = lds_limit(k_small_r<list_regs, LDS>, sbytes);
+    if (e == hipSuccess) e = lds_limit(k_small_r<list_lds, LDS>, LIST_BYTES + sbytes);
+    for (int s0 = 0; s0 < all.nspec && e == hipSuccess; s0 += 32768) {   // the grid's y range
+        sr_args a = all;
+        a.nspec = all.nspec - s0 < 32768 ? all.nspec - s0 : 32768;
+        a.spec += s0;
+        a.out += (int64_t)s0 * per;
+        a.status += (int64_t)s0 * per;
+        hipLaunchKernelGGL((k_small_r<list_regs, LDS>), dim3((per + nw - 1) / nw, a.nspec), dim3(64 * nw), sbytes, s, a,
+                           (size_t)0);
+        hipLaunchKernelGGL((k_small_r<list_lds, LDS>), dim3(per < 64 ? per : 64, a.nspec), dim3(64),
+                           LIST_BYTES + sbytes, s, a, LIST_BYTES);
+        e = hipGetLastError();
+    }
+    return e;
+}
+
+template <bool LDS>
+hipError_t launch_divergent(const div_args &a, int units, size_t sbytes, hipStream_t s)
+{
+    hipError_t e = lds_limit(k_divergent<list_regs, LDS>, sbytes);
+    if (e == hipSuccess) e = lds_limit(k_divergent<list_lds, LDS>, LIST_BYTES + sbytes);
+    if (e != hipSuccess) return e;
+    // four wavefronts share a spline; two rounds of the workgroups that are resident at once
+    // (128 VGPRs; 1116 us, against 1186 with one round, 1195 with eight wavefronts, 1296 at 168
+    // VGPRs and 1379 at 256)
+    const int nw = units <= 2048 ? 1 : 4;
+    const int wg = (units + nw - 1) / nw, most = nw == 1 ? wg : 2048;
+    hipLaunchKernelGGL((k_divergent<list_regs, LDS>), dim3(wg < most ? wg : most), dim3(64 * nw), sbytes, s, a,
+                       (size_t)0);
+    hipLaunchKernelGGL((k_divergent<list_lds, LDS>), dim3(units < 512 ? units : 512), dim3(64), LIST_BYTES + sbytes, s, a,
+                       LIST_BYTES);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 extern "C" int ce_launch_small_r(void *stream, int nspec, int ntab, const ce_spec_dev *d_spec,
                                  const ce_grid_dev *d_grids, const ce_table_desc *d_tabs, const double *d_k,
-                                 const double *d_pk, double epsrel, double *d_out, int *d_status)
+                                 const double *d_pk, int max_n, double epsrel, double *d_out, int *d_status)
 {
     static const double min_sep[CE_MIN_SEP_LEN] = {
         1E-6, 1E-5, 1E-4, 1E-3, 2E-3, 5E-3, 7E-3, 8E-3, 9E-3, 1E-2, 1.1E-2, 1.2E-2, 1.25E-2, 1.3E-2,
@@ -462,9 +776,7 @@ extern "C" int ce_launch_small_r(void *stream, int nspec, int ntab, const ce_spe
     sr_args a;
     a.nspec = nspec; a.ntab = ntab; a.spec = d_spec; a.grids = d_grids; a.tabs = d_tabs;
     a.k = d_k; a.p = d_pk; a.epsrel = epsrel; a.out = d_out; a.status = d_status;
-    const int units = nspec * ntab * (1 + CE_MIN_SEP_LEN);
-    hipLaunchKernelGGL(k_small_r, dim3(units), dim3(64), 0, s, a);
-    return (int)hipGetLastError();
+    return (int)(max_n <= CE_SPL_MAX ? launch_small_r<true>(a, spline_bytes(max_n), s) : launch_small_r<false>(a, 0, s));
 }
 
 extern "C" int ce_launch_divergent(void *stream, const double *d_k, const double *d_pk, int n_in, double kmin,
@@ -485,6 +797,6 @@ extern "C" int ce_launch_divergent(void *stream, const double *d_k, const double
     a.i40 = d_i40; a.r0 = d_r0; a.ren = d_ren; a.status = d_status; a.nint = d_nint;
     const int units = 2 * nsep + nchi * nchi;
     if (units <= 0) return 0;
-    hipLaunchKernelGGL(k_divergent, dim3(units), dim3(64), 0, s, a);
-    return (int)hipGetLastError();
+    return (int)(n_in <= CE_SPL_MAX ? launch_divergent<true>(a, units, spline_bytes(n_in), s)
+                                    : launch_divergent<false>(a, units, 0, s));
 }
