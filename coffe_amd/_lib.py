@@ -54,6 +54,8 @@ def load_library():
     L.coffe_engine_create.argtypes = [i, ctypes.POINTER(vp)]
     L.coffe_engine_destroy.argtypes = [vp]
     L.coffe_engine_destroy.restype = None
+    L.coffe_engine_stream.argtypes = [vp]
+    L.coffe_engine_stream.restype = vp
     L.coffe_engine_inject_alloc_failure.argtypes = [i]
     L.coffe_engine_inject_alloc_failure.restype = None
     L.coffe_engine_default.argtypes = []
@@ -122,7 +124,7 @@ def load_library():
 
 EXPORTED = [
     "coffe_engine_strerror", "coffe_engine_last_error", "coffe_engine_create", "coffe_engine_destroy",
-    "coffe_engine_default", "coffe_engine_synchronize", "twofast_1bessel", "twofast_1bessel_status",
+    "coffe_engine_default", "coffe_engine_stream", "coffe_engine_synchronize", "twofast_1bessel", "twofast_1bessel_status",
     "twofast_1bessel_noalloc", "coffe_engine_inject_alloc_failure",
     "coffe_batch_create", "coffe_batch_destroy", "coffe_batch_input_size", "coffe_batch_forward",
     "coffe_batch_vjp", "coffe_batch_tables", "coffe_batch_prepare", "coffe_batch_tables_stage",

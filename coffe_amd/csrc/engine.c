@@ -352,6 +352,8 @@ void coffe_engine_destroy(coffe_engine *e)
     free(e);
 }
 
+void *coffe_engine_stream(coffe_engine *e) { return e ? (void *)e->stream : NULL; }
+
 int coffe_engine_synchronize(coffe_engine *e)
 {
     if (!e) return COFFE_EINVAL;

@@ -15,7 +15,8 @@ def _ptr(t):
 def _need(t, shape, name):
     """A tensor handed to a kernel must be contiguous float64 on a GPU with exactly this shape."""
     import torch
-    if t is None:
+    if t is None or (type(t) is torch.Tensor and t.dtype is torch.float64 and t.shape == shape and t.is_cuda and
+                     t.is_contiguous()):
         return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name}: expected a torch tensor")
@@ -34,6 +35,28 @@ class Engine:
         check(self.L.coffe_engine_create(device, ctypes.byref(h)), "coffe_engine_create")
         self.h = h
         self.device = device
+        self._ext = None
+
+    def empty(self, *shapes):
+        """New float64 tensors on the device, for a call that gets no stream.  With torch on its
+        default stream such a call runs on the engine's own stream (which the default
+        stream's work waits for and which waits for it); the tensors are then allocated as
+        that stream's, so that the allocator hands their memory to no other stream while
+        the engine still writes it."""
+        import torch
+        if torch._C._cuda_getCurrentRawStream(self.device):
+            return [torch.empty(s, dtype=torch.float64, device=self.device) for s in shapes]
+        # the two switches by the stream's ids: half the time of the stream context manager
+        to, own = torch._C._cuda_setStream, self._ext
+        if own is None:
+            ext = torch.cuda.ExternalStream(self.L.coffe_engine_stream(self.h), device=self.device)
+            cur = torch.cuda.default_stream(self.device)
+            own = self._ext = (ext.stream_id, cur.stream_id, ext.device_index, ext.device_type)
+        to(stream_id=own[0], device_index=own[2], device_type=own[3])
+        try:
+            return [torch.empty(s, dtype=torch.float64, device=self.device) for s in shapes]
+        finally:
+            to(stream_id=own[1], device_index=own[2], device_type=own[3])
 
     def close(self):
         if self.h:
@@ -77,6 +100,10 @@ class Batch:
         self.L = L
         self.offsets = np.concatenate([[0], np.cumsum(self.n_in)])
         self.n_total = int(self.offsets[-1])
+        self._kshape = (self.n_total,)
+        self._Ashape = (nz, nl, len(self.tables), len(self.sep))
+        self._tshape = (self.nspec, len(self.tables), len(self.sep))
+        self._oshape = (self.nspec, nz, nl, len(self.sep))
 
     def close(self):
         if self.h:
@@ -90,45 +117,53 @@ class Batch:
             pass
 
     def _check_io(self, k, pk, A, itab, out):
-        ntab, nsep = len(self.tables), len(self.sep)
-        _need(k, (self.n_total,), "k")
-        _need(pk, (self.n_total,), "pk")
-        _need(A, (self.nz, self.nl, ntab, nsep), "A")
-        _need(itab, (self.nspec, ntab, nsep), "itab")
-        _need(out, (self.nspec, self.nz, self.nl, nsep), "out")
+        _need(k, self._kshape, "k")
+        _need(pk, self._kshape, "pk")
+        _need(A, self._Ashape, "A")
+        _need(itab, self._tshape, "itab")
+        _need(out, self._oshape, "out")
 
-    @staticmethod
-    def _stream():
+    def _stream(self):
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(self.engine.device)
+
+    def _outputs(self, want, stream):
+        """The outputs of `want` ((tensor or None, shape) each), allocated where the caller gave none."""
+        import torch
+        new = [shape for t, shape in want if t is None]
+        if not new:
+            return [t for t, _ in want]
+        got = self.engine.empty(*new) if stream is None else \
+            [torch.empty(shape, dtype=torch.float64, device=self.engine.device) for shape in new]
+        if len(new) == len(want):
+            return got
+        got = iter(got)
+        return [next(got) if t is None else t for t, _ in want]
 
     def forward(self, k, pk, A=None, itab=None, out=None, stream=None):
         """k, pk: float64 cuda tensors (concatenated); A: (nz, nl, ntab, nsep)."""
-        import torch
-        ntab, nsep = len(self.tables), len(self.sep)
-        if itab is None:
-            itab = torch.empty((self.nspec, ntab, nsep), dtype=torch.float64, device=k.device)
-        if A is not None and out is None:
-            out = torch.empty((self.nspec, self.nz, self.nl, nsep), dtype=torch.float64, device=k.device)
+        want = [(itab, self._tshape)]
+        if A is not None:
+            want.append((out, self._oshape))
         self._check_io(k, pk, A, itab, out)
-        check(self.L.coffe_batch_forward(self.h, _ptr(k), _ptr(pk), _ptr(A), _ptr(itab), _ptr(out),
+        if A is None:
+            itab, = self._outputs(want, stream)
+        else:
+            itab, out = self._outputs(want, stream)
+        check(self.L.coffe_batch_forward(self.h, k.data_ptr(), pk.data_ptr(), None if A is None else A.data_ptr(),
+                                         itab.data_ptr(), None if out is None else out.data_ptr(),
                                          stream if stream is not None else self._stream()), "coffe_batch_forward")
         return itab, out
 
     def vjp(self, k, pk, A, gout, itab=None, out=None, gpk=None, stream=None):
-        import torch
-        ntab, nsep = len(self.tables), len(self.sep)
-        if itab is None:
-            itab = torch.empty((self.nspec, ntab, nsep), dtype=torch.float64, device=k.device)
-        if out is None:
-            out = torch.empty((self.nspec, self.nz, self.nl, nsep), dtype=torch.float64, device=k.device)
-        if gpk is None:
-            gpk = torch.empty_like(pk)
         self._check_io(k, pk, A, itab, out)
-        _need(gout, (self.nspec, self.nz, self.nl, nsep), "gout")
-        _need(gpk, (self.n_total,), "gpk")
-        check(self.L.coffe_batch_vjp(self.h, _ptr(k), _ptr(pk), _ptr(A), _ptr(gout), _ptr(itab), _ptr(out),
-                                     _ptr(gpk), stream if stream is not None else self._stream()), "coffe_batch_vjp")
+        _need(gout, self._oshape, "gout")
+        _need(gpk, self._kshape, "gpk")
+        itab, out, gpk = self._outputs([(itab, self._tshape), (out, self._oshape), (gpk, self._kshape)], stream)
+        check(self.L.coffe_batch_vjp(self.h, k.data_ptr(), pk.data_ptr(), None if A is None else A.data_ptr(),
+                                     None if gout is None else gout.data_ptr(), itab.data_ptr(), out.data_ptr(),
+                                     gpk.data_ptr(), stream if stream is not None else self._stream()),
+              "coffe_batch_vjp")
         return itab, out, gpk
 
     # stage-by-stage launches (same kernels as forward / vjp), for pipelining and timing
@@ -182,9 +217,8 @@ class Batch:
         return out
 
     def tables_full(self, k, pk, stream=None):
-        import torch
         ntab = len(self.tables)
-        full = torch.zeros((self.nspec, ntab, int(self.n_fft.max())), dtype=torch.float64, device=k.device)
+        full = self._outputs([(None, (self.nspec, ntab, int(self.n_fft.max())))], stream)[0].zero_()
         self._check_io(k, pk, None, None, None)
         check(self.L.coffe_batch_tables(self.h, _ptr(k), _ptr(pk), _ptr(full),
                                         stream if stream is not None else self._stream()), "coffe_batch_tables")
@@ -472,8 +506,8 @@ def mu_weights_jvp(engine, bg, tangent, bias_z, bias1, bias2, zmean, ls, tables,
     if terms is None:
         terms = terms_of(den, rsd, d1)
     shape = (len(zm), len(ls), len(tables), len(sp))
-    A = torch.empty(shape, dtype=torch.float64, device="cuda")
-    At = torch.empty(shape, dtype=torch.float64, device="cuda")
+    A, At = engine.empty(shape, shape) if stream is None else \
+        [torch.empty(shape, dtype=torch.float64, device="cuda") for _ in range(2)]
     st = stream if stream is not None else ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     check(L.coffe_mu_weights_jvp(engine.h, ctypes.byref(inp), ctypes.byref(tan), int(terms), int(flatsky), 0,
                                  len(zm), zm.ctypes.data_as(dp), len(ls), ls_c, len(tables), tn_c, tl_c, len(sp),
@@ -587,8 +621,11 @@ def mu_weights(engine, bg, bias_z, bias1, bias2, zmean, ls, tables, sep, den=Tru
     if terms is None:
         terms = terms_of(den, rsd, d1, dg is not None)
     shape = (len(zm), len(ls), len(tables)) if paired else (len(zm), len(ls), len(tables), len(sp))
-    A = out if out is not None else torch.empty(shape, dtype=torch.float64, device="cuda")
-    _need(A, shape, "A")
+    if out is not None:
+        A = out
+        _need(A, shape, "A")
+    else:
+        A, = engine.empty(shape) if stream is None else [torch.empty(shape, dtype=torch.float64, device="cuda")]
     if ren_out is not None:
         _need(ren_out, shape[:2] if paired else (len(zm), len(ls), len(sp)), "ren_out")
     st = stream if stream is not None else ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)

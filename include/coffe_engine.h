@@ -334,6 +334,7 @@ int coffe_divergent_tables_device(coffe_engine *e, const double *d_k, const doub
 int coffe_integral_table(int n, int l, size_t N, const double *k, const double *pk, size_t nin, double kmin,
                          double kmax, double *out_x, double *out_y);
 
+
 /*
  * The same table with the reference's integer states (integrals.c:186-207, enum
  * coffe_integer_state of integrals.h:23: 0 COFFE_INTEGER, 1 COFFE_HALF_INTEGER): with
@@ -463,6 +464,8 @@ int coffe_integrated_corrfunc(const coffe_mu_inputs *in, unsigned flags, int nta
                               const double *ren0_x, const double *ren0_y, int nz, const double *zmean, int nmu,
                               const double *mu, int nsep, const double *sep, const int *rule, double *out);
 
+/* the engine's own stream (a hipStream_t), on which the calls given a NULL stream run */
+void *coffe_engine_stream(coffe_engine *e);
 /* synchronise the engine's stream */
 int coffe_engine_synchronize(coffe_engine *e);
 
