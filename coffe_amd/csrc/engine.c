@@ -450,6 +450,37 @@ static int cmp_unit(const void *a, const void *b)
     return x->idx - y->idx;
 }
 
+/*
+ * Input intervals per spline chunk (one wavefront of k_resample and k_spline_adj each): `points`
+ * grid points' worth of a spectrum of n samples on N grid points, 512 at most.  A chunk stages
+ * and solves its own system (about 12 us) and then takes about 1 us per 64 points, so
+ * chunks of two points a lane are best while all of them run at once, and the fewest chunks
+ * once they do not: points starts at 128 and doubles until at most CHUNK_FILL chunks
+ * (15 a CU are resident) are left.  600 samples on 10000 points: 66 us in chunks of 512
+ * intervals, 10 us in these.
+ */
+#define CHUNK_FILL 3840
+static int chunk_len(int64_t n, int64_t N, int64_t points)
+{
+    const double c = ceil((double)(n - 1) * (double)points / (double)N);
+    return c < 8 ? 8 : (c > CE_CHUNK ? CE_CHUNK : (int)c);
+}
+
+static int64_t chunk_points(int nspec, const int64_t *n_in, const int64_t *n_fft)
+{
+    int64_t points = 128;
+    for (;; points *= 2) {
+        int64_t total = 0;
+        int most = 1;   /* every chunk at its largest */
+        for (int s = 0; s < nspec; ++s) {
+            const int c = chunk_len(n_in[s], n_fft[s], points);
+            total += (n_in[s] - 1 + c - 1) / c;
+            if (c < CE_CHUNK) most = 0;
+        }
+        if (most || total <= CHUNK_FILL || points > ((int64_t)1 << 40)) return points;
+    }
+}
+
 int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const int64_t *n_fft, const double *kmin,
                        const double *kmax, int ntab, const int *tab_n, const int *tab_l, int nsep, const double *sep,
                        int nz, int nl, coffe_batch **out)
@@ -476,7 +507,7 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
     int32_t *spec_grid = (int32_t *)calloc((size_t)nspec, sizeof(int32_t));
     if (!b->grids || !b->h_spec || !spec_grid) { free(spec_grid); coffe_batch_destroy(b); return COFFE_ENOMEM; }
     int st = COFFE_OK;
-    int64_t in_off = 0, xf_off = 0, xb_off = 0, ws_off = 0;
+    int64_t in_off = 0, xf_off = 0, xb_off = 0, ws_off = 0, points = 0;
     for (int s = 0; s < nspec && st == COFFE_OK; ++s) {
         if (n_in[s] < 5 || n_fft[s] < 4 || n_fft[s] > 16384) { st = n_in[s] < 5 ? COFFE_EINVAL : COFFE_EUNSUPPORTED; break; }
         ce_grid *g = NULL;
@@ -502,7 +533,6 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
         xf_off += (int64_t)g->nq * (M + 1);
         xb_off += (int64_t)ntab * (M + 1);
         ws_off += 2 * (int64_t)g->N;
-        b->nchunk += (int)((n_in[s] - 1 + CE_CHUNK - 1) / CE_CHUNK);
     }
     b->total_in = in_off;
     /* every FFT pass needs at least M/8 threads (at most 4 butterflies each) */
@@ -531,12 +561,17 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
     }
     ce_chunk_dev *chunks = NULL;
     if (st == COFFE_OK) {
+        points = chunk_points(nspec, n_in, n_fft);
+        for (int s = 0; s < nspec; ++s) {
+            const int len = chunk_len(n_in[s], n_fft[s], points);
+            b->nchunk += (int)((n_in[s] - 1 + len - 1) / len);
+        }
         chunks = (ce_chunk_dev *)malloc(sizeof(ce_chunk_dev) * (size_t)b->nchunk);
         if (!chunks) st = COFFE_ENOMEM;
         int c = 0;
         for (int s = 0; s < nspec && st == COFFE_OK; ++s) {
-            const int nint = (int)n_in[s] - 1;
-            for (int a = 0; a < nint; a += CE_CHUNK) {
+            const int nint = (int)n_in[s] - 1, len = chunk_len(n_in[s], n_fft[s], points);
+            for (int a = 0; a < nint; a += len) {
                 chunks[c].spec = s;
                 chunks[c].grid = b->h_spec[s].grid;
                 chunks[c].in_off = b->h_spec[s].in_off;
@@ -544,7 +579,7 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
                 chunks[c].n_in = b->h_spec[s].n_in;
                 chunks[c].id = c;
                 chunks[c].a = a;
-                chunks[c].b = a + CE_CHUNK < nint ? a + CE_CHUNK : nint;
+                chunks[c].b = a + len < nint ? a + len : nint;
                 ++c;
             }
         }
@@ -881,7 +916,9 @@ int twofast_1bessel_status(double *output_x, double *output_y, size_t output_len
     }
     /* scratch layout: k, P | ws (2N) | xf (M+1 cplx; N cplx on the general path) | out (N) |
        spec, grid, tab, unit, chunks */
-    const int nchunk = (int)((n - 1 + CE_CHUNK - 1) / CE_CHUNK);
+    const int64_t n_in1 = (int64_t)n, n_fft1 = N;
+    const int len = chunk_len(n_in1, n_fft1, chunk_points(1, &n_in1, &n_fft1));
+    const int nchunk = (int)((n - 1 + (size_t)len - 1) / (size_t)len);
     const size_t off_k = 0, off_p = n, off_ws = 2 * n, off_xf = off_ws + 2 * (size_t)N;
     const size_t off_out = off_xf + 2 * (size_t)(general ? N : M + 1), off_meta = off_out + (size_t)N;
     const size_t meta_bytes = sizeof(ce_spec_dev) + sizeof(ce_grid_dev) + sizeof(ce_table_desc) +
@@ -905,8 +942,8 @@ int twofast_1bessel_status(double *output_x, double *output_y, size_t output_len
         h_chunks[c].ws_off = 0;
         h_chunks[c].n_in = (int32_t)n;
         h_chunks[c].id = c;
-        h_chunks[c].a = c * CE_CHUNK;
-        h_chunks[c].b = (c + 1) * CE_CHUNK < (int)n - 1 ? (c + 1) * CE_CHUNK : (int)n - 1;
+        h_chunks[c].a = c * len;
+        h_chunks[c].b = (c + 1) * len < (int)n - 1 ? (c + 1) * len : (int)n - 1;
     }
     ce_spec_dev hs;
     memset(&hs, 0, sizeof(hs));
@@ -1592,12 +1629,12 @@ static int integral_table_any(double n, double l, size_t N, const double *k, con
     if (st != COFFE_OK) return st;
     st = check_small_r_status(h_stat, nodes);
     if (st != COFFE_OK) return st;
+    out_x[0] = 0.0;
     static const double min_sep[CE_MIN_SEP_LEN] = {
         1E-6, 1E-5, 1E-4, 1E-3, 2E-3, 5E-3, 7E-3, 8E-3, 9E-3, 1E-2, 1.1E-2, 1.2E-2, 1.25E-2, 1.3E-2,
         1.35E-2, 1.5E-2, 2E-2, 2.5E-2, 3E-2, 3.5E-2, 5E-2, 7E-2, 8E-2, 9E-2, 1E-1, 1.1E-1, 1.2E-1,
         1.25E-1, 1.3E-1, 1.35E-1, 1.5E-1, 1.75E-1, 2E-1, 2.5E-1, 3E-1, 3.5E-1, 4E-1, 5E-1, 6E-1,
         7E-1, 8E-1, 9E-1};
-    out_x[0] = 0.0;
     for (size_t i = 0; i < CE_MIN_SEP_LEN; ++i) out_x[1 + i] = min_sep[i];
     return COFFE_OK;
 }
