@@ -780,11 +780,10 @@ class Coffe:
         """The 8 default tables (integrals.c:580-660), each the reference's N + 43 nodes."""
         self._need_pk()
         if self._tables is None:
-            from .engine import integral_table
+            from .engine import integral_tables
             k, pk = self._pk
-            N = self._p["integrals_fftlog_sampling"]
             kmin, kmax = self._kwin()
-            self._tables = {t: integral_table(t[0], t[1], k, pk, N, kmin, kmax) for t in TABLES}
+            self._tables = integral_tables(TABLES, k, pk, self._p["integrals_fftlog_sampling"], kmin, kmax)
         return self._tables
 
     def _divergent_table(self):
@@ -1088,12 +1087,13 @@ class Coffe:
         """[z][l][r] multipoles of the full-sky integrated terms: (2 l + 1) / 2 int dmu
         P_l(mu) xi(mu) (signal.c:143-230, 664-672, 743-752), mu = cos(theta) with theta on
         an INTEGRATED_MU_NODES-point Gauss-Legendre rule; None without such terms."""
+        plan = self._lensing_plan()
+        if plan is None or plan["flags"] is None:
+            return None
         t, w = np.polynomial.legendre.leggauss(self.INTEGRATED_MU_NODES)
         theta = np.pi / 2 * (t + 1)
         mus, wm = np.cos(theta), np.pi / 2 * w * np.sin(theta)
         xi = self._integrated_corrfunc(zs, seps, mus)
-        if xi is None:
-            return None
         out = np.empty((len(zs), len(ls), len(seps)))
         for il, l in enumerate(ls):
             pl = np.polynomial.legendre.legval(mus, [0] * int(l) + [1])

@@ -34,6 +34,9 @@ struct coffe_engine {
     void *h_pinned[2];
     size_t pinned_bytes[2];
     int stage_next;
+    /* pinned host memory for the download of several tables (under the lock) */
+    void *h_down;
+    size_t down_bytes;
     /* asynchronous users of the scratch: ev_scratch follows the last kernel that reads
        it, ev_stage[i] the last copy out of staging buffer i (valid when *_pending) */
     hipEvent_t ev_scratch, ev_stage[2];

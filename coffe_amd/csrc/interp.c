@@ -5,7 +5,6 @@
  * (common.c:524-576, 704-710).  Out-of-range points give NaN.
  */
 #include <math.h>
-#include <stdlib.h>
 
 #include "coffe_engine.h"
 
@@ -19,38 +18,40 @@ static size_t bsearch_lo(const double *x, double v, size_t lo, size_t hi)
     return lo;
 }
 
+/* the slope of interval i of n nodes, extended linearly beyond the ends */
+static double slope(size_t n, const double *x, const double *y, long i)
+{
+    const long last = (long)n - 2;
+    if (i >= 0 && i <= last) return (y[i + 1] - y[i]) / (x[i + 1] - x[i]);
+    const long e = i < 0 ? 0 : last, in = i < 0 ? 1 : last - 1;   /* the end interval and its neighbour */
+    const double m0 = (y[e + 1] - y[e]) / (x[e + 1] - x[e]), m1 = (y[in + 1] - y[in]) / (x[in + 1] - x[in]);
+    return (i == -1 || i == last + 1) ? 2.0 * m0 - m1 : 3.0 * m0 - 2.0 * m1;
+}
+
+/* the coefficients are made for the queries' intervals only: the API reads a few hundred values of
+   tables of 10^4 nodes */
 int coffe_akima_eval(size_t n, const double *x, const double *y, size_t nq, const double *xq, double *out)
 {
     if (n < 5 || !x || !y || (nq && (!xq || !out))) return COFFE_EINVAL;
-    double *buf = (double *)malloc(sizeof(double) * (4 * n + 4));
-    if (!buf) return COFFE_ENOMEM;
-    double *m = buf + 2, *b = buf + n + 4, *c = b + n, *d = c + n;
-    for (size_t i = 0; i + 1 < n; ++i) m[i] = (y[i + 1] - y[i]) / (x[i + 1] - x[i]);
-    m[-2] = 3.0 * m[0] - 2.0 * m[1];
-    m[-1] = 2.0 * m[0] - m[1];
-    m[n - 1] = 2.0 * m[n - 2] - m[n - 3];
-    m[n] = 3.0 * m[n - 2] - 2.0 * m[n - 3];
-    for (long i = 0; i + 1 < (long)n; ++i) {
-        const double ne = fabs(m[i + 1] - m[i]) + fabs(m[i - 1] - m[i - 2]);
-        if (ne == 0.0) {
-            b[i] = m[i]; c[i] = 0.0; d[i] = 0.0;
-            continue;
-        }
-        const double h = x[i + 1] - x[i];
-        const double nn = fabs(m[i + 2] - m[i + 1]) + fabs(m[i] - m[i - 1]);
-        const double al = fabs(m[i - 1] - m[i - 2]) / ne;
-        const double tn = nn == 0.0 ? m[i] : (1.0 - fabs(m[i] - m[i - 1]) / nn) * m[i] + fabs(m[i] - m[i - 1]) / nn * m[i + 1];
-        b[i] = (1.0 - al) * m[i - 1] + al * m[i];
-        c[i] = (3.0 * m[i] - 2.0 * b[i] - tn) / h;
-        d[i] = (b[i] + tn - 2.0 * m[i]) / (h * h);
-    }
     for (size_t q = 0; q < nq; ++q) {
         const double v = xq[q];
         if (!(v >= x[0] && v <= x[n - 1])) { out[q] = NAN; continue; }
-        const size_t i = bsearch_lo(x, v, 0, n - 1);
+        const long i = (long)bsearch_lo(x, v, 0, n - 1);
+        double m[5];   /* the slopes of intervals i - 2 ... i + 2 */
+        for (int j = 0; j < 5; ++j) m[j] = slope(n, x, y, i - 2 + j);
+        const double ne = fabs(m[3] - m[2]) + fabs(m[1] - m[0]);
+        double b = m[2], c = 0.0, d = 0.0;
+        if (ne != 0.0) {
+            const double h = x[i + 1] - x[i];
+            const double nn = fabs(m[4] - m[3]) + fabs(m[2] - m[1]);
+            const double al = fabs(m[1] - m[0]) / ne;
+            const double tn = nn == 0.0 ? m[2] : (1.0 - fabs(m[2] - m[1]) / nn) * m[2] + fabs(m[2] - m[1]) / nn * m[3];
+            b = (1.0 - al) * m[1] + al * m[2];
+            c = (3.0 * m[2] - 2.0 * b - tn) / h;
+            d = (b + tn - 2.0 * m[2]) / (h * h);
+        }
         const double dx = v - x[i];
-        out[q] = y[i] + dx * (b[i] + dx * (c[i] + d[i] * dx));
+        out[q] = y[i] + dx * (b + dx * (c + d * dx));
     }
-    free(buf);
     return COFFE_OK;
 }

@@ -256,6 +256,24 @@ def integral_table(n, l, k, pk, N, kmin=None, kmax=None):
     return ox, oy
 
 
+def integral_tables(tables, k, pk, N, kmin=None, kmax=None):
+    """{(n, l): (x, y)} for several of integral_table's tables of one spectrum, in one call
+    (coffe_integral_tables); host arrays."""
+    L = load_library()
+    k = np.ascontiguousarray(k, dtype=np.float64)
+    pk = np.ascontiguousarray(pk, dtype=np.float64)
+    kmin = float(k[0]) if kmin is None else kmin
+    kmax = float(k[-1]) if kmax is None else kmax
+    tables = list(tables)
+    ox, oy = np.empty(N + 43), np.empty((len(tables), N + 43))
+    dp = ctypes.POINTER(ctypes.c_double)
+    tn = (ctypes.c_int * len(tables))(*[int(t[0]) for t in tables])
+    tl = (ctypes.c_int * len(tables))(*[int(t[1]) for t in tables])
+    check(L.coffe_integral_tables(len(tables), tn, tl, int(N), k.ctypes.data_as(dp), pk.ctypes.data_as(dp), len(k), kmin,
+                                  kmax, ox.ctypes.data_as(dp), oy.ctypes.data_as(dp)), "coffe_integral_tables")
+    return {t: (ox, oy[i]) for i, t in enumerate(tables)}
+
+
 def integral_table_state(n, l, state_n, state_l, k, pk, N, kmin=None, kmax=None):
     """The full (N + 43)-point table with the reference's integer states
     (coffe_integral_table_state; state 1 = half-integer: the table of (n/2, l/2)); host

@@ -333,6 +333,9 @@ int coffe_divergent_tables_device(coffe_engine *e, const double *d_k, const doub
 
 int coffe_integral_table(int n, int l, size_t N, const double *k, const double *pk, size_t nin, double kmin,
                          double kmax, double *out_x, double *out_y);
+/* ntab such tables (1..8) of one spectrum in one call: out_x [N + 43], out_y [ntab][N + 43] */
+int coffe_integral_tables(int ntab, const int *n, const int *l, size_t N, const double *k, const double *pk,
+                          size_t nin, double kmin, double kmax, double *out_x, double *out_y);
 
 
 /*
