@@ -265,6 +265,18 @@ int ce_launch_mu_weights_jvp(void *stream, const ce_mu_dev *in, const ce_mu_tan 
 #define CE_INTG_VAL 4         /* doubles per Akima value record {y, b, c, d} */
 #define CE_INTG_PAIR 2        /* doubles per node pair {x_j, x_(j+1)} */
 #define CE_INTG_NBGC 5        /* background curves with value records */
+#define CE_INTG_POINTS 65536  /* (z, mu, r) points a pass: their end-point values stand in device memory */
+#define CE_INTG_POINT 24      /* doubles a point */
+#define CE_INTG_WIDE 32       /* doubles per node of the records of tables that share their nodes */
+#define CE_INTG_BGW 16        /* doubles per node of the background curves on bg_z */
+#define CE_INTG_ZOF 8         /* doubles per node of z against chi */
+/* doubles of the workspace coef: ntab_values table nodes in all, nshared of them shared
+   by the standard tables (0: none) */
+static inline size_t ce_intg_coef_len(size_t ntab_values, size_t nshared, size_t nbg)
+{
+    return CE_INTG_WIDE * nshared + (CE_INTG_BGW + CE_INTG_ZOF) * nbg + CE_INTG_VAL * ntab_values +
+           CE_INTG_PAIR * (ntab_values + nbg);
+}
 typedef struct ce_intg_dev {
     int nbg;
     const double *bg_z, *bg_chi, *bg_D1, *bg_a, *bg_f, *bg_cH, *bg_G1, *bg_G2;
@@ -282,12 +294,14 @@ typedef struct ce_intg_dev {
     int tab_ref;   /* a slot whose nodes every present standard table shares, or -1 */
     int nguess;
     const double *chi_guess;
-    /* workspace of (CE_INTG_VAL + CE_INTG_PAIR) (ntab_values + CE_INTG_NBGC nbg)
-       doubles, 64-byte aligned, for the Akima value records and node pairs, and
+    /* workspace of ce_intg_coef_len doubles, 256-byte aligned, for the Akima value
+       records and node pairs, and
        CE_INTG_ARGS_BYTES of device memory for the kernel's arguments */
     int ntab_values;
     double *coef;
     void *args_dev;
+    /* CE_INTG_POINT doubles for each of up to CE_INTG_POINTS points */
+    double *points;
     int nren0;
     const double *ren0_x, *ren0_y;
     int nren;

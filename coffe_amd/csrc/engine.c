@@ -2023,13 +2023,27 @@ int coffe_integrated_corrfunc(const coffe_mu_inputs *in, unsigned flags, int nta
     const size_t nren = want_ren ? (size_t)in->nren : 0, nnode = nren * nren, n0 = want_ren ? (size_t)nren0 : 0;
     const size_t ngl = 2 * (size_t)(r[1] + r[3] + r[5]), nout = 2 * (size_t)nz * nmu * nsep;
     const int nguess = 4096;
-    /* the Akima value records and node pairs, and 7 doubles of slack to align them to
-       64 bytes */
-    const size_t nrec = (CE_INTG_VAL + CE_INTG_PAIR) * ((size_t)total_tab + CE_INTG_NBGC * nbg) + 7;
+    /* one interval serves every standard table when they share their nodes (the tables of
+       one spectrum and one N do) */
+    int tab_ref = -1;
+    for (int t = 0; t < CE_INTG_NSLOT - 1; ++t) {
+        if (len[t] < 5) continue;
+        if (tab_ref < 0) {
+            tab_ref = t;
+        } else if (len[t] != len[tab_ref] ||
+                   memcmp(tab_x + off[t], tab_x + off[tab_ref], sizeof(double) * (size_t)len[t]) != 0) {
+            tab_ref = -1;
+            break;
+        }
+    }
+    /* the Akima value records and node pairs, and 31 doubles of slack to align them to
+       256 bytes */
+    const size_t nrec = ce_intg_coef_len((size_t)total_tab, tab_ref < 0 ? 0 : (size_t)len[tab_ref], nbg) + 31;
+    const size_t npts = CE_INTG_POINT * (nout / 2 < CE_INTG_POINTS ? nout / 2 : CE_INTG_POINTS);
     const size_t total = 8 * nbg + 3 * nb + 5 * nmb + 2 * (size_t)total_tab + 2 * n0 + nren + 4 * nnode +
-                         (size_t)nz + (size_t)nmu + (size_t)nsep + ngl + (size_t)nguess + 2 + nout + nrec +
+                         (size_t)nz + (size_t)nmu + (size_t)nsep + ngl + (size_t)nguess + 2 + nout + nrec + npts +
                          CE_INTG_ARGS_BYTES / sizeof(double);
-    double *h = (double *)malloc(sizeof(double) * (total - nout - nrec - CE_INTG_ARGS_BYTES / sizeof(double)));
+    double *h = (double *)malloc(sizeof(double) * (total - nout - nrec - npts - CE_INTG_ARGS_BYTES / sizeof(double)));
     double *work = (double *)malloc(sizeof(double) * (2 * nren + 2));
     double *planes = (double *)malloc(sizeof(double) * (4 * nnode + 1));
     if (!h || !work || !planes) {
@@ -2087,19 +2101,6 @@ int coffe_integrated_corrfunc(const coffe_mu_inputs *in, unsigned flags, int nta
             dv.tab_lsc[t] = (double)(n - 1 - f0) / (log(x[n - 1]) - log(x[f0]));
         }
     }
-    /* one interval serves every standard table when they share their nodes (the tables of
-       one spectrum and one N do) */
-    dv.tab_ref = -1;
-    for (int t = 0; t < CE_INTG_NSLOT - 1; ++t) {
-        if (len[t] < 5) continue;
-        if (dv.tab_ref < 0) {
-            dv.tab_ref = t;
-        } else if (len[t] != len[dv.tab_ref] ||
-                   memcmp(tab_x + off[t], tab_x + off[dv.tab_ref], sizeof(double) * (size_t)len[t]) != 0) {
-            dv.tab_ref = -1;
-            break;
-        }
-    }
     /* guesses of bg_chi's interval on a uniform chi grid */
     {
         double *g = h + o;
@@ -2153,8 +2154,10 @@ int coffe_integrated_corrfunc(const coffe_mu_inputs *in, unsigned flags, int nta
 #undef IG_PUT
     double *d_out = d + o;
     dv.ntab_values = (int)total_tab;
-    dv.coef = (double *)(((uintptr_t)(d_out + nout) + 63) & ~(uintptr_t)63);
+    dv.tab_ref = tab_ref;
+    dv.coef = (double *)(((uintptr_t)(d_out + nout) + 255) & ~(uintptr_t)255);
     dv.args_dev = d_out + nout + nrec;
+    dv.points = d_out + nout + nrec + CE_INTG_ARGS_BYTES / sizeof(double);
     hipStream_t s = e->stream;
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(d, h, sizeof(double) * o, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK && ce_launch_integrated(s, &dv, flags, nz, d_z, nmu, d_mu, nsep, d_sep, r, d_gl, d_out))

@@ -32,34 +32,51 @@ constexpr unsigned F_DEN = 1u << 0, F_RSD = 1u << 1, F_D1 = 1u << 2, F_D2 = 1u <
                    F_G2 = 1u << 5, F_G3 = 1u << 6, F_LEN = 1u << 7, F_G4 = 1u << 8, F_G5 = 1u << 9,
                    F_ONLY_CROSS = 1u << 10, F_FLAT_LL = 1u << 11, F_FLAT_DL = 1u << 12;
 
+// A pointer into device memory that is read from device memory itself: typed, so that the
+// loads through it are global ones (through a generic pointer they are flat loads,
+// which occupy the LDS path as well and cannot be scalar)
+struct gmem {
+    const __attribute__((address_space(1))) double *p;
+    __host__ __device__ operator const double *() const { return (const double *)p; }
+    gmem &operator=(const double *q)
+    {
+        p = (const __attribute__((address_space(1))) double *)q;
+        return *this;
+    }
+};
+
 struct intg_args {
     int nbg;
-    const double *bg_z, *bg_chi, *bg_D1, *bg_a, *bg_f, *bg_cH, *bg_G1, *bg_G2;
+    gmem bg_z, bg_chi, bg_D1, bg_a, bg_f, bg_cH, bg_G1, bg_G2;
     int nb;
-    const double *bias_z, *b1, *b2;
+    gmem bias_z, b1, b2;
     int nmb;
-    const double *mb_z, *s1, *s2, *fe1, *fe2;
-    const double *tab_x, *tab_y;
+    gmem mb_z, s1, s2, fe1, fe2;
+    gmem tab_x, tab_y;
     int tab_off[NSLOT], tab_len[NSLOT];
     int tab_f0[NSLOT];                 // first node of the log-uniform part (-1: bisection)
     int tab_ref;                       // a slot whose nodes every present standard table shares (-1: none)
     double tab_lx0[NSLOT], tab_lsc[NSLOT];   // its log(x[f0]) and nodes per unit of log x
     int nguess;                        // chi -> interval guesses on [0, chi_max], nguess + 1 of them
-    const double *chi_guess;
-    // Akima value records and node pairs (below): the tables' in the layout of tab_y,
-    // the background curves' [NBGC][nbg]
-    const double *tab_val, *tab_pair, *bgc_val, *bgc_pair;
+    gmem chi_guess;
+    // Akima value records and node pairs (below)
+    gmem tab_val[NSLOT];      // table s's records, tab_stride[s] doubles apart
+    int tab_stride[NSLOT];
+    gmem tab_pair;            // in the layout of tab_y
+    gmem tab_wide;            // the shared-node tables' records, WIDE a node (if tab_ref >= 0)
+    gmem bgc_wide, bgz_pair; // D1, a, f, conformal H: BGW a node; bg_z's node pairs
+    gmem zof;                 // z against chi: {x_j, x_(j+1), y, b, c, d, 0, 0} a node
     int nren0;
-    const double *ren0_x, *ren0_y;
+    gmem ren0_x, ren0_y;
     int nren;
-    const double *ren_chi;
-    const double *ren_rec;   // per grid node (x fastest): {value, d/dx, d/dy, d2/dxdy}
+    gmem ren_chi;
+    gmem ren_rec;   // per grid node (x fastest): {value, d/dx, d/dy, d2/dxdy}
     double Om, H0h;
     unsigned flags;
     int nz, nmu, nsep;
-    const double *zmean, *mu, *sep;
+    gmem zmean, mu, sep;
     int p1, n1, pu, nu, ps, ns;
-    const double *g1x, *g1w, *gux, *guw, *gsx, *gsw;   // Gauss-Legendre rules on [-1, 1]
+    gmem g1x, g1w, gux, guw, gsx, gsw;   // Gauss-Legendre rules on [-1, 1]
     double *out;                                       // [nz][nmu][nsep][2]: single, double
 };
 
@@ -68,11 +85,14 @@ __device__ inline double ak(const double *x, const double *y, int n, double v) {
 // An Akima lookup reads two arrays: node pairs {x_j, x_(j+1)} (16 bytes, one load: both
 // ends of interval j, which also test a guessed interval), shared by the curves on one
 // grid, and each curve's value records {y_j, b_j, c_j, d_j} (32 bytes, two loads).  The
-// lookups of this kernel gather at random per lane, so the L1 cache's throughput in
-// cache lines, not arithmetic, bounds them: separate node and coefficient arrays cost
-// five scattered lines per lookup, this layout three, and two for each further curve
-// or table on the same interval.
-constexpr int VAL = CE_INTG_VAL, PAIR = CE_INTG_PAIR;
+// curves of one grid keep their records side by side: the eight standard tables 256 bytes
+// a node (two lines), D1, a, conformal H and f 128 bytes, z(chi) 64 with its node pair, so
+// a lookup of all of them moves whole lines, and k_integrated_double fetches them
+// a line at a time (below).
+constexpr int VAL = CE_INTG_VAL, PAIR = CE_INTG_PAIR, WIDE = CE_INTG_WIDE, BGW = CE_INTG_BGW, ZOF = CE_INTG_ZOF;
+// the place of each shared-node table in the record of a node: the two halves are what
+// the double integral's fetches take
+constexpr int WSLOT[NSLOT - 1] = {0, 3, 5, 2, 4, 1, 7, 6};
 struct nodes {
     double x0, x1;
 };
@@ -91,13 +111,14 @@ __device__ __forceinline__ bool pair_hit(const nodes &g, int j, int n, double v)
     return g.x0 <= v && (j == n - 2 || v < g.x1);
 }
 
-// y(xq) on the segment of interval j with lower node x0 (the value akima_at gives there)
-__device__ __forceinline__ double val_at(const double *__restrict__ r, int j, double x0, double xq)
+// y(xq) on the segment of record r with lower node x0 (the value akima_at gives there)
+__device__ __forceinline__ double cubic(double2 p, double2 q, double dx)
 {
-    const double2 p = *reinterpret_cast<const double2 *>(r + (size_t)VAL * j),
-                  q = *reinterpret_cast<const double2 *>(r + (size_t)VAL * j + 2);
-    const double dx = xq - x0;
     return p.x + dx * (p.y + dx * (q.x + q.y * dx));
+}
+__device__ __forceinline__ double val_at(const double *__restrict__ r, double x0, double xq)
+{
+    return cubic(*reinterpret_cast<const double2 *>(r), *reinterpret_cast<const double2 *>(r + 2), xq - x0);
 }
 
 // The lookups: Akima of raw nodes as ce::akima_general, with the interval found from a
@@ -131,45 +152,38 @@ struct lk {
         const int g = bg_guess(z);
         return g < 0 ? -1 : ce::interval_from(a.bg_z, a.nbg, z, g);
     }
-    // curve k's value records, and the node pairs of its grid (bg_z for D1, a, f and
-    // conformal H; bg_chi for z(chi))
-    __device__ const double *bgv(int k) const { return a.bgc_val + (size_t)VAL * k * a.nbg; }
-    __device__ const double *bgp(int k) const
-    {
-        return a.bgc_pair + (size_t)PAIR * (k == C_ZOF ? C_ZOF : C_D1) * a.nbg;
-    }
+    // the node pair of bg_z's interval j, and curve k's value record there
+    __device__ nodes bgz(int j) const { return pair_at(a.bgz_pair, j); }
+    __device__ const double *bgv(int k, int j) const { return a.bgc_wide + (size_t)BGW * j + VAL * k; }
     // D1, a, f or conformal H (curve k) in interval j (NaN for j < 0)
     __device__ double bgcj(int k, int j, double z) const
     {
-        return j < 0 ? __builtin_nan("") : val_at(bgv(k), j, pair_at(bgp(k), j).x0, z);
+        return j < 0 ? __builtin_nan("") : val_at(bgv(k, j), bgz(j).x0, z);
     }
-    // curve k at z, the interval found from the guess; *jz (if given) receives it
-    __device__ double bgc(int k, double z, int *jz = nullptr) const
-    {
-        int j = bg_guess(z);
-        double v = __builtin_nan("");
-        if (j >= 0) {
-            const nodes g = pair_at(bgp(k), j);
-            v = val_at(bgv(k), j, g.x0, z);
-            if (!pair_hit(g, j, a.nbg, z)) {
-                j = ce::interval_from(a.bg_z, a.nbg, z, j);
-                v = bgcj(k, j, z);
-            }
-        }
-        if (jz) *jz = j;
-        return v;
-    }
-    __device__ double z_of(double chi) const
+    // curve k at z
+    __device__ double bgc(int k, double z) const { return bgcj(k, bg_interval(z), z); }
+    // the first guess of chi's interval on bg_chi (-1 outside it)
+    __device__ int zof_guess(double chi) const
     {
         const double *x = a.bg_chi;
         const int n = a.nbg;
-        if (!(chi >= x[0] && chi <= x[n - 1])) return __builtin_nan("");
+        if (!(chi >= x[0] && chi <= x[n - 1])) return -1;
         const int k = ce::clamp_index(chi / x[n - 1] * a.nguess, a.nguess + 1);
-        const int j = below_last(max((int)a.chi_guess[k], 0), n);
-        const nodes g = pair_at(bgp(C_ZOF), j);
-        const double v = val_at(bgv(C_ZOF), j, g.x0, chi);
-        if (pair_hit(g, j, n, chi)) return v;
-        return bgcj(C_ZOF, ce::interval_from(x, n, chi, j), chi);
+        return below_last(max((int)a.chi_guess[k], 0), n);
+    }
+    __device__ double zofj(int j, double chi) const
+    {
+        const double *r = a.zof + (size_t)ZOF * j;
+        return val_at(r + 2, r[0], chi);
+    }
+    __device__ double z_of(double chi) const
+    {
+        const int j = zof_guess(chi);
+        if (j < 0) return __builtin_nan("");
+        const double *r = a.zof + (size_t)ZOF * j;
+        const nodes g = pair_at(r, 0);
+        if (pair_hit(g, j, a.nbg, chi)) return val_at(r + 2, g.x0, chi);
+        return zofj(ce::interval_from(a.bg_chi, a.nbg, chi, j), chi);
     }
     // a first interval of r on table s's nodes (-1: r outside them): by bisection below
     // the log-uniform part (exact), from the log above it (a guess)
@@ -182,7 +196,7 @@ struct lk {
         if (r < x[f0]) return ce::interval_bisect(x, 0, f0, r);
         return below_last(f0 + ce::clamp_index((log(r) - a.tab_lx0[s]) * a.tab_lsc[s], n - f0), n);
     }
-    __device__ const double *tabv(int s) const { return a.tab_val + (size_t)VAL * a.tab_off[s]; }
+    __device__ const double *tabv(int s, int j) const { return a.tab_val[s] + (size_t)a.tab_stride[s] * j; }
     __device__ const double *tabp(int s) const { return a.tab_pair + (size_t)PAIR * a.tab_off[s]; }
     // interval j of table s settled from its guess g (-1 stays -1); *x0 its lower node
     __device__ int tab_settle(int s, int g, double r, double *x0) const
@@ -201,10 +215,10 @@ struct lk {
         const int g = tab_guess(s, r);
         if (g < 0) return __builtin_nan("");
         const nodes nd = pair_at(tabp(s), g);
-        const double v = val_at(tabv(s), g, nd.x0, r);
+        const double v = val_at(tabv(s, g), nd.x0, r);
         if (pair_hit(nd, g, a.tab_len[s], r)) return v;
         const int j = ce::interval_from(a.tab_x + a.tab_off[s], a.tab_len[s], r, g);
-        return val_at(tabv(s), j, pair_at(tabp(s), j).x0, r);
+        return val_at(tabv(s, j), pair_at(tabp(s), j).x0, r);
     }
     // the interval of r on the standard tables' shared nodes (-1: none shared, or r
     // outside them) and its lower node; a standard table's value there
@@ -214,7 +228,7 @@ struct lk {
     }
     __device__ double tabj(int s, int j, double x0, double r) const
     {
-        return j < 0 ? tab(s, r) : val_at(tabv(s), j, x0, r);
+        return j < 0 ? tab(s, r) : val_at(tabv(s, j), x0, r);
     }
     // GSL interp2d bicubic of the renormalisation grid at (x, y) (node derivatives of
     // natural cubic splines, Hermite patches; common.c:712-719)
@@ -226,20 +240,25 @@ struct lk {
         const int i = ce::interval_from(c, n, x, ce::interval_guess(c, n, x));
         const int j = ce::interval_from(c, n, y, ce::interval_guess(c, n, y));
         const double dx = c[i + 1] - c[i], dy = c[j + 1] - c[j];
-        const double t = (x - c[i]) / dx, u = (y - c[j]) / dy;
-        const double ht[4] = {(1 + 2 * t) * (1 - t) * (1 - t), t * t * (3 - 2 * t), t * (1 - t) * (1 - t),
-                              t * t * (t - 1)};
-        const double hu[4] = {(1 + 2 * u) * (1 - u) * (1 - u), u * u * (3 - 2 * u), u * (1 - u) * (1 - u),
-                              u * u * (u - 1)};
+        double2 q[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+            q[m] = *reinterpret_cast<const double2 *>(a.ren_rec + 4 * ((size_t)(j + m / 4) * n + i) + 2 * (m % 4));
+        return patch(q, (x - c[i]) / dx, dx, (y - c[j]) / dy, dy);
+    }
+    // the Hermite patch at (t, u): q the records of nodes (i, j), (i + 1, j), then of j + 1
+    static __device__ __forceinline__ double patch(const double2 *q, double t, double dx, double u, double dy)
+    {
+        const double t1 = 1 - t, u1 = 1 - u;
+        const double ht[4] = {(1 + 2 * t) * t1 * t1, t * t * (3 - 2 * t), dx * t * t1 * t1, -dx * t * t * t1};
+        const double hu[4] = {(1 + 2 * u) * u1 * u1, u * u * (3 - 2 * u), dy * u * u1 * u1, -dy * u * u * u1};
         double r = 0.0;
 #pragma unroll
         for (int p = 0; p < 2; ++p)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const double *g = a.ren_rec + 4 * ((size_t)(j + q) * n + i + p);
-                const double2 vx = *reinterpret_cast<const double2 *>(g), yxy = *reinterpret_cast<const double2 *>(g + 2);
-                r += vx.x * ht[p] * hu[q] + vx.y * dx * ht[2 + p] * hu[q] + yxy.x * dy * ht[p] * hu[2 + q] +
-                     yxy.y * dx * dy * ht[2 + p] * hu[2 + q];
+            for (int m = 0; m < 2; ++m) {
+                const double2 vx = q[4 * m + 2 * p], yxy = q[4 * m + 2 * p + 1];
+                r += hu[m] * (vx.x * ht[p] + vx.y * ht[2 + p]) + hu[2 + m] * (yxy.x * ht[p] + yxy.y * ht[2 + p]);
             }
         return r;
     }
@@ -294,87 +313,169 @@ __device__ pt make_pt(const intg_args &a, double zm, double mu, double sep)
     return p;
 }
 
-// The values along line of sight 1 that the double-integrated terms read at one x1:
-// D1, a, conformal H and f at z(chi1 x1) (the last two with g5 only)
-enum { X1_D1, X1_A, X1_CH, X1_F, X1_N };
+// The double integral's constants of one (z, mu, r), and what it reads at one x1: lambda1,
+// the weight times the sinh scale, the scale, the u interval's start and panel length,
+// D1 / a, G1 chi1 H (f - 1), G1 chi1 H (H - 1) and (1 - x1) / x1
+struct dco {
+    double c, cc1, chi2, q2, a1, a2, g2chi2, k9;
+    bool T, P, g4, g5, oc;
+};
+enum { X1_L, X1_W, X1_SC, X1_U, X1_DU, X1_DA, X1_E, X1_H, X1_IW, X1_N };
 
-__device__ void x1_values(const intg_args &a, double l1, double *v)
+// v in scalar registers (every lane holds the same)
+__device__ __forceinline__ double uniform(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// v again, which the compiler is not to take for the same in the next pass of a loop:
+// what is made of it stays in the loop instead of in registers across it
+template <typename V> __device__ __forceinline__ V again(V v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+__device__ dco double_consts(const intg_args &a, const pt &p)
+{
+    const unsigned f = a.flags;
+    dco k;
+    k.c = uniform(p.c);
+    k.cc1 = uniform(p.c * p.c - 1);
+    k.chi2 = uniform(p.chi2);
+    k.a1 = uniform(2 - 5 * p.s1);
+    k.a2 = uniform(2 - 5 * p.s2);
+    k.q2 = uniform((2 - 5 * p.s1) * (2 - 5 * p.s2));
+    k.g2chi2 = uniform(p.G2c * p.chi2);
+    k.k9 = uniform(9 * a.Om * a.Om);
+    k.g4 = f & F_G4;
+    k.g5 = f & F_G5;
+    k.oc = f & F_ONLY_CROSS;
+    k.T = (f & F_LEN) && !k.oc && !(f & F_FLAT_LL);
+    k.P = (f & F_LEN) && (k.g4 || k.g5);
+    return k;
+}
+
+__device__ void x1_record(const intg_args &a, const pt &p, double x1, double w1, double *v)
 {
     const lk L(a);
+    const double l1 = p.chi1 * x1, centre = l1 * p.c;
+    const double sc = fmax(l1 * p.sint, 1e-9 * p.chi2);
+    const double lo = asinh((0.0 - centre) / sc), hi = asinh((p.chi2 - centre) / sc);
+    v[X1_L] = l1;
+    v[X1_W] = w1 * sc;
+    v[X1_SC] = sc;
+    v[X1_U] = lo;
+    v[X1_DU] = (hi - lo) / a.pu;
     const double z1 = L.z_of(l1);
     const int j1 = L.bg_interval(z1);
-    v[X1_D1] = L.bgcj(C_D1, j1, z1);
-    v[X1_A] = L.bgcj(C_A, j1, z1);
-    v[X1_CH] = v[X1_F] = 0.0;
+    v[X1_DA] = L.bgcj(C_D1, j1, z1) / L.bgcj(C_A, j1, z1);
+    v[X1_E] = v[X1_H] = 0.0;
     if (a.flags & F_G5) {
-        v[X1_CH] = L.bgcj(C_CH, j1, z1);
-        v[X1_F] = L.bgcj(C_F, j1, z1);
+        const double cH = L.bgcj(C_CH, j1, z1);
+        v[X1_E] = p.G1c * p.chi1 * cH * (L.bgcj(C_F, j1, z1) - 1);
+        v[X1_H] = p.G1c * p.chi1 * cH * (cH - 1);
     }
+    v[X1_IW] = (1 - x1) / x1;
 }
 
-// functions_double_integrated (functions.c:3460-4017) at (x1, x2), times (H0 h)^4; v1
-// holds x1_values at chi1 x1
-__device__ __forceinline__ double double_point(const intg_args &a, const pt &p, double x1, double x2,
-                                               const double *v1)
+// functions_double_integrated (functions.c:3460-4017) at (lambda1, lambda2) without the
+// factor (H0 h)^4: v1 the x1 record, D2, a2 (and f2, cH2 with g5) at z(lambda2), ren the
+// renormalised I_0^4 (g4, g5) and t the tables at r in the order of WSLOT (the first half
+// where k.T, the second where k.T or k.P).  One reciprocal of r^2 serves all terms.
+__device__ __forceinline__ double double_sum(const intg_args &a, const dco &k, const double *v1, double l2, double r2,
+                                             double D2, double a2, double f2, double cH2, double ren, const double *t)
 {
-    const lk L(a);
-    const unsigned f = a.flags;
-    const double c = p.c, Om2 = a.Om * a.Om;
-    const double l1 = p.chi1 * x1, l2 = p.chi2 * x2;
-    const double r2 = fmax(l1 * l1 + l2 * l2 - 2 * l1 * l2 * c, 0.0);
-    const double r = sqrt(r2);
-    const double z2 = L.z_of(l2);
-    int j2;
-    const double D1 = v1[X1_D1], D2 = L.bgc(C_D1, z2, &j2);
-    const double DD = D1 * D2 / v1[X1_A] / L.bgcj(C_A, j2, z2);
-    const double LL = l1 * l2;
-    const double q2 = (2 - 5 * p.s1) * (2 - 5 * p.s2);
-    const bool lens = f & F_LEN, g4 = f & F_G4, g5 = f & F_G5, oc = f & F_ONLY_CROSS;
-    double xr = 0.0;
-    const int jr = L.tab_interval(r, &xr);
+    const double c = again(k.c), cc1 = again(k.cc1), q2 = again(k.q2), l1 = v1[X1_L], iw1 = v1[X1_IW];
+    const double LL = l1 * l2, m2 = k.chi2 - l2;
     double res = 0.0;
-    double ren = 0.0;
-    if (g4 || g5) ren = L.ren(r2, l1, l2, r2 <= 1e-12, l1);
-    if (lens && !oc && !(f & F_FLAT_LL)) {
+    if (k.T) {
         double T;
         if (r2 > 1e-20) {
-            const double cc1 = c * c - 1;
-            T = 2 * cc1 * LL * L.tabj(S00, jr, xr, r) / 5 + 4 * c * L.tabj(S20, jr, xr, r) / 3 +
-                4 * c * (r2 + 6 * c * LL) * L.tabj(S11, jr, xr, r) / 15 +
-                2 * cc1 * LL * (2 * r2 + 3 * c * LL) * L.tabj(S02, jr, xr, r) / 7 / r2 +
-                2 * c * (2 * r2 * r2 + 12 * c * r2 * LL + 15 * cc1 * LL * LL) * L.tabj(S13, jr, xr, r) / 15 / r2 +
-                cc1 * LL * (6 * r2 * r2 + 30 * c * r2 * LL + 35 * cc1 * LL * LL) * L.tabj(S04, jr, xr, r) / 35 / r2 / r2;
+            const double s = LL / r2;
+            T = (2.0 / 5) * cc1 * LL * t[0] + (4.0 / 3) * c * t[1] + (4.0 / 15) * c * (r2 + 6 * c * LL) * t[2] +
+                (2.0 / 7) * cc1 * LL * (2 + 3 * c * s) * t[3] +
+                (2.0 / 15) * c * (2 * r2 + LL * (12 * c + 15 * cc1 * s)) * t[4] +
+                (1.0 / 35) * cc1 * LL * (6 + s * (30 * c + 35 * cc1 * s)) * t[5];
         } else {
-            T = 4 + 24 * LL * L.tab(S11, 0.0) / 15;
+            T = 4 + 24 * LL * lk(a).tab(S11, 0.0) / 15;
         }
-        res += 9 * Om2 * q2 / 4 * p.chi1 * p.chi2 * DD * (1 - x1) * (1 - x2) * T;
+        // chi1 chi2 (1 - x1) (1 - x2) = lambda1 (1 - x1) / x1 (chi2 - lambda2)
+        res += q2 / 4 * iw1 * l1 * m2 * T;
     }
-    double cH1 = 0, cH2 = 0, f1 = 0, f2 = 0;
-    if (g5) {
-        cH1 = v1[X1_CH];
-        cH2 = L.bgcj(C_CH, j2, z2);
-        f1 = v1[X1_F];
-        f2 = L.bgcj(C_F, j2, z2);
+    const double e1 = v1[X1_E], h1 = v1[X1_H];
+    double e2 = 0.0, h2 = 0.0;
+    if (k.g5) {
+        e2 = k.g2chi2 * cH2 * (f2 - 1);
+        h2 = k.g2chi2 * cH2 * (cH2 - 1);
     }
-    if (g4 && !oc) res += 9 * Om2 * q2 * DD * ren;
-    if (g5 && !oc) res += 9 * Om2 * p.G1c * p.G2c * p.chi1 * p.chi2 * DD * cH1 * cH2 * (f1 - 1) * (f2 - 1) * ren;
-    if ((g4 || g5) && lens) {
-        const double P = r2 != 0.0 ? 2 * LL * c * L.tabj(S31, jr, xr, r) - LL * LL * (1 - c * c) * L.tabj(S22, jr, xr, r)
-                                   : 2 * LL * L.tab(S31, 0.0);
-        const double w2 = (1 - x2) / x2, w1 = (1 - x1) / x1;
-        if (g4) res += 9 * Om2 / 2 * q2 * DD * (w2 + w1) * P;
+    if (k.g4 && !k.oc) res += q2 * ren;
+    if (k.g5 && !k.oc) res += e1 * e2 * ren;
+    if (k.g4 && k.g5) res += ren * (k.a1 * e2 + k.a2 * e1);
+    if (k.P) {
+        const double P = r2 != 0.0 ? 2 * LL * c * t[6] + LL * LL * cc1 * t[7] : 2 * LL * lk(a).tab(S31, 0.0);
+        const double w2 = m2 / l2;
+        if (k.g4) res += 0.5 * q2 * (w2 + iw1) * P;
         // functions.c:3927-3940: conformal_Hz (conformal_Hz - 1) as written there
-        if (g5)
-            res += 9 * Om2 / 2 * DD * P *
-                   ((2 - 5 * p.s2) * p.G1c * p.chi1 * cH1 * (cH1 - 1) * w2 +
-                    (2 - 5 * p.s1) * p.G2c * p.chi2 * cH2 * (cH2 - 1) * w1);
+        if (k.g5) res += 0.5 * P * (k.a2 * h1 * w2 + k.a1 * h2 * iw1);
     }
-    if (g4 && g5)
-        res += 9 * Om2 * DD * ren *
-               (p.G2c * (2 - 5 * p.s1) * p.chi2 * cH2 * (f2 - 1) + p.G1c * (2 - 5 * p.s2) * p.chi1 * cH1 * (f1 - 1));
-    const double h2 = a.H0h * a.H0h;
-    return res * h2 * h2;
+    return k.k9 * (v1[X1_DA] * D2 / a2) * res;
 }
+
+// Fetches by the whole wavefront.  A lookup by lanes of their own costs the L1 cache an
+// access per lane and load; here eight lanes take one lane's 128-byte record (four
+// a 64-byte one), 16 bytes each, straight into the wavefront's LDS buffer: an instruction
+// moves 1 KB of full lines, 16 cycles of the cache where 64 gathers take 64 for 16 bytes
+// a lane (measured: 8 KB of records in 229 cycles of a CU, 535 by gathers).  Instruction T
+// takes the records of the lanes that are T modulo 8 (4); the 16-byte pieces of a record
+// are permuted by T, so that the lanes' reads of one piece spread over the banks.  Every
+// lane of the wavefront must take part.
+typedef __attribute__((address_space(1))) const void *global_ptr;
+typedef __attribute__((address_space(3))) void *lds_ptr;
+
+__device__ __forceinline__ void to_lds(const char *src, char *buf)
+{
+    __builtin_amdgcn_global_load_lds((global_ptr)src, (lds_ptr)buf, 16, 0, 0);
+}
+// lanes 0-7 of each row of 16 get lane T's v, lanes 8-15 lane T + 8's
+template <int T> __device__ __forceinline__ unsigned of_eight(unsigned v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, 0x150 + T, 0xf, 0x3, false);
+    return (unsigned)__builtin_amdgcn_update_dpp(lo, (int)v, 0x158 + T, 0xf, 0xc, false);
+}
+// each quad of lanes gets its lane T's v
+template <int T> __device__ __forceinline__ unsigned of_four(unsigned v)
+{
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, T * 0x55, 0xf, 0xf, false);
+}
+// piece: the lane's own 16-byte piece of a record, (lane & 7) * 16 or (lane & 3) * 16; off:
+// the byte offset of its record
+template <int T = 0> __device__ __forceinline__ void fetch128(const char *base, unsigned off, char *buf, unsigned piece)
+{
+    if constexpr (T < 8) {
+        if (T == 0) piece = again(piece);
+        to_lds(base + (size_t)((piece ^ (T << 4)) + of_eight<T>(off)), buf + T * 1024);
+        fetch128<T + 1>(base, off, buf, piece);
+    }
+}
+template <int T = 0> __device__ __forceinline__ void fetch64(const char *base, unsigned off, char *buf, unsigned piece)
+{
+    if constexpr (T < 4) {
+        if (T == 0) piece = again(piece);
+        to_lds(base + (size_t)((piece ^ (T << 4)) + of_four<T>(off)), buf + T * 1024);
+        fetch64<T + 1>(base, off, buf, piece);
+    }
+}
+// the lane's piece q of its record; at: its place in the buffer of the wavefront
+__device__ __forceinline__ double2 piece_at(const char *smem, unsigned at, int q)
+{
+    return *reinterpret_cast<const double2 *>(smem + (at ^ (unsigned)(q << 4)));
+}
+// the buffer is filled; its reads are done and it may be filled again
+__device__ __forceinline__ void fetched() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void taken() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // The numerators of the single-integrated lensing terms that lose digits near the
 // line of closest approach (functions.c:2183-2187, 2296-2303, 2638-2644; chi the local
@@ -590,8 +691,8 @@ __device__ int single_pieces(const pt &p, piece *pc)
 struct coef_list {
     int ncurve;
     const double *x[16], *y[16];
-    int n[16];
-    double *val[16], *pair[16];
+    int n[16], stride[16], pstride[16];
+    double *val[16], *pair[16];   // pair null: another curve of the grid writes it
 };
 
 __global__ void __launch_bounds__(256) k_intg_coef(coef_list L)
@@ -609,112 +710,367 @@ __global__ void __launch_bounds__(256) k_intg_coef(coef_list L)
         v[3] = cf.d;
         x1 = x[j + 1];
     }
-    double *r = L.val[t] + (size_t)VAL * j;
+    double *r = L.val[t] + (size_t)L.stride[t] * j;
     *reinterpret_cast<double2 *>(r) = double2{v[0], v[1]};
     *reinterpret_cast<double2 *>(r + 2) = double2{v[2], v[3]};
-    *reinterpret_cast<double2 *>(L.pair[t] + (size_t)PAIR * j) = double2{x[j], x1};
+    if (L.pair[t]) *reinterpret_cast<double2 *>(L.pair[t] + (size_t)L.pstride[t] * j) = double2{x[j], x1};
 }
 
-// one workgroup per (z, mu, r): PART 0 sums the single-integrated terms into out[..][0],
-// PART 1 the double-integrated ones into out[..][1]; two kernels, so that each gets the
-// registers of its own part (together they held 252 VGPRs, two wavefronts per SIMD).
-// The arguments live in device memory (a pointer, not a by-value struct, whose address
-// the lookups would otherwise take in private memory).
-template <int PART>
-__device__ __forceinline__ void integrated_body(const intg_args *__restrict__ pa)
+// workgroup sum: wavefront shuffles, then one slot per wavefront in LDS
+__device__ __forceinline__ void put_sum(double acc, double *out)
 {
-    const intg_args &a = *pa;
-    const int idx = blockIdx.x;   // (z, mu, r), r fastest
-    const int ir = idx % a.nsep;
-    const int im = (idx / a.nsep) % a.nmu;
-    const int iz = idx / (a.nsep * a.nmu);
-    const pt p = make_pt(a, a.zmean[iz], a.mu[im], a.sep[ir]);
-    const unsigned f = a.flags;
-    double acc_s = 0.0, acc_d = 0.0;
-    const bool want_single =
-        ((f & F_LEN) && (f & (F_DEN | F_RSD | F_D1 | F_D2 | F_G1 | F_G2 | F_G3))) ||
-        ((f & (F_G4 | F_G5)) && (f & (F_DEN | F_RSD | F_D1 | F_D2 | F_G1 | F_G2 | F_G3)));
-    if (PART == 0 && want_single) {
-        // the pieces in LDS (a private array indexed by node would live in scratch)
-        __shared__ piece pc[4];
-        __shared__ int npc;
-        __shared__ pt sp;
-        if (threadIdx.x == 0) {
-            sp = p;
-            piece t[4];
-            npc = single_pieces(p, t);
-            for (int i = 0; i < 4; ++i) pc[i] = t[i];
-        }
-        __syncthreads();
-        const int np = npc;
-        const int per = a.ps * a.ns;
-        for (int q = threadIdx.x; q < np * per; q += blockDim.x) {
-            const piece &P = pc[q / per];
-            const double sgn = P.a >= P.cc ? 1.0 : -1.0;
-            const double ua = asinh(sgn * (P.a - P.cc) / P.s), ub = asinh(sgn * (P.b - P.cc) / P.s);
-            double w;
-            const double u = composite(fmin(ua, ub), fmax(ua, ub), a.ps, a.ns, a.gsx, a.gsw, q % per, &w);
-            const double x = P.cc + sgn * P.s * sinh(u);
-            acc_s += w * P.s * cosh(u) * single_point(a, sp, x);
-        }
-    }
-    if (PART == 1 && (f & (F_LEN | F_G4 | F_G5))) {
-        const double xb = p.chi1 * p.c > p.chi2 ? p.chi2 / (p.chi1 * p.c) : 1.0;
-        const int pA = a.p1, pB = xb < 1.0 ? (a.p1 / 2 > 1 ? a.p1 / 2 : 1) : 0;
-        const int n1 = (pA + pB) * a.n1, nuu = a.pu * a.nu;
-        // per x1 node (CE_INTG_MAX_X1 at most, checked by the host; the launch sizes the
-        // dynamic LDS for the rule's count): the node, its weight, the sinh scale, the u
-        // interval and x1_values, once per workgroup
-        extern __shared__ double sxd[];
-        double(*sx)[5 + X1_N] = reinterpret_cast<double(*)[5 + X1_N]>(sxd);
-        for (int i1 = threadIdx.x; i1 < n1; i1 += blockDim.x) {
-            double w1;
-            const double x1 = i1 < pA * a.n1 ? composite(0.0, xb, pA, a.n1, a.g1x, a.g1w, i1, &w1)
-                                             : composite(xb, 1.0, pB, a.n1, a.g1x, a.g1w, i1 - pA * a.n1, &w1);
-            const double l1 = p.chi1 * x1, centre = l1 * p.c;
-            const double sc = fmax(l1 * p.sint, 1e-9 * p.chi2);
-            sx[i1][0] = x1;
-            sx[i1][1] = w1;
-            sx[i1][2] = sc;
-            sx[i1][3] = asinh((0.0 - centre) / sc);
-            sx[i1][4] = asinh((p.chi2 - centre) / sc);
-            x1_values(a, l1, &sx[i1][5]);
-        }
-        __syncthreads();
-        for (int q = threadIdx.x; q < n1 * nuu; q += blockDim.x) {
-            const int i1 = q / nuu, iu = q - i1 * nuu;
-            const double x1 = sx[i1][0], w1 = sx[i1][1], sc = sx[i1][2];
-            double wu;
-            const double u = composite(sx[i1][3], sx[i1][4], a.pu, a.nu, a.gux, a.guw, iu, &wu);
-            // sinh and cosh from one exponential (lambda2's absolute error stays ~eps sc)
-            const double eu = exp(u), ei = 1.0 / eu;
-            const double lam2 = p.chi1 * x1 * p.c + sc * (0.5 * (eu - ei));
-            acc_d += w1 * wu * sc * (0.5 * (eu + ei)) / p.chi2 * double_point(a, p, x1, lam2 / p.chi2, &sx[i1][5]);
-        }
-    }
-    // workgroup sum: wavefront shuffles, then one slot per wavefront in LDS
-    double acc = PART == 0 ? acc_s : acc_d;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
-    __shared__ double red[4];
+    __shared__ double red[16];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) red[wv] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
         double ss = 0.0;
         for (int k = 0; k < (int)(blockDim.x >> 6); ++k) ss += red[k];
-        a.out[2 * (int64_t)idx + PART] = ss;
+        *out = ss;
     }
 }
 
-__global__ void __launch_bounds__(256) k_integrated_single(const intg_args *__restrict__ pa)
+// the points' end-point values, a thread each: a chain of some twenty searches, which a
+// workgroup of the integrals would otherwise wait for before its first node
+__global__ void __launch_bounds__(64) k_intg_points(const intg_args *__restrict__ pa, int64_t first, int count,
+                                                    pt *__restrict__ pts)
 {
-    integrated_body<0>(pa);
+    const intg_args &a = *pa;
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= count) return;
+    const int64_t idx = first + i;   // (z, mu, r), r fastest
+    pts[i] = make_pt(a, a.zmean[idx / ((int64_t)a.nsep * a.nmu)], a.mu[(idx / a.nsep) % a.nmu], a.sep[idx % a.nsep]);
 }
 
-__global__ void __launch_bounds__(256) k_integrated_double(const intg_args *__restrict__ pa)
+// one workgroup per (z, mu, r): the single-integrated terms into out[..][0].  The
+// arguments live in device memory (a pointer, not a by-value struct, whose address
+// the lookups would otherwise take in private memory).
+__global__ void __launch_bounds__(256) k_integrated_single(const intg_args *__restrict__ pa, const pt *__restrict__ pts,
+                                                           int64_t first)
 {
-    integrated_body<1>(pa);
+    const intg_args &a = *pa;
+    const unsigned f = a.flags;
+    double acc = 0.0;
+    if ((f & (F_LEN | F_G4 | F_G5)) && (f & (F_DEN | F_RSD | F_D1 | F_D2 | F_G1 | F_G2 | F_G3))) {
+        // the pieces in LDS (a private array indexed by node would live in scratch), with
+        // the ends of their u intervals
+        __shared__ piece pc[4];
+        __shared__ double ends[4][2];
+        __shared__ int npc;
+        const pt &p = pts[blockIdx.x];
+        if (threadIdx.x == 0) {
+            piece t[4];
+            npc = single_pieces(p, t);
+            for (int i = 0; i < 4; ++i) pc[i] = t[i];
+        }
+        __syncthreads();
+        const int np = npc;
+        if ((int)threadIdx.x < 2 * np) {
+            const int i = threadIdx.x >> 1;
+            const piece &P = pc[i];
+            const double sgn = P.a >= P.cc ? 1.0 : -1.0;
+            // the lower end of u: that of b where the piece is mirrored
+            const double e = ((threadIdx.x & 1) != 0) == (sgn > 0.0) ? P.b : P.a;
+            ends[i][threadIdx.x & 1] = asinh(sgn * (e - P.cc) / P.s);
+        }
+        __syncthreads();
+        const int per = a.ps * a.ns;
+        for (int q = threadIdx.x; q < np * per; q += blockDim.x) {
+            const int i = q / per;
+            const piece &P = pc[i];
+            const double sgn = P.a >= P.cc ? 1.0 : -1.0;
+            double w;
+            const double u = composite(ends[i][0], ends[i][1], a.ps, a.ns, a.gsx, a.gsw, q - i * per, &w);
+            // sinh and cosh from one exponential (x's absolute error stays ~eps s)
+            const double eu = exp(u), ei = 1.0 / eu;
+            const double x = P.cc + sgn * P.s * (0.5 * (eu - ei));
+            acc += w * P.s * (0.5 * (eu + ei)) * single_point(a, p, x);
+        }
+    }
+    put_sum(acc, a.out + 2 * (first + blockIdx.x));
+}
+
+// The LDS of the double integral: the wavefronts' buffers and the lookup tables of the
+// fetching variant (n40, nren, f0: 0 where they are not read), the x1 records.
+constexpr int DWAVES = 12;   // wavefronts a workgroup of the fetching variant, at most
+constexpr int N40 = 512, NREN = 512, BUCKETS = 512;
+constexpr int DLDS_MAX = 160 * 1024 - 512;   // beside the static LDS of the kernel
+struct dlds {
+    int s40v, sx, s40x, chi, rchi, head, bucket, guess, bytes;   // byte offsets
+    __host__ __device__ dlds(int waves, int n1, int n40, int nren, int f0, int nguess)
+    {
+        s40v = 8192 * waves;
+        sx = s40v + 32 * n40;
+        s40x = sx + 8 * X1_N * n1;
+        chi = s40x + 8 * n40;
+        rchi = chi + 8 * nren;
+        head = rchi + 8 * nren;
+        bucket = head + 8 * (f0 + 1);
+        guess = bucket + (n40 ? 2 * (BUCKETS + 2) : 0);
+        bytes = guess + 2 * nguess;
+    }
+};
+
+// One workgroup per (z, mu, r): the double-integrated terms into out[..][1], 192 lambda2
+// nodes for each of 128 to 192 x1 nodes by the default rule; a lane takes one node.
+// FETCH: the tables that are read share their nodes, and I_0^4 and the renormalisation grid
+// are small enough for LDS (the launcher's rule).  Before, 56 gathers of 64 lanes a
+// node, through generic pointers, bounded it (10.3 ms for 4096 points with every term).
+// Now the records come by the line (36 fetches of 1 KB a wavefront's 64 nodes, 28 cycles of
+// the CU's cache path each), I_0^4 with a bucket index, the chi guesses and the
+// renormalisation grid's abscissae stand in LDS, and 2 gathers are left: 5.5 ms, of it about
+// 90% by those fetches and 53% by the FP64 pipes.  DWAVES: 12 wavefronts a workgroup,
+// 168 registers each, whose 8 KB buffers and the tables they share fill the LDS; 16 spill
+// (8.4 ms), 8 hide less (6.1 ms).  FETCH false: tables on nodes of their own, or larger ones,
+// looked up lane by lane.
+template <bool FETCH>
+__global__ void __launch_bounds__(FETCH ? 64 * DWAVES : 256) k_integrated_double(const intg_args *__restrict__ pa, const pt *__restrict__ pts, int64_t first)
+{
+    const intg_args &a = *pa;
+    const lk L(a);
+    const pt &sp = pts[blockIdx.x];
+    extern __shared__ __align__(16) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const bool g45 = a.flags & (F_G4 | F_G5);
+    const int pB = a.p1 / 2 > 1 ? a.p1 / 2 : 1;
+    const int n40 = FETCH && g45 ? a.tab_len[S40] : 0, nren = FETCH && g45 ? a.nren : 0;
+    const int ref = a.tab_ref, f0 = FETCH && ref >= 0 && a.tab_f0[ref] > 0 ? a.tab_f0[ref] : 0;
+    const dlds o(FETCH ? waves : 0, (a.p1 + pB) * a.n1, n40, nren, f0, FETCH ? a.nguess + 1 : 0);
+    char *buf = smem + 8192 * wave;
+    const unsigned p128 = (lane & 7) << 4, p64 = (lane & 3) << 4;
+    const unsigned l128 = 8192 * wave + ((lane & 7) << 10) + ((lane >> 3) << 7) + p128;
+    const unsigned l64 = 8192 * wave + ((lane & 3) << 10) + ((lane >> 2) << 6) + p64;
+    double *sx = reinterpret_cast<double *>(smem + o.sx);
+    double *x40 = reinterpret_cast<double *>(smem + o.s40x), *v40 = reinterpret_cast<double *>(smem + o.s40v);
+    double *chi = reinterpret_cast<double *>(smem + o.chi), *rchi = reinterpret_cast<double *>(smem + o.rchi);
+    double *head = reinterpret_cast<double *>(smem + o.head);
+    unsigned short *bucket = reinterpret_cast<unsigned short *>(smem + o.bucket);
+    unsigned short *guess = reinterpret_cast<unsigned short *>(smem + o.guess);
+    double lx40 = 0.0, ls40 = 0.0;
+    if (FETCH) {
+        const double *x = a.tab_x + a.tab_off[S40];
+        for (int i = threadIdx.x; i < n40; i += blockDim.x) {
+            x40[i] = x[i];
+            const double2 *v = reinterpret_cast<const double2 *>(L.tabv(S40, i));
+            reinterpret_cast<double2 *>(v40 + 4 * i)[0] = v[0];
+            reinterpret_cast<double2 *>(v40 + 4 * i)[1] = v[1];
+        }
+        for (int i = threadIdx.x; i < nren; i += blockDim.x) {
+            chi[i] = a.ren_chi[i];
+            rchi[i] = i < nren - 1 ? 1.0 / (a.ren_chi[i + 1] - a.ren_chi[i]) : 0.0;
+        }
+        for (int i = threadIdx.x; i <= a.nguess; i += blockDim.x) guess[i] = (unsigned short)max((int)a.chi_guess[i], 0);
+        if (f0)
+            for (int i = threadIdx.x; i <= f0; i += blockDim.x) head[i] = a.tab_x[a.tab_off[ref] + i];
+        if (n40) {
+            // uniform in log r from the second node (the first may be 0) to the last
+            lx40 = uniform(log(x[1]));
+            ls40 = uniform(BUCKETS / (log(x[n40 - 1]) - lx40));
+            for (int i = threadIdx.x; i <= BUCKETS; i += blockDim.x)
+                bucket[i] = (unsigned short)ce::interval_bisect(x, 0, n40 - 1, exp(lx40 + i / ls40));
+        }
+    }
+    __syncthreads();
+    double acc = 0.0;
+    if (a.flags & (F_LEN | F_G4 | F_G5)) {
+        const double xb = sp.chi1 * sp.c > sp.chi2 ? sp.chi2 / (sp.chi1 * sp.c) : 1.0;
+        const int pA = a.p1, n1 = (xb < 1.0 ? pA + pB : pA) * a.n1, nu = a.nu, nuu = a.pu * nu;
+        for (int i = threadIdx.x; i < n1; i += blockDim.x) {
+            double w1;
+            const double x1 = i < pA * a.n1 ? composite(0.0, xb, pA, a.n1, a.g1x, a.g1w, i, &w1)
+                                            : composite(xb, 1.0, pB, a.n1, a.g1x, a.g1w, i - pA * a.n1, &w1);
+            x1_record(a, sp, x1, w1, sx + X1_N * i);
+        }
+        __syncthreads();
+        const dco k = double_consts(a, sp);
+        const float inu = 1.0f / (float)nu;
+        const int di = (int)blockDim.x / nuu, dr = (int)blockDim.x - di * nuu;
+        int i1 = (int)threadIdx.x / nuu, iu = (int)threadIdx.x - i1 * nuu;
+        // the lookups' uniform values
+        const bool tabs = k.T || k.P;
+        const int nt = ref >= 0 ? a.tab_len[ref] : 0, nbg = a.nbg, nguess = a.nguess;
+        const double *tx = ref >= 0 ? a.tab_x + a.tab_off[ref] : a.tab_x;
+        const double *tp = ref >= 0 ? a.tab_pair + PAIR * (size_t)a.tab_off[ref] : a.tab_pair;
+        const double *gux = a.gux, *guw = a.guw, *zp = a.bgz_pair;
+        const char *zof = reinterpret_cast<const char *>((const double *)a.zof);
+        const char *bgw = reinterpret_cast<const char *>((const double *)a.bgc_wide);
+        const char *wide = reinterpret_cast<const char *>((const double *)a.tab_wide);
+        const char *rec = reinterpret_cast<const char *>((const double *)a.ren_rec);
+        double t_lo = 0.0, t_hi = 0.0, t_lx0 = 0.0, t_lsc = 0.0;
+        if (FETCH && tabs) {
+            t_lo = tx[0];
+            t_hi = tx[nt - 1];
+            t_lx0 = a.tab_lx0[ref];
+            t_lsc = a.tab_lsc[ref];
+        }
+        const double zx0 = a.bg_z[0], zx1 = a.bg_z[nbg - 1], zsc = uniform((nbg - 1) / (zx1 - zx0));
+        const double cx0 = a.bg_chi[0], cx1 = a.bg_chi[nbg - 1], csc = uniform(nguess / cx1);
+        const double n_lo = nren ? uniform(chi[0]) : 0.0, n_hi = nren ? uniform(chi[nren - 1]) : 0.0;
+        const double nsc = nren ? uniform((nren - 1) / (n_hi - n_lo)) : 0.0;
+        const double x40_lo = n40 ? uniform(x40[0]) : 0.0, x40_hi = n40 ? uniform(x40[n40 - 1]) : 0.0;
+        // whole wavefronts to the end: the lanes past the last node repeat one of its row
+        for (int q = wave * 64; q < n1 * nuu; q += (int)blockDim.x) {
+            const bool live = i1 < n1;
+            const double *v1 = sx + X1_N * (live ? i1 : n1 - 1);
+            const int kp = (int)(((float)iu + 0.5f) * inu), ju = iu - kp * nu;
+            const double du = v1[X1_DU];
+            // sinh and cosh from one exponential (lambda2's absolute error stays ~eps sc)
+            const double eu = exp(v1[X1_U] + du * (kp + 0.5 * (1.0 + gux[ju]))), ei = 1.0 / eu;
+            const double wt = v1[X1_W] * (0.25 * du * guw[ju]) * (eu + ei);
+            const double l1 = v1[X1_L], l2 = l1 * k.c + v1[X1_SC] * (0.5 * (eu - ei));
+            const double r2 = fmax(l1 * l1 + l2 * l2 - 2 * l1 * l2 * k.c, 0.0), r = sqrt(r2);
+            double D2, a2, f2 = 0.0, cH2 = 0.0, ren = 0.0, t[8];
+            if (FETCH) {
+                // z(lambda2) on its way
+                int jc = -1;
+                if (l2 >= cx0 && l2 <= cx1)
+                    jc = lk::below_last(guess[ce::clamp_index(l2 * csc, nguess + 1)], nbg);
+                const unsigned jz = jc < 0 ? 0u : (unsigned)jc;
+                taken();
+                fetch64(zof, jz * (8u * ZOF), buf, p64);
+                // r's interval on the tables' nodes: exact in the head, else from the log
+                const double lr = log(r);
+                int jr = -1;
+                double xr = 0.0;
+                if (tabs && r >= t_lo && r <= t_hi) {
+                    if (!f0) {
+                        jr = ce::interval_bisect(tx, 0, nt - 1, r);
+                    } else if (r < head[f0]) {
+                        jr = ce::interval_bisect(head, 0, f0, r);
+                    } else {
+                        jr = lk::below_last(f0 + ce::clamp_index((lr - t_lx0) * t_lsc, nt - f0), nt);
+                    }
+                    nodes nd = pair_at(tp, jr);
+                    if (!pair_hit(nd, jr, nt, r)) {
+                        jr = ce::interval_from(tx, nt, r, jr);
+                        nd = pair_at(tp, jr);
+                    }
+                    xr = nd.x0;
+                }
+                const unsigned orec = (jr < 0 ? 0u : (unsigned)jr) * (8u * WIDE);
+                fetched();
+                unsigned at = again(l64);
+                const double2 zn = piece_at(smem, at, 0);
+                double z2 = cubic(piece_at(smem, at, 1), piece_at(smem, at, 2), l2 - zn.x);
+                if (jc < 0) z2 = __builtin_nan("");
+                else if (!pair_hit(nodes{zn.x, zn.y}, jc, nbg, l2)) z2 = L.zofj(ce::interval_from(a.bg_chi, a.nbg, l2, jc), l2);
+                // the curves at z2
+                int jb = -1;
+                double xz = 0.0;
+                if (z2 >= zx0 && z2 <= zx1) {
+                    jb = lk::below_last(ce::clamp_index((z2 - zx0) * zsc, nbg), nbg);
+                    nodes nb = pair_at(zp, jb);
+                    if (!pair_hit(nb, jb, nbg, z2)) {
+                        jb = ce::interval_from(a.bg_z, a.nbg, z2, jb);
+                        nb = pair_at(zp, jb);
+                    }
+                    xz = nb.x0;
+                }
+                const double dz = jb < 0 ? __builtin_nan("") : z2 - xz;
+                taken();
+                fetch128(bgw, (jb < 0 ? 0u : (unsigned)jb) * (8u * BGW), buf, p128);
+                // I_0^4 r^4 from LDS
+                int ix = 0, jy = 0;
+                bool patched = false;
+                if (n40) {
+                    ren = __builtin_nan("");
+                    if (r >= x40_lo && r <= x40_hi) {
+                        const int b = ce::clamp_index((lr - lx40) * ls40, BUCKETS);
+                        int lo = bucket[b], hi = min(bucket[b + 1] + 1, n40 - 1);
+                        if (!(x40[lo] <= r && (hi == n40 - 1 || r < x40[hi]))) {
+                            lo = 0;
+                            hi = n40 - 1;
+                        }
+                        lo = ce::interval_bisect(x40, lo, hi, r);
+                        ren = val_at(v40 + 4 * lo, x40[lo], r);
+                    }
+                    if (l1 >= n_lo && l1 <= n_hi && l2 >= n_lo && l2 <= n_hi) {
+                        patched = true;
+                        ix = ce::interval_from(chi, nren, l1, ce::clamp_index((l1 - n_lo) * nsc, nren));
+                        jy = ce::interval_from(chi, nren, l2, ce::clamp_index((l2 - n_lo) * nsc, nren));
+                    }
+                }
+                fetched();
+                at = again(l128);
+                D2 = cubic(piece_at(smem, at, 2 * C_D1), piece_at(smem, at, 2 * C_D1 + 1), dz);
+                a2 = cubic(piece_at(smem, at, 2 * C_A), piece_at(smem, at, 2 * C_A + 1), dz);
+                if (k.g5) {
+                    f2 = cubic(piece_at(smem, at, 2 * C_F), piece_at(smem, at, 2 * C_F + 1), dz);
+                    cH2 = cubic(piece_at(smem, at, 2 * C_CH), piece_at(smem, at, 2 * C_CH + 1), dz);
+                }
+                if (n40) {
+                    const unsigned on = (unsigned)(jy * nren + ix) * 32u, row = (unsigned)nren * 32u;
+                    taken();
+                    fetch64(rec, on, buf, p64);
+                    fetch64(rec + row, on, buf + 4096, p64);
+                    fetched();
+                    at = again(l64);
+                    double2 p[8];
+#pragma unroll
+                    for (int m = 0; m < 8; ++m) p[m] = piece_at(smem, at + 4096 * (m / 4), m % 4);
+                    const double bic = lk::patch(p, (l1 - chi[ix]) * rchi[ix], chi[ix + 1] - chi[ix],
+                                                 (l2 - chi[jy]) * rchi[jy], chi[jy + 1] - chi[jy]);
+                    ren -= patched ? bic : __builtin_nan("");
+                    if (r2 <= 1e-12) ren = ak(a.ren0_x, a.ren0_y, a.nren0, l1);
+                }
+                at = again(l128);
+                const double dr2 = jr < 0 ? __builtin_nan("") : r - xr;
+                if (k.T) {
+                    taken();
+                    fetch128(wide, orec, buf, p128);
+                    fetched();
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) t[m] = cubic(piece_at(smem, at, 2 * m), piece_at(smem, at, 2 * m + 1), dr2);
+                }
+                if (tabs) {
+                    taken();
+                    fetch128(wide + 128, orec, buf, p128);
+                    fetched();
+#pragma unroll
+                    for (int m = 0; m < 4; ++m)
+                        t[4 + m] = cubic(piece_at(smem, at, 2 * m), piece_at(smem, at, 2 * m + 1), dr2);
+                }
+            } else {
+                const double z2 = L.z_of(l2);
+                const int j2 = L.bg_interval(z2);
+                D2 = L.bgcj(C_D1, j2, z2);
+                a2 = L.bgcj(C_A, j2, z2);
+                if (k.g5) {
+                    f2 = L.bgcj(C_F, j2, z2);
+                    cH2 = L.bgcj(C_CH, j2, z2);
+                }
+                double xr = 0.0;
+                const int jr = tabs ? L.tab_interval(r, &xr) : -1;
+                if (g45) ren = L.ren(r2, l1, l2, r2 <= 1e-12, l1);
+                if (k.T) {
+                    t[0] = L.tabj(S00, jr, xr, r);
+                    t[1] = L.tabj(S20, jr, xr, r);
+                    t[2] = L.tabj(S11, jr, xr, r);
+                    t[3] = L.tabj(S02, jr, xr, r);
+                    t[4] = L.tabj(S13, jr, xr, r);
+                    t[5] = L.tabj(S04, jr, xr, r);
+                }
+                if (k.P) {
+                    t[6] = L.tabj(S31, jr, xr, r);
+                    t[7] = L.tabj(S22, jr, xr, r);
+                }
+            }
+            const double v = double_sum(a, k, v1, l2, r2, D2, a2, f2, cH2, ren, t);
+            if (live) acc += wt * v;
+            iu += dr;
+            i1 += di;
+            if (iu >= nuu) {
+                iu -= nuu;
+                ++i1;
+            }
+        }
+        const double h2 = a.H0h * a.H0h;
+        acc *= h2 * h2 / sp.chi2;
+    }
+    put_sum(acc, a.out + 2 * (first + blockIdx.x) + 1);
 }
 
 }  // namespace
@@ -755,26 +1111,34 @@ extern "C" int ce_launch_integrated(void *stream, const ce_intg_dev *in, unsigne
     a.nguess = in->nguess;
     a.chi_guess = in->chi_guess;
     a.tab_ref = in->tab_ref;
-    // the value records, then the node pairs; each the tables' in tab_y's layout, then
-    // the background curves'
-    const size_t nrec = (size_t)in->ntab_values + (size_t)NBGC * in->nbg;
-    double *tval = in->coef, *bval = tval + (size_t)VAL * in->ntab_values;
-    double *tpair = in->coef + (size_t)VAL * nrec, *bpair = tpair + (size_t)PAIR * in->ntab_values;
-    a.tab_val = tval;
-    a.bgc_val = bval;
+    // records, then node pairs (ce_intg_coef_len): the shared nodes' tables and the
+    // background curves wide, z(chi), then the other tables in tab_y's layout
+    const int nsh = in->tab_ref < 0 ? 0 : in->tab_len[in->tab_ref];
+    double *wide = in->coef, *bgw = wide + (size_t)WIDE * nsh, *zof = bgw + (size_t)BGW * in->nbg;
+    double *own = zof + (size_t)ZOF * in->nbg, *tpair = own + (size_t)VAL * in->ntab_values;
+    double *zpair = tpair + (size_t)PAIR * in->ntab_values;
+    a.tab_wide = wide;
     a.tab_pair = tpair;
-    a.bgc_pair = bpair;
+    a.bgc_wide = bgw;
+    a.bgz_pair = zpair;
+    a.zof = zof;
     coef_list cl;
     cl.ncurve = 0;
     int nmax = 0;
     for (int t = 0; t < NSLOT; ++t) {
+        const bool shared = nsh && t != S40;
+        double *val = shared ? wide + VAL * WSLOT[t] : own + (size_t)VAL * in->tab_off[t];
+        a.tab_val[t] = val;
+        a.tab_stride[t] = shared ? WIDE : VAL;
         if (in->tab_len[t] < 5) continue;
         const int q = cl.ncurve++;
         cl.x[q] = in->tab_x + in->tab_off[t];
         cl.y[q] = in->tab_y + in->tab_off[t];
         cl.n[q] = in->tab_len[t];
-        cl.val[q] = tval + (size_t)VAL * in->tab_off[t];
+        cl.val[q] = val;
+        cl.stride[q] = a.tab_stride[t];
         cl.pair[q] = tpair + (size_t)PAIR * in->tab_off[t];
+        cl.pstride[q] = PAIR;
         nmax = cl.n[q] > nmax ? cl.n[q] : nmax;
     }
     const double *bx[NBGC] = {in->bg_z, in->bg_z, in->bg_z, in->bg_z, in->bg_chi};
@@ -784,8 +1148,10 @@ extern "C" int ce_launch_integrated(void *stream, const ce_intg_dev *in, unsigne
         cl.x[q] = bx[k];
         cl.y[q] = by[k];
         cl.n[q] = in->nbg;
-        cl.val[q] = bval + (size_t)VAL * k * in->nbg;
-        cl.pair[q] = bpair + (size_t)PAIR * k * in->nbg;
+        cl.val[q] = k == C_ZOF ? zof + 2 : bgw + VAL * k;
+        cl.stride[q] = k == C_ZOF ? ZOF : BGW;
+        cl.pair[q] = k == C_ZOF ? zof : (k == C_D1 ? zpair : nullptr);
+        cl.pstride[q] = k == C_ZOF ? ZOF : PAIR;
         nmax = in->nbg > nmax ? in->nbg : nmax;
     }
     hipLaunchKernelGGL(k_intg_coef, dim3((unsigned)((nmax + 255) / 256), (unsigned)cl.ncurve), dim3(256), 0,
@@ -825,11 +1191,37 @@ extern "C" int ce_launch_integrated(void *stream, const ce_intg_dev *in, unsigne
     hipError_t e = hipMemcpyAsync(in->args_dev, &a, sizeof(a), hipMemcpyHostToDevice, (hipStream_t)stream);
     if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);   /* `a` is on this stack */
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(k_integrated_single, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
-                       (const intg_args *)in->args_dev);
-    const int p1b = a.p1 / 2 > 1 ? a.p1 / 2 : 1;
-    const size_t x1_lds = (size_t)(a.p1 + p1b) * a.n1 * (5 + X1_N) * sizeof(double);
-    hipLaunchKernelGGL(k_integrated_double, dim3((unsigned)blocks), dim3(256), x1_lds, (hipStream_t)stream,
-                       (const intg_args *)in->args_dev);
+    // the fetching variant where the tables that are read share their nodes, what it keeps in
+    // LDS is small and its 16- and 32-bit indices hold; with the most wavefronts whose
+    // buffers fit beside it
+    const bool g45 = flags & (F_G4 | F_G5);
+    const bool tabs = (flags & F_LEN) && (g45 || (!(flags & F_ONLY_CROSS) && !(flags & F_FLAT_LL)));
+    const int n1 = (a.p1 + (a.p1 / 2 > 1 ? a.p1 / 2 : 1)) * a.n1;
+    const int n40 = g45 ? a.tab_len[S40] : 0, nren = g45 ? a.nren : 0;
+    const int f0 = nsh && a.tab_f0[a.tab_ref] > 0 ? a.tab_f0[a.tab_ref] : 0;
+    const bool fetch = (!tabs || nsh) && n40 <= N40 && nren <= NREN && nsh <= (1 << 23) && a.nbg <= (1 << 16);
+    int waves = fetch ? DWAVES : 0;
+    while (waves > 4 && dlds(waves, n1, n40, nren, f0, a.nguess + 1).bytes > DLDS_MAX) --waves;
+    const size_t lds = (size_t)(fetch ? dlds(waves, n1, n40, nren, f0, a.nguess + 1) : dlds(0, n1, 0, 0, 0, 0)).bytes;
+    if (fetch) {
+        e = hipFuncSetAttribute((const void *)k_integrated_double<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    const intg_args *d_args = (const intg_args *)in->args_dev;
+    pt *pts = (pt *)in->points;
+    static_assert(sizeof(pt) <= CE_INTG_POINT * sizeof(double), "a point outgrew its record");
+    for (int64_t first = 0; first < blocks; first += CE_INTG_POINTS) {
+        const int count = (int)(blocks - first < CE_INTG_POINTS ? blocks - first : CE_INTG_POINTS);
+        hipLaunchKernelGGL(k_intg_points, dim3((unsigned)(count + 63) / 64), dim3(64), 0, (hipStream_t)stream, d_args, first,
+                           count, pts);
+        hipLaunchKernelGGL(k_integrated_single, dim3((unsigned)count), dim3(256), 0, (hipStream_t)stream, d_args,
+                           (const pt *)pts, first);
+        if (fetch)
+            hipLaunchKernelGGL(k_integrated_double<true>, dim3((unsigned)count), dim3(64 * waves), lds, (hipStream_t)stream,
+                               d_args, (const pt *)pts, first);
+        else
+            hipLaunchKernelGGL(k_integrated_double<false>, dim3((unsigned)count), dim3(256), lds, (hipStream_t)stream, d_args,
+                               (const pt *)pts, first);
+    }
     return (int)hipGetLastError();
 }
