@@ -266,8 +266,8 @@ def run_covariance(args):
     torch.cuda.synchronize()
     ms = (time.perf_counter() - t0) * 1e3 / args.steps
     entries = cov.numel()
-    # the integrals launch (k_cov_diag, k_cov_rows, k_cov_cols) timed on its stream with
-    # HIP events over 3 calls back to back; k_cov_rows is the dominant kernel
+    # the integrals launch (k_cov_diag, k_cov_many, k_cov_sum) timed on its stream with
+    # HIP events over 3 calls back to back; k_cov_many is the dominant kernel
     stream = torch.cuda.current_stream()
     ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
     reps = 3
@@ -289,9 +289,7 @@ def run_covariance(args):
     torch.cuda.synchronize()
     vjp_us = ev[0].elapsed_time(ev[1]) * 1e3 / reps
     N = 8000
-    row_flops = 7.5 * N * np.log2(N) + 8.0 * N + 2.0 * 72 * len(sep)
-    nrows_launch = 64 * 2 * plan.npair * plan.nrows
-    cov_flops = row_flops * nrows_launch
+    cov_flops = 2.0 * N * len(sep) ** 2 * 64 * 2 * plan.npair
     res = {
         "metric": "Gaussian covariance entries/sec (64 P(k), 2D FFTLog N=8000, 4 z x (3 l x 256 r)^2), 1 MI355X",
         "value": entries / (ms / 1e3), "unit": "entries/s", "n_gpus": 1, "steps": args.steps,
@@ -300,13 +298,12 @@ def run_covariance(args):
         "config": {"workload": "64 seeded P(k) (4096 samples), 2D FFTLog N=8000, l=0,2,4, 256 seps 10-200 Mpc/h, "
                                "4 z bins; step = P and P^2 integrals of 6 pairs + assembly",
                    "transform_rows_per_pair": plan.nrows, "transforms_per_step": 64 * 2 * plan.npair},
-        "roofline": {"bound": "mfma", "kernel": "k_cov_rows", "achieved": cov_flops / (rows_us * 1e-6) / 1e12,
+        "roofline": {"bound": "mfma", "kernel": "k_cov_many", "achieved": cov_flops / (rows_us * 1e-6) / 1e12,
                      "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s", "frac": cov_flops / (rows_us * 1e-6) / PEAK_FP64,
-                     "traffic": traffic_of("covariance_64spec_n8000", "k_cov_rows"), "launch_us": rows_us,
-                     "note": "per transform row 7.5 N log2 N (complex FFT_N + c2r) + 8 N (kernel products) + "
-                             "2 x 72 x R (column functionals), N = 8000, R = 256, x 64 spectra x 2 powers x 6 pairs x "
-                             "rows per pair; time = HIP events over 3 integrals calls (k_cov_diag + k_cov_rows + "
-                             "k_cov_cols, rows > 95 % in the kernel trace); FP64 peak 78.6 TFLOP/s"},
+                     "traffic": traffic_of("covariance_64spec_n8000", "k_cov_many"), "launch_us": rows_us,
+                     "note": "FP64 MFMA contraction over k of the plan's tables, 2 N R^2 flop per spectrum, power and "
+                             "pair (N = 8000, R = 256, x 64 x 2 x 6); time = HIP events over 3 integrals calls, every "
+                             "kernel of them; FP64 peak 78.6 TFLOP/s"},
         "adjoint": {"integrals_us": rows_us, "integrals_vjp_us": vjp_us,
                     "note": "coffe_cov_integrals_vjp on the same 64 spectra (d<G, integrals>/dP for every input "
                             "sample), HIP events over 3 calls"},
@@ -509,7 +506,7 @@ def run_integrated(args):
                      "note": f"{INTG_FLOP_PER_NODE:.0f} flop per integrand node (estimated from the source), "
                              "divided by the whole synchronous call (uploads, allocation, the kernel, download): "
                              "a lower bound of the kernels' own rate, whose durations the rocprof summary gives; "
-                             "FP64 VALU, with table lookups bound by the L1's gather throughput (random lines per lane)"},
+                             "FP64 VALU, with table records fetched by the line into LDS"},
         "parity": {"vs_oracle_max_rel": max(chk), "points": len(chk)},
     }
     if not args.no_cpu:
