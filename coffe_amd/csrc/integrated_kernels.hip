@@ -1204,7 +1204,8 @@ extern "C" int ce_launch_integrated(void *stream, const ce_intg_dev *in, unsigne
     while (waves > 4 && dlds(waves, n1, n40, nren, f0, a.nguess + 1).bytes > DLDS_MAX) --waves;
     const size_t lds = (size_t)(fetch ? dlds(waves, n1, n40, nren, f0, a.nguess + 1) : dlds(0, n1, 0, 0, 0, 0)).bytes;
     if (fetch) {
-        e = hipFuncSetAttribute((const void *)k_integrated_double<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        // the most of any call: threads whose calls differ in size don't lower each other's limit
+        e = hipFuncSetAttribute((const void *)k_integrated_double<true>, hipFuncAttributeMaxDynamicSharedMemorySize, DLDS_MAX);
         if (e != hipSuccess) return (int)e;
     }
     const intg_args *d_args = (const intg_args *)in->args_dev;

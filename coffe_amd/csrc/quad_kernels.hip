@@ -703,6 +703,7 @@ __global__ void __launch_bounds__(256, 4) k_divergent(div_args a, size_t list_by
 
 constexpr size_t LIST_BYTES = 4 * CE_QAG_CAP * sizeof(double);
 
+// always a kernel's own most: threads whose launches differ in size don't lower each other's limit
 template <class F>
 hipError_t lds_limit(F *fn, size_t bytes)
 {
@@ -717,8 +718,9 @@ hipError_t launch_small_r(const sr_args &all, size_t sbytes, hipStream_t s)
     // wavefronts per workgroup: one while the integrals do not fill the chip (each then makes
     // its own spline in a microsecond or two), eight beyond
     const int nw = (int64_t)all.nspec * per <= 2048 ? 1 : 8;
-    hipError_t e = lds_limit(k_small_r<list_regs, LDS>, sbytes);
-    if (e == hipSuccess) e = lds_limit(k_small_r<list_lds, LDS>, LIST_BYTES + sbytes);
+    const size_t smost = LDS ? spline_bytes(CE_SPL_MAX) : 0;
+    hipError_t e = lds_limit(k_small_r<list_regs, LDS>, smost);
+    if (e == hipSuccess) e = lds_limit(k_small_r<list_lds, LDS>, LIST_BYTES + smost);
     for (int s0 = 0; s0 < all.nspec && e == hipSuccess; s0 += 32768) {   // the grid's y range
         sr_args a = all;
         a.nspec = all.nspec - s0 < 32768 ? all.nspec - s0 : 32768;
@@ -737,8 +739,9 @@ hipError_t launch_small_r(const sr_args &all, size_t sbytes, hipStream_t s)
 template <bool LDS>
 hipError_t launch_divergent(const div_args &a, int units, size_t sbytes, hipStream_t s)
 {
-    hipError_t e = lds_limit(k_divergent<list_regs, LDS>, sbytes);
-    if (e == hipSuccess) e = lds_limit(k_divergent<list_lds, LDS>, LIST_BYTES + sbytes);
+    const size_t smost = LDS ? spline_bytes(CE_SPL_MAX) : 0;
+    hipError_t e = lds_limit(k_divergent<list_regs, LDS>, smost);
+    if (e == hipSuccess) e = lds_limit(k_divergent<list_lds, LDS>, LIST_BYTES + smost);
     if (e != hipSuccess) return e;
     // four wavefronts share a spline; two rounds of the workgroups that are resident at once
     // (128 VGPRs; 1116 us, against 1186 with one round, 1195 with eight wavefronts, 1296 at 168
