@@ -38,3 +38,37 @@ def test_outputs_belong_to_the_engines_stream():
         assert torch.allclose(g, w, rtol=1e-12, atol=0)
     for b in batches:
         b.close()
+
+
+def test_overlapping_passes_of_two_engines():
+    """three forward + adjoint passes with nothing between them, the second on another engine's batch
+    of other spectra and dropped at once, at the benchmark's size (256 ragged spectra, 512
+    separations, 130 us a pass): the third pass' outputs are what a pass alone gives.  Its
+    memory must not be that of the second pass, which may still be written: every element was at
+    risk when both came from the default stream's pool (1e-12: the sums' order is the same)."""
+    import torch
+    from coffe_amd.engine import Batch, Engine
+    from tests.synth import batch_spectra
+    sep = np.linspace(5.0, 300.0, 512) / 0.67
+    A = torch.tensor(flat_weights([0, 2, 4], 1.5, 0.87, 0.6, 512), device="cuda")
+    sets = []
+    for seed in (0, 1):
+        specs = batch_spectra(256, seed=seed)
+        n = [len(s[0]) for s in specs]
+        b = Batch(Engine(0), n, n, [s[0][0] for s in specs], [s[0][-1] for s in specs], [(0, 0), (0, 2), (0, 4)], sep, 1, 3)
+        rng = np.random.default_rng(seed)
+        sets.append((b, torch.tensor(np.concatenate([s[0] for s in specs]), device="cuda"),
+                     torch.tensor(np.concatenate([s[1] for s in specs]), device="cuda"), A,
+                     torch.tensor(rng.standard_normal((256, 1, 3, 512)), device="cuda")))
+    run = lambda s: s[0].vjp(*s[1:])  # noqa: E731
+    want = [t.clone() for t in run(sets[0])]
+    for _ in range(10):
+        torch.cuda.synchronize()
+        got = run(sets[0])
+        run(sets[1])
+        got = run(sets[0])
+        torch.cuda.synchronize()
+        for g, w in zip(got, want):
+            assert float((g - w).norm()) <= 1e-12 * float(w.norm())
+    for s in sets:
+        s[0].close()
