@@ -202,7 +202,11 @@ struct sr_unit {
 // of the intervals in LDS (LDS = true), or the samples themselves where they do not fit
 // (LDS = false: a bisection in L2 and the coefficients anew at every value).
 #define CE_SPL_BUCKETS 1024
-#define CE_SPL_MAX 3000     // samples in LDS: 40 bytes each of the CU's 160 KB
+// samples in LDS: 40 bytes each of the CU's 160 KB, which beside them hold the second kernel's list.
+// At 2999 samples, LDS against L2: 4194 divergent integrals 539 and 499 us, 40995 2588 and 2556, 2000
+// 317 and 360; small-r nodes 83 and 90 (344), 283 and 343 (13760): even there, far ahead below
+// (1293 against 2324 us for 40995 integrals at 600)
+#define CE_SPL_MAX 3000
 struct lds_spline {
     const double *x;        // [n]
     const double2 *yb, *cd; // [n]: value and coefficients of the interval from node j
@@ -715,9 +719,11 @@ template <bool LDS>
 hipError_t launch_small_r(const sr_args &all, size_t sbytes, hipStream_t s)
 {
     const int per = all.ntab * (1 + CE_MIN_SEP_LEN);
-    // wavefronts per workgroup: one while the integrals do not fill the chip (each then makes
-    // its own spline in a microsecond or two), eight beyond
-    const int nw = (int64_t)all.nspec * per <= 2048 ? 1 : 8;
+    // eight wavefronts share a spline, also where the integrals do not fill the chip: making it
+    // takes eight times as long in one wavefront, and above 2000 samples (more than half a CU's
+    // LDS) a CU then runs one wavefront.  1720 integrals: 77 us at 600 samples and 86 at 2999,
+    // against 123 and 629 with one wavefront, 80 and 126 with four; 43 integrals of 600: 69, 83, 68.
+    const int nw = 8;
     const size_t smost = LDS ? spline_bytes(CE_SPL_MAX) : 0;
     hipError_t e = lds_limit(k_small_r<list_regs, LDS>, smost);
     if (e == hipSuccess) e = lds_limit(k_small_r<list_lds, LDS>, LIST_BYTES + smost);
@@ -743,11 +749,13 @@ hipError_t launch_divergent(const div_args &a, int units, size_t sbytes, hipStre
     hipError_t e = lds_limit(k_divergent<list_regs, LDS>, smost);
     if (e == hipSuccess) e = lds_limit(k_divergent<list_lds, LDS>, LIST_BYTES + smost);
     if (e != hipSuccess) return e;
-    // four wavefronts share a spline; two rounds of the workgroups that are resident at once
-    // (128 VGPRs; 1116 us, against 1186 with one round, 1195 with eight wavefronts, 1296 at 168
-    // VGPRs and 1379 at 256)
-    const int nw = units <= 2048 ? 1 : 4;
-    const int wg = (units + nw - 1) / nw, most = nw == 1 ? wg : 2048;
+    // four wavefronts share a spline, whatever the number of integrals (2000 of them: 214 us at 600
+    // samples and 317 at 2999, against 306 and 1216 with a spline a wavefront, 218 and 557 with
+    // two); two rounds of the workgroups that are resident at once (40995 integrals, 600 samples, 128
+    // VGPRs: 1116 us, against 1186 with one round, 1195 with eight wavefronts, 1296 at 168 VGPRs
+    // and 1379 at 256)
+    const int nw = 4;
+    const int wg = (units + nw - 1) / nw, most = 2048;
     hipLaunchKernelGGL((k_divergent<list_regs, LDS>), dim3(wg < most ? wg : most), dim3(64 * nw), sbytes, s, a,
                        (size_t)0);
     hipLaunchKernelGGL((k_divergent<list_lds, LDS>), dim3(units < 512 ? units : 512), dim3(64), LIST_BYTES + sbytes, s, a,

@@ -68,3 +68,26 @@ def test_small_r_few_and_many(engine, nspec):
         for t, (n, l) in enumerate(tabs):
             _, oy = O.integral_table(n, l, *specs[s], 512, small_r=True)
             assert np.all(np.abs(got[s, t] - oy[:43]) <= 1e-10 * np.abs(oy[:43]) + 1e-12 * np.max(np.abs(oy[:43]))), (n, l)
+
+
+def test_small_r_shared_spline(engine):
+    """eight wavefronts share one LDS spline: a batch whose spectra all fit (3000 samples, one short
+    of that, a few dozen, the smallest), two tables and all eight; the longest sets the
+    launch's LDS, the others fill a part of it"""
+    import torch
+    from coffe_amd.engine import Batch
+    tabs = [(0, 0), (0, 2), (0, 4), (1, 1), (1, 3), (2, 0), (2, 2), (3, 1)]
+    for ns, use in (([3000, 30, 600, 2999, 64, 5, 1200], tabs), ([40, 3000], tabs[3:5])):
+        print("small r, shared spline", ns, flush=True)
+        # the few samples over a narrow range: the integrands stay resolved
+        specs = [spectrum(n, kmin=1e-5 if n > 50 else 0.02) for n in ns]
+        b = Batch(engine, ns, [512] * len(ns), [s[0][0] for s in specs], [s[0][-1] for s in specs], use,
+                  np.array([20.0, 50.0]), 1, 1)
+        got = b.small_r(torch.tensor(np.concatenate([s[0] for s in specs]), device="cuda"),
+                        torch.tensor(np.concatenate([s[1] for s in specs]), device="cuda")).cpu().numpy()
+        b.close()
+        for s in range(len(ns)):
+            for t, (n, l) in enumerate(use):
+                _, oy = O.integral_table(n, l, *specs[s], 512, small_r=True)
+                assert np.all(np.abs(got[s, t] - oy[:43]) <= 1e-10 * np.abs(oy[:43]) + 1e-12 * np.max(np.abs(oy[:43]))), \
+                    (ns[s], n, l)
