@@ -298,7 +298,7 @@ __device__ __forceinline__ double integrand(const sr_unit &u, const spline<LDS> 
     switch (u.kind) {
     case SR_PREFACTOR: return ipow(k, 2 + u.l - u.n) * pk;
     case SR_RENORM0: {
-        const double x = k * u.r;
+        const double x = fabs(k * u.r);
         // 1 - j0^2 ~ x^2 / 3 keeps what the rounding of j0 leaves: the series is the closer
         // one below 0.5 (at most half a unit off)
         double j0 = sph_j0(x), term = 1.0, sum = 1.0;
@@ -312,9 +312,11 @@ __device__ __forceinline__ double integrand(const sr_unit &u, const spline<LDS> 
     }
     case SR_RENORM: {
         // the product of the two Bessel factors first: symmetric in (r, r2) bit for bit
+        // (j_0 is 1 below 1e-8; from 1e-100 down, so that the product below does not underflow)
         const double xa = k * u.r, xb = k * u.r2;
-        const double ss = (xa == 0.0 ? 1.0 : sin(xa)) * (xb == 0.0 ? 1.0 : sin(xb));
-        return pk * ss / ((xa == 0.0 ? 1.0 : xa) * (xb == 0.0 ? 1.0 : xb) * (k * k));
+        const bool za = fabs(xa) < 1e-100, zb = fabs(xb) < 1e-100;
+        const double ss = (za ? 1.0 : sin(xa)) * (zb ? 1.0 : sin(xb));
+        return pk * ss / ((za ? 1.0 : xa) * (zb ? 1.0 : xb) * (k * k));
     }
     default: {
         const double x = k * u.r;

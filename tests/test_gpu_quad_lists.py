@@ -91,3 +91,30 @@ def test_small_r_shared_spline(engine):
                 _, oy = O.integral_table(n, l, *specs[s], 512, small_r=True)
                 assert np.all(np.abs(got[s, t] - oy[:43]) <= 1e-10 * np.abs(oy[:43]) + 1e-12 * np.max(np.abs(oy[:43]))), \
                     (ns[s], n, l)
+
+
+def test_divergent_arguments_at_the_edges(engine):
+    """chi so small that the product of two arguments underflows, next to 0 (j_0 is 1 at both); device
+    arrays, whose signs are not checked: j_0 is even, so the integrals of -r are those of r (the
+    factor r^4 is left out for r <= 0)"""
+    import ctypes
+    import torch
+    from coffe_amd.engine import divergent_tables
+    from coffe_amd._lib import check
+    k, pk = spectrum(400)
+    chi = np.array([0.0, 1e-300, 1e-170, 25.0, 900.0])
+    _, _, _, ren = divergent_tables(k, pk, sep=np.array([5.0]), chi=chi)
+    assert np.isfinite(ren).all()
+    for i in (1, 2):
+        assert np.array_equal(ren[i, 3:], ren[0, 3:]) and np.all(np.abs(ren[i, :3] / ren[0, 0] - 1) <= 1e-13)
+    dev = dict(device="cuda", dtype=torch.float64)
+    sep = np.array([7.0, -7.0, 60.0, -60.0])
+    kt, pt, st = torch.tensor(k, **dev), torch.tensor(pk, **dev), torch.tensor(sep, **dev)
+    i40, r0 = torch.zeros(4, **dev), torch.zeros(4, **dev)
+    status = torch.zeros(8, dtype=torch.int32, device="cuda")
+    check(engine.L.coffe_divergent_tables_device(engine.h, kt.data_ptr(), pt.data_ptr(), len(k), float(k[0]), float(k[-1]),
+                                                 st.data_ptr(), 4, None, 0, i40.data_ptr(), r0.data_ptr(), None,
+                                                 status.data_ptr(), None, ctypes.c_void_p(0)), "divergent")
+    torch.cuda.synchronize()
+    for v in (i40.cpu().numpy(), r0.cpu().numpy()):
+        assert np.all(np.abs(v[1::2] * sep[::2] ** 4 / v[::2] - 1) <= 1e-13), v
