@@ -21,9 +21,10 @@ extern "C" {
 /* intervals an adaptive QAG keeps in LDS (the reference allows 50000; the small-r
    integrands converge within a few hundred) */
 #define CE_QAG_CAP 1024
-/* input intervals per spline chunk and LDS nodes staged per chunk (chunk + 2 halos
-   of 64 + end nodes) */
+/* input intervals per spline chunk at most, nodes of the system to either side of them, and LDS
+   nodes staged per chunk (chunk + 2 halos + end nodes) */
 #define CE_CHUNK 512
+#define CE_SPLINE_HALO 64
 #define CE_CHUNK_NODES 648
 
 /* FFT radix schedule for a complex transform of length M = N/2 */
@@ -63,14 +64,15 @@ typedef struct ce_spec_dev {
     int64_t ws_off;    /* offset (doubles) of the real workspace: 2 N (S(x_i), then its cotangent) */
 } ce_spec_dev;
 
-/* one chunk of input intervals [a, b) of a spectrum (b = n_in - 1 on the last) */
+/* one chunk of input intervals [a, b) of a spectrum (b = n_in - 1 on the last); a chunk of the adjoint
+   is the resample chunks id ... last of one spectrum */
 typedef struct ce_chunk_dev {
-    int32_t spec;
+    int32_t last;
     int32_t a, b;
     int32_t grid;      /* copies of the spectrum's fields: one load gives everything */
     int64_t in_off, ws_off;
     int32_t n_in;
-    int32_t id;        /* the chunk's index in the batch: its slot of the resample ranges */
+    int32_t id;        /* the (first) resample chunk's index in the batch: its slot of the resample ranges */
 } ce_chunk_dev;
 
 /* work unit of the table kernels */

@@ -379,7 +379,7 @@ coffe_engine *coffe_engine_default(void)
 
 struct coffe_batch {
     coffe_engine *e;
-    int nspec, ntab, nsep, nz, nl, nq, nunit, ngrid, nchunk;
+    int nspec, ntab, nsep, nz, nl, nq, nunit, ngrid, nchunk, nadj;
     int max_M, max_N, threads;
     int64_t total_in;
     ce_grid **grids;
@@ -389,7 +389,7 @@ struct coffe_batch {
     ce_grid_dev *d_grids;
     ce_table_desc *d_tabs;
     ce_unit_dev *d_units;
-    ce_chunk_dev *d_chunks;
+    ce_chunk_dev *d_chunks; /* the resample chunks, then those of k_spline_adj */
     int32_t *d_ranges; /* resample index ranges per chunk (4 each), from the prepare stage */
     int32_t *d_packs;  /* table workgroups: first unit, unit count, groups, 0 */
     int npack, lt_off;
@@ -482,6 +482,51 @@ static int64_t chunk_points(int nspec, const int64_t *n_in, const int64_t *n_fft
     }
 }
 
+/*
+ * k_spline_adj takes whole runs of resample chunks: `merge` of them (512 intervals at most) in a
+ * chunk.  It scatters the grid points of 64 intervals to either side of its own as well, so
+ * with few samples a spectrum short chunks do the same points again many times over; a chunk of
+ * `steps` wavefront steps of 64 points takes about 10 us + 0.55 us a step alone on its CU, and
+ * every further chunk there 0.33 us a step (the LDS atomics).  200 samples on 10000 points, 200
+ * spectra: 487 us in the resample's chunks of 8 intervals, 90 in one a spectrum; 600 samples,
+ * 51 spectra: 168 in chunks of 8, 40 of 128, 80 of 512; one spectrum: 23, 39 and 80.
+ */
+static int adj_merged(int len, int merge)
+{
+    const int most = CE_CHUNK / len;
+    return merge < most ? merge : most;
+}
+
+static double adj_time(int nspec, const int64_t *n_in, const int64_t *n_fft, int64_t points, int merge)
+{
+    double most = 0.0, sum = 0.0, chunks = 0.0;
+    for (int s = 0; s < nspec; ++s) {
+        const int len = chunk_len(n_in[s], n_fft[s], points);
+        const double nint = (double)n_in[s] - 1, c = (double)len * adj_merged(len, merge), n = ceil(nint / c);
+        const double staged = c + 2 * CE_SPLINE_HALO < nint ? c + 2 * CE_SPLINE_HALO : nint;
+        const double steps = staged / nint * (double)n_fft[s] / 64;
+        if (steps > most) most = steps;
+        sum += n * steps;
+        chunks += n;
+    }
+    return 10.0 + 0.22 * most + 0.33 * ceil(chunks / 256) * (sum / chunks);
+}
+
+/* runs twice as long where they gain 3 %: below that short ones (2 x 51 chunks of 1024 samples) are ahead */
+static int adj_merge(int nspec, const int64_t *n_in, const int64_t *n_fft, int64_t points)
+{
+    int best = 1;
+    double t = adj_time(nspec, n_in, n_fft, points, 1);
+    for (int m = 2; m <= CE_CHUNK / 8; m *= 2) {
+        const double tm = adj_time(nspec, n_in, n_fft, points, m);
+        if (tm < 0.97 * t) {
+            t = tm;
+            best = m;
+        }
+    }
+    return best;
+}
+
 int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const int64_t *n_fft, const double *kmin,
                        const double *kmax, int ntab, const int *tab_n, const int *tab_l, int nsep, const double *sep,
                        int nz, int nl, coffe_batch **out)
@@ -567,21 +612,32 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
             const int len = chunk_len(n_in[s], n_fft[s], points);
             b->nchunk += (int)((n_in[s] - 1 + len - 1) / len);
         }
-        chunks = (ce_chunk_dev *)malloc(sizeof(ce_chunk_dev) * (size_t)b->nchunk);
+        /* at most as many of the adjoint */
+        chunks = (ce_chunk_dev *)malloc(sizeof(ce_chunk_dev) * 2 * (size_t)b->nchunk);
         if (!chunks) st = COFFE_ENOMEM;
+        const int merge = adj_merge(nspec, n_in, n_fft, points);
         int c = 0;
         for (int s = 0; s < nspec && st == COFFE_OK; ++s) {
             const int nint = (int)n_in[s] - 1, len = chunk_len(n_in[s], n_fft[s], points);
             for (int a = 0; a < nint; a += len) {
-                chunks[c].spec = s;
                 chunks[c].grid = b->h_spec[s].grid;
                 chunks[c].in_off = b->h_spec[s].in_off;
                 chunks[c].ws_off = b->h_spec[s].ws_off;
                 chunks[c].n_in = b->h_spec[s].n_in;
-                chunks[c].id = c;
+                chunks[c].id = chunks[c].last = c;
                 chunks[c].a = a;
                 chunks[c].b = a + len < nint ? a + len : nint;
                 ++c;
+            }
+        }
+        b->nadj = 0;
+        for (c = 0; c < b->nchunk && st == COFFE_OK;) {
+            ce_chunk_dev *q = &chunks[b->nchunk + b->nadj++];
+            *q = chunks[c];
+            const int m = adj_merged(q->b - q->a, merge);
+            while (++c < b->nchunk && chunks[c].a != 0 && c < q->id + m) {
+                q->b = chunks[c].b;
+                q->last = c;
             }
         }
     }
@@ -599,7 +655,7 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_grids, sizeof(ce_grid_dev) * (size_t)b->ngrid);
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_tabs, sizeof(ce_table_desc) * (size_t)ntab);
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_units, sizeof(ce_unit_dev) * (size_t)b->nunit);
-    if (st == COFFE_OK) st = dev_alloc((void **)&b->d_chunks, sizeof(ce_chunk_dev) * (size_t)b->nchunk);
+    if (st == COFFE_OK) st = dev_alloc((void **)&b->d_chunks, sizeof(ce_chunk_dev) * (size_t)(b->nchunk + b->nadj));
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_ranges, 4 * sizeof(int32_t) * (size_t)b->nchunk);
     if (st == COFFE_OK) st = hip_ok(hipMemset(b->d_ranges, 0, 4 * sizeof(int32_t) * (size_t)b->nchunk));
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_sidx, sizeof(int32_t) * (size_t)b->ngrid * (size_t)nsep);
@@ -676,7 +732,8 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_grids, hg, sizeof(ce_grid_dev) * (size_t)b->ngrid, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_tabs, tabs, sizeof(ce_table_desc) * (size_t)ntab, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_units, units, sizeof(ce_unit_dev) * (size_t)b->nunit, hipMemcpyHostToDevice, s));
-    if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_chunks, chunks, sizeof(ce_chunk_dev) * (size_t)b->nchunk, hipMemcpyHostToDevice, s));
+    if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_chunks, chunks, sizeof(ce_chunk_dev) * (size_t)(b->nchunk + b->nadj),
+                                                      hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_sidx, sidx, sizeof(int32_t) * (size_t)b->ngrid * (size_t)nsep, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_sep, sep, sizeof(double) * (size_t)nsep, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipStreamSynchronize(s));
@@ -723,8 +780,8 @@ int coffe_batch_adj_c2r(coffe_batch *b, void *stream)
 int coffe_batch_spline_adj(coffe_batch *b, const double *d_k, double *d_gpk, void *stream)
 {
     if (!b || !d_k || !d_gpk) return COFFE_EINVAL;
-    return ce_launch_spline_adj(pick_stream(b, stream), b->nchunk, b->d_chunks, b->d_spec, b->d_grids, d_k, b->d_ws,
-                                d_gpk, b->d_ranges)
+    return ce_launch_spline_adj(pick_stream(b, stream), b->nadj, b->d_chunks + b->nchunk, b->d_spec, b->d_grids, d_k,
+                                b->d_ws, d_gpk, b->d_ranges)
                ? COFFE_EDEVICE
                : COFFE_OK;
 }
@@ -767,7 +824,8 @@ int coffe_batch_prepare_adj(coffe_batch *b, const double *d_k, const double *d_p
     if (ce_launch_adj_c2r(s, b->nspec, b->d_spec, b->d_grids, b->d_tabs, b->ntab, b->nq, b->d_ws, b->d_xb,
                           b->threads, b->max_M, NULL, NULL, NULL, 0, 0, 0))
         return COFFE_EDEVICE;
-    return ce_launch_spline_adj(s, b->nchunk, b->d_chunks, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk, b->d_ranges)
+    return ce_launch_spline_adj(s, b->nadj, b->d_chunks + b->nchunk, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk,
+                                b->d_ranges)
                ? COFFE_EDEVICE
                : COFFE_OK;
 }
@@ -804,7 +862,8 @@ int coffe_batch_vjp(coffe_batch *b, const double *d_k, const double *d_pk, const
     if (ce_launch_adj_c2r(s, b->nspec, b->d_spec, b->d_grids, b->d_tabs, b->ntab, b->nq, b->d_ws, b->d_xb,
                           b->threads, b->max_M, d_A, itab, d_out, b->nz, b->nl, b->nsep))
         return COFFE_EDEVICE;
-    return ce_launch_spline_adj(s, b->nchunk, b->d_chunks, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk, b->d_ranges)
+    return ce_launch_spline_adj(s, b->nadj, b->d_chunks + b->nchunk, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk,
+                                b->d_ranges)
                ? COFFE_EDEVICE
                : COFFE_OK;
 }
@@ -937,7 +996,7 @@ int twofast_1bessel_status(double *output_x, double *output_y, size_t output_len
     ce_chunk_dev *h_chunks = (ce_chunk_dev *)malloc(sizeof(ce_chunk_dev) * (size_t)nchunk);
     if (!h_chunks) { pthread_mutex_unlock(&e->lock); return COFFE_ENOMEM; }
     for (int c = 0; c < nchunk; ++c) {
-        h_chunks[c].spec = 0;
+        h_chunks[c].last = c;
         h_chunks[c].grid = 0;
         h_chunks[c].in_off = 0;
         h_chunks[c].ws_off = 0;
@@ -1717,7 +1776,7 @@ int coffe_integral_tables(int ntab, const int *n, const int *l, size_t N, const 
     memset(ch, 0, sizeof(ce_chunk_dev) * (size_t)nchunk);
     for (int c = 0; c < nchunk; ++c) {
         ch[c].n_in = (int32_t)nin;
-        ch[c].id = c;
+        ch[c].id = ch[c].last = c;
         ch[c].a = c * len;
         ch[c].b = (c + 1) * len < (int)nin - 1 ? (c + 1) * len : (int)nin - 1;
     }

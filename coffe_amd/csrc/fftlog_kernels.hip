@@ -160,8 +160,6 @@ __global__ void k_grid_tables(grid_tab_args a)
 // LDL^T multiplier gamma is below 1/2), 5e-20 for W = 64; the global ends carry the
 // exact natural boundary c_0 = c_{n-1} = 0.
 
-#define CE_SPLINE_HALO 64
-
 // 1/x within about one ulp without the division sequence: the hardware estimate
 // refined by two Newton steps (no VCC, so independent reciprocals overlap); for
 // normal x of moderate size, as the spacings and diagonals here are
@@ -1002,9 +1000,9 @@ __global__ void __launch_bounds__(64) k_spline_adj(const ce_chunk_dev *__restric
         if (i < cnt) kv[u] = k[G.lo + i];
     }
     // resample points with intervals in the staged range [lo, hi), as k_resample of
-    // the same prepare stage found them
+    // the same prepare stage found them for the first and the last of its chunks here
     // (clamped to the grid, so that a stage run out of order stays in bounds)
-    const int i1 = min(max(ranges[4 * ch.id + 3], 0), N);
+    const int i1 = min(max(ranges[4 * ch.last + 3], 0), N);
     const int i0 = min(max(ranges[4 * ch.id + 2], 0), i1);
     const double klo = k[0], khi = k[n - 1];
     // loads at clamped indices, unconditionally, so that they all go out at once

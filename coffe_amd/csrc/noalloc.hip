@@ -94,7 +94,7 @@ __global__ void k_noalloc_setup(setup_args a)
     if (i < a.nchunk) {
         const int nint = (int)a.n - 1;
         ce_chunk_dev c;
-        c.spec = 0;
+        c.last = (int32_t)i;
         c.grid = 0;
         c.in_off = 0;
         c.ws_off = 0;

@@ -137,3 +137,35 @@ def test_vjp_exact_dot_product_white_noise(engine, tables):
               f"rel {abs(lhs - rhs) / scale:.2e}", flush=True)
         assert abs(lhs - rhs) <= 1e-9 * scale, (trial, lhs, rhs)
     b.close()
+
+
+@pytest.mark.parametrize("n,N,nspec", [(7, 1024, 3), (70, 4096, 40), (200, 10000, 1), (200, 10000, 60), (600, 10000, 16),
+                                       (1300, 8192, 30), (1025, 16384, 2)])
+def test_adjoint_chunks_of_few_samples(engine, n, N, nspec):
+    """few samples on a long grid: k_spline_adj takes runs of the resample's chunks (one chunk, a run that ends
+    inside the spectrum, a whole spectrum, spectra of two lengths).  A batch's gradients against
+    those of its spectra one at a time, which take other runs: 1e-12 of the largest, for sums of up to 200
+    points an interval in another order"""
+    import torch
+    from coffe_amd.engine import Batch
+    from tests.synth import batch_spectra
+    specs = [s for m in (n, n + 3) for s in batch_spectra((nspec + 1) // 2, seed=n, lengths=(m,))][:nspec]
+    sep = np.linspace(20.0, 200.0, 9)
+    A = torch.ones((1, 2, 2, 9), dtype=torch.float64, device="cuda")
+    gout = torch.tensor(np.random.default_rng(2).standard_normal((nspec, 1, 2, 9)), device="cuda")
+
+    def grads(sel):
+        ns = [len(specs[i][0]) for i in sel]
+        b = Batch(engine, ns, [N] * len(sel), [specs[i][0][0] for i in sel], [specs[i][0][-1] for i in sel],
+                  [(0, 0), (1, 1)], sep, 1, 2)
+        gpk = b.vjp(torch.tensor(np.concatenate([specs[i][0] for i in sel]), device="cuda"),
+                    torch.tensor(np.concatenate([specs[i][1] for i in sel]), device="cuda"), A,
+                    gout[list(sel)].contiguous())[2].cpu().numpy()
+        b.close()
+        return np.split(gpk, np.cumsum(ns)[:-1])
+
+    print(f"adjoint chunks n={n} N={N} nspec={nspec}", flush=True)
+    both = grads(range(nspec))
+    for i in {0, nspec - 1}:
+        one = grads([i])[0]
+        assert np.isfinite(one).all() and np.max(np.abs(both[i] - one)) <= 1e-12 * np.max(np.abs(one))
