@@ -103,6 +103,8 @@ def load_library():
     L.coffe_cov_plan_destroy.restype = None
     L.coffe_cov_plan_rows.argtypes = [vp]
     L.coffe_cov_plan_pairs.argtypes = [vp]
+    L.coffe_cov_plan_set_path.argtypes = [vp, i]
+    L.coffe_cov_plan_path.argtypes = [vp]
     L.coffe_cov_integrals.argtypes = [vp, i, i64p, vp, vp, vp, vp]
     L.coffe_cov_integrals_vjp.argtypes = [vp, i, i64p, vp, vp, vp, vp, vp]
     L.coffe_cov_assemble_vjp.argtypes = [vp, i, i, ip, dp, dp, dp, dp, dp, dp, i, i, vp, vp, vp, dp, dp, vp]
@@ -133,6 +135,7 @@ EXPORTED = [
     "coffe_batch_resample", "coffe_batch_fft_prepare", "coffe_batch_adj_c2r", "coffe_batch_spline_adj",
     "coffe_mu_weights", "coffe_mu_weights_terms", "coffe_mu_weights_ex", "coffe_terms_of", "coffe_integral_table", "coffe_integral_tables", "coffe_integral_table_state", "coffe_divergent_tables", "coffe_divergent_tables_device", "coffe_batch_set_radix", "coffe_batch_small_r",
     "coffe_cov_plan_create", "coffe_cov_plan_destroy", "coffe_cov_plan_rows", "coffe_cov_plan_pairs",
+    "coffe_cov_plan_set_path", "coffe_cov_plan_path",
     "coffe_cov_integrals", "coffe_cov_integrals_vjp", "coffe_cov_assemble", "coffe_cov_assemble_vjp", "two_sph_bessel", "two_sph_bessel_status",
     "coffe_mu_weights_rule", "coffe_mu_weights_jvp", "coffe_fft_any", "coffe_flat_lensing_multipoles", "coffe_flat_lensing_corrfunc", "coffe_integrated_corrfunc", "coffe_refabi_set_spline_ops", "coffe_find_integral", "coffe_integrals_init",
     "coffe_integrals_free", "coffe_integrate", "coffe_multipoles_init", "coffe_multipoles_free",

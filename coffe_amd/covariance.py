@@ -51,6 +51,18 @@ class CovPlan:
         self.nrows = self.L.coffe_cov_plan_rows(h)
         self.pairs = [(i, j) for i in range(len(self.ls)) for j in range(i, len(self.ls))]
 
+    PATHS = ("auto", "rows", "contract")
+
+    def set_path(self, path):
+        """Whether the calls that follow are contractions over k ("contract"), row transforms ("rows") or
+        the faster of the two for their size ("auto", the default)."""
+        check(self.L.coffe_cov_plan_set_path(self.h, self.PATHS.index(path)), "coffe_cov_plan_set_path")
+
+    @property
+    def path(self):
+        """The way the last call went: "rows" or "contract" ("auto" before the first)."""
+        return self.PATHS[self.L.coffe_cov_plan_path(self.h)]
+
     def close(self):
         if self.h:
             self.L.coffe_cov_plan_destroy(self.h)

@@ -193,18 +193,17 @@ int ce_launch_cov_diag_vjp(void *stream, int nspec, int N, const double *d_dbar,
                            int64_t n_total);
 /* the integrals as contractions over k (cov_contract.hip): tables of nl 4 Rp Np doubles (Rp, Np: R
    and N rounded up to 16) and diagonals, nblk = 2 nspec rounded up to 16 of Np each, in
-   fragments; the adjoint reads the tables as plain rows (cov_unfold).  Splits of the
-   contracted range: d_part holds that many times the output (unused with one split), the
-   adjoint's [splits][nblk][Np] */
+   fragments; the adjoint reads the tables as plain rows (cov_unfold).  The contracted range is
+   split: d_part holds ce_cov_contract_work doubles of partial sums, the adjoint's
+   [splits][nblk][Np] */
 int ce_launch_cov_fold(void *stream, int nl, int N, int Np, int R, int Rp, const double *d_ahat, const double *d_bhat,
                        const int *d_lo, const int *d_cnt, const int *d_off, const double *d_uw, const double *d_fws,
                        const double *d_prn, double *d_tab);
 int ce_launch_cov_unfold(void *stream, int nl, int Np, int Rp, const double *d_tab, double *d_rows);
-int ce_cov_contract_splits(int nblk, int npair, int R, int Np);
+size_t ce_cov_contract_work(int nblk, int npair, int R, int Np);
 int ce_cov_contract_splits_T(int nblk, int npair, int R, int Np);
 int ce_launch_cov_contract(void *stream, int nblk, int Np, int R, int npair, const int *d_pl1, const int *d_pl2,
-                           const double *d_tab, const double *d_d, const double *d_fac, int nsplit, double *d_part,
-                           double *d_out);
+                           const double *d_tab, const double *d_d, const double *d_fac, double *d_part, double *d_out);
 int ce_launch_cov_contract_T(void *stream, int nblk, int N, int Np, int R, int npair, const int *d_pl1,
                              const int *d_pl2, const double *d_tab, const double *d_gint, const double *d_fac,
                              int nsplit, double *d_part, double *d_dbar);

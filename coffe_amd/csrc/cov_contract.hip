@@ -122,7 +122,9 @@ struct con_args {
     const double *tab;
     const double *d;         // [nblk / 16][Np / 16] fragments
     const double *fac;       // [2][npair]
-    double *out;             // [nsplit][nblk][npair][R][R], (m, n) at R n + m; scaled when nsplit = 1
+    int unit0, units;        // k_cov_few: the (diagonal, pair) units of this launch
+    double *out;             // k_cov_many: [nsplit][nblk][npair][R][R], (m, n) at R n + m, scaled when
+                             // nsplit = 1; k_cov_few: [nsplit][units][R][R]
 };
 
 // the fragments of rows 16 mt ... 16 mt + 15
@@ -243,19 +245,20 @@ __global__ void __launch_bounds__(256, 2) k_cov_many(con_args a)
 }
 
 // one diagonal and pair, a 32 x 32 tile (n, m) per wave; per step of 16 t 32 MFMAs against
-// nine 32-byte loads per lane, the next step's issued before them.  With splits every XCD
-// has its own ranges of t, so that its L2 holds the tables' part that all pairs and tiles
-// of a range read.
+// nine 32-byte loads per lane, the next step's issued before them.  nsplit is a multiple of the 8
+// XCDs, each of which has its own ranges of t, so that its L2 holds the tables' part that
+// all pairs and tiles of a range read (also where the tiles alone fill the chip: 4 spectra, 400
+// separations, N = 8000: 5.0 ms in 8 splits, 7.2 in one).
 __global__ void __launch_bounds__(256, 2) k_cov_few(con_args a)
 {
     const int lane = threadIdx.x & 63, q16 = lane & 15, g = lane >> 4;
-    const int E = (a.R + 31) / 32;
-    const int W = (E * E + 3) / 4 * a.npair * a.nblk;   // workgroups per split
+    const int E = (a.R + 31) / 32, wu = (E * E + 3) / 4;
+    const int W = wu * a.units;   // workgroups per split
     const int x = (int)blockIdx.x;
-    const int id = a.nsplit % 8 == 0 ? (x >> 3) % W : x % W;
-    const int z = a.nsplit % 8 == 0 ? (x >> 3) / W * 8 + (x & 7) : x / W;
-    const int w = id % ((E * E + 3) / 4) * 4 + (int)(threadIdx.x >> 6);
-    const int bp = id / ((E * E + 3) / 4);
+    const int id = (x >> 3) % W;
+    const int z = (x >> 3) / W * 8 + (x & 7);
+    const int w = id % wu * 4 + (int)(threadIdx.x >> 6);
+    const int unit = id / wu, bp = a.unit0 + unit;
     if (w >= E * E) return;
     const int m0 = (w % E) * 32, n0 = (w / E) * 32;
     const int pr = bp % a.npair, b = bp / a.npair;
@@ -309,8 +312,7 @@ __global__ void __launch_bounds__(256, 2) k_cov_few(con_args a)
                     for (int j = 0; j < 2; ++j)
                         if (!((h && !n2) || (j && !m2))) acc[h][j] = mfma(B[h][c][i], A[j][c][i], acc[h][j]);
     }
-    const double f = a.nsplit == 1 ? a.fac[(b & 1) * a.npair + pr] : 1.0;
-    double *o = a.out + (((int64_t)z * a.nblk + b) * a.npair + pr) * a.R * a.R;
+    double *o = a.out + ((int64_t)z * a.units + unit) * a.R * a.R;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -318,12 +320,12 @@ __global__ void __launch_bounds__(256, 2) k_cov_few(con_args a)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int n = n0 + 16 * h + crow(g, i), m = m0 + 16 * j + q16;
-                if (n < a.R && m < a.R) o[(int64_t)a.R * n + m] = acc[h][j][i] * f;
+                if (n < a.R && m < a.R) o[(int64_t)a.R * n + m] = acc[h][j][i];
             }
 }
 
-// out = fac sum_z part[z]: the splits in order
-__global__ void __launch_bounds__(256) k_cov_sum(int64_t n, int64_t RR, int npair, int nsplit,
+// out = fac sum_z part[z], the splits in order; the n values of units unit0, unit0 + 1, ...
+__global__ void __launch_bounds__(256) k_cov_sum(int64_t n, int64_t RR, int npair, int nsplit, int unit0,
                                                  const double *__restrict__ part, const double *__restrict__ fac,
                                                  double *__restrict__ out)
 {
@@ -331,14 +333,14 @@ __global__ void __launch_bounds__(256) k_cov_sum(int64_t n, int64_t RR, int npai
     if (e >= n) return;
     double s = part[e];
     for (int z = 1; z < nsplit; ++z) s += part[z * n + e];
-    const int64_t bp = e / RR;
-    out[e] = s * fac[((bp / npair) & 1) * npair + bp % npair];
+    const int64_t bp = unit0 + e / RR;
+    out[unit0 * RR + e] = s * fac[((bp / npair) & 1) * npair + bp % npair];
 }
 
 #define CE_FEW_T_N 64      // n per wave of k_cov_few_T
 
 struct conT_args {
-    int N, Np, R, Rp, npair, nblk, nsplit;
+    int Np, R, Rp, npair, nblk, nsplit;
     const int *pl1, *pl2;
     const double *tab;       // plain rows [nl][4][Rp][Np]
     const double *gint;      // [nblk][npair][R][R]
@@ -548,7 +550,7 @@ int splits(int64_t waves, int steps, int most)
 {
     int best = 1;
     double cost = 1e300;
-        for (int n = 1; n <= most; n += n < 8 ? 1 : 8) {
+    for (int n = 1; n <= most; n += n < 8 ? 1 : 8) {
         const double c = (double)((waves * n + 2047) / 2048) * ((steps + n - 1) / n + 2) + 2.0 * n;
         if (c < cost) {
             cost = c;
@@ -574,11 +576,18 @@ int64_t many_tiles(int nblk, int npair, int R)
 
 int many_groups(int nblk) { return (nblk + 16 * many_st(nblk) - 1) / (16 * many_st(nblk)); }
 
-}  // namespace
+// The forward's partial sums keep to WORK bytes (the doubles of one unit's splits, 64 R^2 bytes, at the
+// least): k_cov_many takes fewer splits, k_cov_few its (diagonal, pair) units in groups.
+constexpr int64_t WORK = (int64_t)512 << 20;
 
-extern "C" int ce_cov_contract_splits(int nblk, int npair, int R, int Np)
+int many_splits(int nblk, int npair, int R, int Np)
 {
-    if (many(nblk)) return splits(many_tiles(nblk, npair, R) * many_groups(nblk), Np / 16, 32);
+    const int64_t fit = WORK / ((int64_t)8 * nblk * npair * R * R);
+    return splits(many_tiles(nblk, npair, R) * many_groups(nblk), Np / 16, fit < 1 ? 1 : (fit > 32 ? 32 : (int)fit));
+}
+
+int few_splits(int nblk, int npair, int R, int Np)
+{
     const int64_t E = (R + 31) / 32;
     const int64_t waves = (E * E + 3) / 4 * 4 * npair * nblk;
     int n = (int)((3072 + waves - 1) / waves);   // 1.5 waves a SIMD: 130 us at 16 splits of 192 waves, 153 at 8, 135 at 32
@@ -586,6 +595,27 @@ extern "C" int ce_cov_contract_splits(int nblk, int npair, int R, int Np)
     if (n > 32) n = 32;
     while (n > 8 && n > Np / 128) n -= 8;
     return n;
+}
+
+// units per launch: as many as WORK holds, the launches alike
+int few_units(int nblk, int npair, int R, int nsplit)
+{
+    const int64_t all = (int64_t)nblk * npair, fit = WORK / ((int64_t)8 * nsplit * R * R);
+    const int64_t most = fit < 1 ? 1 : fit;
+    return (int)((all + (all + most - 1) / most - 1) / ((all + most - 1) / most));
+}
+
+}  // namespace
+
+extern "C" size_t ce_cov_contract_work(int nblk, int npair, int R, int Np)
+{
+    const size_t RR = (size_t)R * R;
+    if (many(nblk)) {
+        const int n = many_splits(nblk, npair, R, Np);
+        return n > 1 ? (size_t)n * nblk * npair * RR : 0;
+    }
+    const int n = few_splits(nblk, npair, R, Np);
+    return (size_t)n * few_units(nblk, npair, R, n) * RR;
 }
 
 extern "C" int ce_cov_contract_splits_T(int nblk, int npair, int R, int Np)
@@ -615,26 +645,37 @@ extern "C" int ce_launch_cov_unfold(void *stream, int nl, int Np, int Rp, const 
 
 extern "C" int ce_launch_cov_contract(void *stream, int nblk, int Np, int R, int npair, const int *d_pl1,
                                       const int *d_pl2, const double *d_tab, const double *d_d, const double *d_fac,
-                                      int nsplit, double *d_part, double *d_out)
+                                      double *d_part, double *d_out)
 {
+    const int64_t RR = (int64_t)R * R;
     con_args a;
-    a.Np = Np; a.R = R; a.Rp = (R + 15) / 16 * 16; a.npair = npair; a.nblk = nblk; a.nsplit = nsplit;
+    a.Np = Np; a.R = R; a.Rp = (R + 15) / 16 * 16; a.npair = npair; a.nblk = nblk;
     a.pl1 = d_pl1; a.pl2 = d_pl2; a.tab = d_tab; a.d = d_d; a.fac = d_fac;
-    a.out = nsplit == 1 ? d_out : d_part;
+    a.unit0 = 0;
+    a.units = nblk * npair;
     hipStream_t s = (hipStream_t)stream;
+    auto sum = [&](int unit0, int units) {
+        const int64_t n = units * RR;
+        hipLaunchKernelGGL(k_cov_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, RR, npair, a.nsplit, unit0,
+                           d_part, d_fac, d_out);
+    };
     if (many(nblk)) {
+        a.nsplit = many_splits(nblk, npair, R, Np);
+        a.out = a.nsplit == 1 ? d_out : d_part;
         const int64_t wgs = (many_tiles(nblk, npair, R) + 3) / 4;
-        const dim3 grid((unsigned)((wgs + 7) / 8 * 8 * many_groups(nblk)), 1, (unsigned)nsplit);
+        const dim3 grid((unsigned)((wgs + 7) / 8 * 8 * many_groups(nblk)), 1, (unsigned)a.nsplit);
         if (many_st(nblk) == 1) hipLaunchKernelGGL(k_cov_many<1>, grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL(k_cov_many<2>, grid, dim3(256), 0, s, a);
-    } else {
-        const int E = (R + 31) / 32;
-        hipLaunchKernelGGL(k_cov_few, dim3((unsigned)((E * E + 3) / 4 * npair * nblk * nsplit)), dim3(256), 0, s, a);
+        if (a.nsplit > 1) sum(0, a.units);
+        return (int)hipGetLastError();
     }
-    if (nsplit > 1) {
-        const int64_t n = (int64_t)nblk * npair * R * R;
-        hipLaunchKernelGGL(k_cov_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, (int64_t)R * R, npair,
-                           nsplit, d_part, d_fac, d_out);
+    a.nsplit = few_splits(nblk, npair, R, Np);
+    a.out = d_part;
+    const int E = (R + 31) / 32, all = nblk * npair, most = few_units(nblk, npair, R, a.nsplit);
+    for (a.unit0 = 0; a.unit0 < all; a.unit0 += most) {
+        a.units = all - a.unit0 < most ? all - a.unit0 : most;
+        hipLaunchKernelGGL(k_cov_few, dim3((unsigned)((E * E + 3) / 4 * a.units * a.nsplit)), dim3(256), 0, s, a);
+        sum(a.unit0, a.units);
     }
     return (int)hipGetLastError();
 }
@@ -644,7 +685,7 @@ extern "C" int ce_launch_cov_contract_T(void *stream, int nblk, int N, int Np, i
                                         const double *d_fac, int nsplit, double *d_part, double *d_dbar)
 {
     conT_args a;
-    a.N = N; a.Np = Np; a.R = R; a.Rp = (R + 15) / 16 * 16; a.npair = npair; a.nblk = nblk; a.nsplit = nsplit;
+    a.Np = Np; a.R = R; a.Rp = (R + 15) / 16 * 16; a.npair = npair; a.nblk = nblk; a.nsplit = nsplit;
     a.pl1 = d_pl1; a.pl2 = d_pl2; a.tab = d_tab; a.gint = d_gint; a.fac = d_fac; a.part = d_part;
     hipStream_t s = (hipStream_t)stream;
     if (many(nblk)) {

@@ -273,6 +273,8 @@ struct coffe_cov_plan {
     int *d_uelo, *d_uehi;   /* monotone envelopes of the windows in row order (adjoint) */
     /* the contraction's tables (cov_contract.hip); NULL: the integrals go row by row */
     int Np;            /* N rounded up to 16: the stride of the diagonals and of the tables' rows */
+    int path, ran;     /* the caller's choice and what the last call took (COFFE_COV_*) */
+    int no_tab;        /* their memory could not be had in a call: the plan keeps to the rows */
     double *d_tab;
     double *d_tabT;    /* the same as plain rows, made at the first adjoint call */
     /* per call, grown on demand; d_W: the rows' column functionals, or the contraction's splits */
@@ -288,7 +290,9 @@ struct coffe_cov_plan {
     double *d_Wbar, *d_dbar;
 };
 
-/* the contraction's tables take 32 bytes per multipole, separation and k; at most 16 of the 288 GB */
+/* the contraction's tables take 32 bytes per multipole, separation and k, twice that once the adjoint has
+   run (which lengths outside the LDS kernels do not have): at most 16 of the 288 GB in all.  The
+   partial sums beside them stay below 512 MB (cov_contract.hip). */
 #define TAB_CONTRACT ((size_t)16 << 30)
 static size_t contract_bytes(int nl, int N, int R)
 {
@@ -313,10 +317,15 @@ static int contract_faster(const coffe_cov_plan *p, int nblk, int adjoint)
     return con < row;
 }
 
+static int contract_fits(const coffe_cov_plan *p)
+{
+    return (p->fft ? 1 : 2) * contract_bytes(p->nl, p->N, p->R) <= TAB_CONTRACT;
+}
+
 /* whether any call of a plan would take the contraction: the tables are made then */
 static int contract_ok(const coffe_cov_plan *p)
 {
-    return contract_bytes(p->nl, p->N, p->R) <= TAB_CONTRACT &&
+    return contract_fits(p) &&
            (contract_faster(p, 2, 0) || contract_faster(p, 2, 1) || contract_faster(p, 16, 0) || contract_faster(p, 16, 1));
 }
 
@@ -344,6 +353,81 @@ static int upload(void **d, const void *h, size_t bytes, hipStream_t s)
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(*d, h, bytes, hipMemcpyHostToDevice, s));
     return st;
 }
+
+/* the contraction's tables, from the arrays already on the device; B: the column axis' array (NULL: read
+   back).  Nothing is left behind on failure. */
+static int contract_tables(coffe_cov_plan *p, const double *B)
+{
+    const int N = p->N, R = p->R, nl = p->nl;
+    const size_t nb = 2 * sizeof(double) * (size_t)N * (size_t)nl;
+    hipStream_t s = p->e->stream;
+    /* with the c2r's weights, zero above N/2, transformed as A is */
+    double *Bf = (double *)calloc(2 * (size_t)N * (size_t)nl, sizeof(double)), *Bh = NULL;
+    double *d_Bf = NULL, *d_bhat = NULL;
+    int st = Bf ? COFFE_OK : COFFE_ENOMEM;
+    if (st == COFFE_OK && !B) {
+        const size_t bytes = 2 * sizeof(double) * (size_t)(N / 2 + 1) * (size_t)nl;
+        Bh = (double *)malloc(bytes);
+        st = Bh ? ce_hip_ok(hipMemcpy(Bh, p->d_B, bytes, hipMemcpyDeviceToHost)) : COFFE_ENOMEM;
+        B = Bh;
+    }
+    for (int i = 0; i < nl && st == COFFE_OK; ++i)
+        for (int q = 0; q <= N / 2; ++q)
+            for (int c = 0; c < 2; ++c)
+                Bf[2 * ((size_t)N * i + q) + c] = B[2 * ((size_t)(N / 2 + 1) * i + q) + c] *
+                                                  (q == 0 || q == N / 2 ? 1.0 : 2.0);
+    if (st == COFFE_OK) st = upload((void **)&d_Bf, Bf, nb, s);
+    if (st == COFFE_OK) st = ce_dev_alloc((void **)&d_bhat, nb);
+    if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_tab, contract_bytes(nl, N, R));
+    if (st == COFFE_OK) {
+        if (p->fft) st = ce_general_cov_ahat(p->fft, s, nl, N, d_Bf, d_bhat);
+        else if (ce_launch_cov_ahat(s, nl, N, &p->rpN, p->d_tw, d_Bf, d_bhat)) st = COFFE_EDEVICE;
+    }
+    if (st == COFFE_OK && ce_launch_cov_fold(s, nl, N, p->Np, R, (R + 15) / 16 * 16, p->d_ahat, d_bhat, p->d_flo,
+                                             p->d_fcnt, p->d_foff, p->d_fw, p->d_fws, p->d_prn1, p->d_tab))
+        st = COFFE_EDEVICE;
+    const int sync = ce_hip_ok(hipStreamSynchronize(s));   /* Bf and the device arrays are released here */
+    if (st == COFFE_OK) st = sync;
+    free(Bf);
+    free(Bh);
+    hipFree(d_Bf);
+    hipFree(d_bhat);
+    if (st != COFFE_OK) {
+        hipFree(p->d_tab);
+        p->d_tab = NULL;
+    }
+    return st;
+}
+
+/* whether a call of nblk diagonals takes the contraction; its tables are there then */
+static int contract_now(coffe_cov_plan *p, int nblk, int adjoint)
+{
+    if (p->path == COFFE_COV_ROWS || p->no_tab || !contract_fits(p) ||
+        (p->path == COFFE_COV_AUTO && !contract_faster(p, nblk, adjoint)))
+        return 0;
+    if (!p->d_tab && contract_tables(p, NULL) != COFFE_OK) p->no_tab = 1;
+    return p->d_tab != NULL;
+}
+
+/* a call's workspace beside the tables could not be had: their memory goes to the rows */
+static void contract_drop(coffe_cov_plan *p)
+{
+    hipFree(p->d_tab);
+    hipFree(p->d_tabT);
+    p->d_tab = p->d_tabT = NULL;
+    p->no_tab = 1;
+}
+
+int coffe_cov_plan_set_path(coffe_cov_plan *p, int path)
+{
+    if (!p || path < COFFE_COV_AUTO || path > COFFE_COV_CONTRACT) return COFFE_EINVAL;
+    if (path == COFFE_COV_CONTRACT && !contract_fits(p)) return COFFE_EUNSUPPORTED;
+    p->path = path;
+    if (path == COFFE_COV_CONTRACT) p->no_tab = 0;
+    return COFFE_OK;
+}
+
+int coffe_cov_plan_path(const coffe_cov_plan *p) { return p ? p->ran : 0; }
 
 int coffe_cov_plan_create(coffe_engine *e, int N, double kmin, double kmax, int nl, const int *ls, int R,
                           const double *sep, coffe_cov_plan **out)
@@ -479,34 +563,12 @@ int coffe_cov_plan_create(coffe_engine *e, int N, double kmin, double kmax, int 
         if (p->fft) st = ce_general_cov_ahat(p->fft, s, nl, N, p->d_A, p->d_ahat);
         else if (ce_launch_cov_ahat(s, nl, N, &p->rpN, p->d_tw, p->d_A, p->d_ahat)) st = COFFE_EDEVICE;
     }
-    p->Np = N;
-    double *d_Bf = NULL, *d_bhat = NULL;
+    p->Np = (N + 15) / 16 * 16;
     if (st == COFFE_OK && contract_ok(p)) {
-        /* the column axis' array with the c2r's weights, zero above N/2, transformed as A is */
-        p->Np = (N + 15) / 16 * 16;
-        double *Bf = (double *)calloc(2 * (size_t)N * (size_t)nl, sizeof(double));
-        if (!Bf) st = COFFE_ENOMEM;
-        for (int i = 0; i < nl && st == COFFE_OK; ++i)
-            for (int q = 0; q <= N / 2; ++q)
-                for (int c = 0; c < 2; ++c)
-                    Bf[2 * ((size_t)N * i + q) + c] = B[2 * ((size_t)(N / 2 + 1) * i + q) + c] *
-                                                      (q == 0 || q == N / 2 ? 1.0 : 2.0);
-        if (st == COFFE_OK) st = upload((void **)&d_Bf, Bf, 2 * nb * (size_t)nl, s);
-        if (st == COFFE_OK) st = ce_dev_alloc((void **)&d_bhat, 2 * nb * (size_t)nl);
-        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_tab, contract_bytes(nl, N, R));
-        if (st == COFFE_OK) {
-            if (p->fft) st = ce_general_cov_ahat(p->fft, s, nl, N, d_Bf, d_bhat);
-            else if (ce_launch_cov_ahat(s, nl, N, &p->rpN, p->d_tw, d_Bf, d_bhat)) st = COFFE_EDEVICE;
-        }
-        if (st == COFFE_OK && ce_launch_cov_fold(s, nl, N, p->Np, R, (R + 15) / 16 * 16, p->d_ahat, d_bhat, p->d_flo,
-                                                 p->d_fcnt, p->d_foff, p->d_fw, p->d_fws, p->d_prn1, p->d_tab))
-            st = COFFE_EDEVICE;
-        const int sync = ce_hip_ok(hipStreamSynchronize(s));   /* Bf and the device arrays are released here */
-        if (st == COFFE_OK) st = sync;
-        free(Bf);
+        st = contract_tables(p, B);
+        if (st == COFFE_ENOMEM) st = COFFE_OK;   /* the first call that wants them tries again, or does without */
     }
     if (st == COFFE_OK) st = ce_hip_ok(hipStreamSynchronize(s));
-    hipFree(d_Bf); hipFree(d_bhat);
     free(k); free(r); free(k3); free(kn); free(prn); free(tw); free(A); free(B);
     free(mark); free(pos); free(rows); free(upos);
     functionals_free(&f);
@@ -518,32 +580,34 @@ int coffe_cov_plan_create(coffe_engine *e, int N, double kmin, double kmax, int 
 int coffe_cov_plan_rows(const coffe_cov_plan *p) { return p ? p->nrows : 0; }
 int coffe_cov_plan_pairs(const coffe_cov_plan *p) { return p ? p->npair : 0; }
 
-static size_t wsize(const coffe_cov_plan *p, int nspec, int contract)
+/* room for nspec spectra */
+static int grow(coffe_cov_plan *p, int nspec)
 {
-    const size_t blk = 2 * (size_t)nspec * (size_t)p->npair * (size_t)p->R;
-    if (!contract) return blk * (size_t)p->nrows;
-    const int ns = ce_cov_contract_splits(2 * nspec, p->npair, p->R, p->Np);
-    return ns > 1 ? blk * (size_t)p->R * (size_t)ns : 0;
+    if (nspec <= p->spec_cap) return COFFE_OK;
+    hipFree(p->d_in_off); hipFree(p->d_n_in); hipFree(p->d_d);
+    p->d_in_off = NULL; p->d_n_in = NULL; p->d_d = NULL; p->spec_cap = 0;
+    int st = ce_dev_alloc((void **)&p->d_in_off, sizeof(int64_t) * (size_t)nspec);
+    if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_n_in, sizeof(int32_t) * (size_t)nspec);
+    if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_d, sizeof(double) * 16 * (size_t)p->Np * (size_t)((nspec + 7) / 8));
+    if (st == COFFE_OK) p->spec_cap = nspec;
+    return st;
 }
 
-static int grow(coffe_cov_plan *p, int nspec, size_t w)
+/* a workspace of n doubles */
+static int grow_work(double **w, size_t *cap, size_t n)
 {
-    int st = COFFE_OK;
-    if (nspec > p->spec_cap) {
-        hipFree(p->d_in_off); hipFree(p->d_n_in); hipFree(p->d_d);
-        p->d_in_off = NULL; p->d_n_in = NULL; p->d_d = NULL; p->spec_cap = 0;
-        st = ce_dev_alloc((void **)&p->d_in_off, sizeof(int64_t) * (size_t)nspec);
-        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_n_in, sizeof(int32_t) * (size_t)nspec);
-        if (st == COFFE_OK) st = ce_dev_alloc((void **)&p->d_d, sizeof(double) * 16 * (size_t)p->Np * (size_t)((nspec + 7) / 8));
-        if (st == COFFE_OK) p->spec_cap = nspec;
-    }
-    if (st == COFFE_OK && w > p->w_cap) {
-        hipFree(p->d_W);
-        p->d_W = NULL; p->w_cap = 0;
-        st = ce_dev_alloc((void **)&p->d_W, sizeof(double) * w);
-        if (st == COFFE_OK) p->w_cap = w;
-    }
+    if (n <= *cap) return COFFE_OK;
+    hipFree(*w);
+    *w = NULL; *cap = 0;
+    const int st = ce_dev_alloc((void **)w, sizeof(double) * n);
+    if (st == COFFE_OK) *cap = n;
     return st;
+}
+
+/* doubles of the rows' functionals (forward) or their cotangents */
+static size_t rows_work(const coffe_cov_plan *p, int nspec)
+{
+    return 2 * (size_t)nspec * (size_t)p->npair * (size_t)p->nrows * (size_t)p->R;
 }
 
 int coffe_cov_integrals(coffe_cov_plan *p, int nspec, const int64_t *n_in, const double *d_k, const double *d_pk,
@@ -563,9 +627,15 @@ int coffe_cov_integrals(coffe_cov_plan *p, int nspec, const int64_t *n_in, const
         cnt[i] = (int32_t)n_in[i];
         o += n_in[i];
     }
-    const int contract = p->d_tab && contract_faster(p, 2 * nspec, 0);
-    /* the splits shrink as spectra are added: the workspace is no multiple of nspec */
-    if (st == COFFE_OK) st = grow(p, nspec, wsize(p, nspec, contract));
+    if (st == COFFE_OK) st = grow(p, nspec);
+    int contract = st == COFFE_OK && contract_now(p, 2 * nspec, 0);
+    /* the splits shrink as spectra are added: the contraction's workspace is no multiple of nspec */
+    if (contract && grow_work(&p->d_W, &p->w_cap, ce_cov_contract_work(2 * nspec, p->npair, p->R, p->Np)) != COFFE_OK) {
+        contract_drop(p);
+        contract = 0;
+    }
+    if (st == COFFE_OK && !contract) st = grow_work(&p->d_W, &p->w_cap, rows_work(p, nspec));
+    p->ran = contract ? COFFE_COV_CONTRACT : COFFE_COV_ROWS;
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_in_off, off, sizeof(int64_t) * (size_t)nspec,
                                                       hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_n_in, cnt, sizeof(int32_t) * (size_t)nspec,
@@ -576,7 +646,7 @@ int coffe_cov_integrals(coffe_cov_plan *p, int nspec, const int64_t *n_in, const
         st = COFFE_EDEVICE;
     if (st == COFFE_OK && contract) {
         if (ce_launch_cov_contract(s, 2 * nspec, p->Np, p->R, p->npair, p->d_pl1, p->d_pl2, p->d_tab, p->d_d, p->d_fac,
-                                   ce_cov_contract_splits(2 * nspec, p->npair, p->R, p->Np), p->d_W, d_out))
+                                   p->d_W, d_out))
             st = COFFE_EDEVICE;
     } else if (st == COFFE_OK && p->fft)
         st = ce_general_cov_rows(p->fft, s, 2 * nspec, p->N, p->d_ahat, p->d_B, p->d_d, p->npair, p->d_pl1, p->d_pl2,
@@ -619,17 +689,28 @@ int coffe_cov_integrals_vjp(coffe_cov_plan *p, int nspec, const int64_t *n_in, c
         cnt[i] = (int32_t)n_in[i];
         o += n_in[i];
     }
-    const int contract = p->d_tab && contract_faster(p, 2 * nspec, 1);
-    if (st == COFFE_OK) st = grow(p, nspec, 0);
-    const int nsplit = contract ? ce_cov_contract_splits_T(2 * nspec, p->npair, p->R, p->Np) : 0;
-    const size_t need = contract ? 2 * (size_t)nspec * (size_t)nsplit * (size_t)p->Np
-                                 : 2 * (size_t)nspec * (size_t)p->npair * (size_t)p->nrows * (size_t)p->R;
-    if (st == COFFE_OK && need > p->wbar_cap) {
-        hipFree(p->d_Wbar);
-        p->d_Wbar = NULL; p->wbar_cap = 0;
-        st = ce_dev_alloc((void **)&p->d_Wbar, sizeof(double) * need);
-        if (st == COFFE_OK) p->wbar_cap = need;
+    if (st == COFFE_OK) st = grow(p, nspec);
+    int contract = st == COFFE_OK && contract_now(p, 2 * nspec, 1);
+    if (contract && !p->d_tabT) {
+        /* without room for the second copy the forward keeps the first */
+        double *rows = NULL;
+        if (ce_dev_alloc((void **)&rows, contract_bytes(p->nl, p->N, p->R)) != COFFE_OK) {
+            contract = 0;
+        } else if (ce_launch_cov_unfold(s, p->nl, p->Np, (p->R + 15) / 16 * 16, p->d_tab, rows)) {
+            hipFree(rows);
+            st = COFFE_EDEVICE;
+            contract = 0;
+        } else {
+            p->d_tabT = rows;
+        }
     }
+    const int nsplit = contract ? ce_cov_contract_splits_T(2 * nspec, p->npair, p->R, p->Np) : 0;
+    if (contract && grow_work(&p->d_Wbar, &p->wbar_cap, 2 * (size_t)nspec * (size_t)nsplit * (size_t)p->Np) != COFFE_OK) {
+        contract_drop(p);
+        contract = 0;
+    }
+    if (st == COFFE_OK && !contract) st = grow_work(&p->d_Wbar, &p->wbar_cap, rows_work(p, nspec));
+    p->ran = contract ? COFFE_COV_CONTRACT : COFFE_COV_ROWS;
     if (st == COFFE_OK && nspec > p->adj_cap) {
         hipFree(p->d_dbar);
         p->d_dbar = NULL; p->adj_cap = 0;
@@ -640,16 +721,6 @@ int coffe_cov_integrals_vjp(coffe_cov_plan *p, int nspec, const int64_t *n_in, c
                                                       hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = ce_hip_ok(hipMemcpyAsync(p->d_n_in, cnt, sizeof(int32_t) * (size_t)nspec,
                                                       hipMemcpyHostToDevice, s));
-    if (st == COFFE_OK && contract && !p->d_tabT) {
-        double *rows = NULL;
-        st = ce_dev_alloc((void **)&rows, contract_bytes(p->nl, p->N, p->R));
-        if (st == COFFE_OK && ce_launch_cov_unfold(s, p->nl, p->Np, (p->R + 15) / 16 * 16, p->d_tab, rows)) {
-            st = COFFE_EDEVICE;
-            hipFree(rows);
-        } else {
-            p->d_tabT = rows;
-        }
-    }
     if (st == COFFE_OK && contract) {
         if (ce_launch_cov_contract_T(s, 2 * nspec, p->N, p->Np, p->R, p->npair, p->d_pl1, p->d_pl2, p->d_tabT, d_gint,
                                      p->d_fac, nsplit, p->d_Wbar, p->d_dbar))

@@ -93,8 +93,11 @@ static int injected_failure(void)
 static int dev_alloc(void **p, size_t bytes)
 {
     if (bytes == 0) bytes = 8;
-    if (injected_failure()) { *p = NULL; return COFFE_ENOMEM; }
-    return hipMalloc(p, bytes) == hipSuccess ? COFFE_OK : COFFE_ENOMEM;
+    if (injected_failure()) bytes = (size_t)1 << 60;
+    if (hipMalloc(p, bytes) == hipSuccess) return COFFE_OK;
+    *p = NULL;
+    (void)hipGetLastError();   /* a caller that does without the memory goes on to its launches */
+    return COFFE_ENOMEM;
 }
 
 int ce_dev_alloc(void **p, size_t bytes) { return dev_alloc(p, bytes); }

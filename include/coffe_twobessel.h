@@ -52,6 +52,15 @@ void coffe_cov_plan_destroy(coffe_cov_plan *p);
 /* transform rows one call computes per (spectrum, power, pair); pairs l1 <= l2 */
 int coffe_cov_plan_rows(const coffe_cov_plan *p);
 int coffe_cov_plan_pairs(const coffe_cov_plan *p);
+/*
+ * The integrals and their adjoint are contractions over k with tables that the plan holds, or row
+ * transforms: by default the faster of the two for the call's size, and the rows where the tables
+ * cannot be allocated.  set_path chooses for the calls that follow (COFFE_EUNSUPPORTED for tables
+ * of more than 16 GiB); coffe_cov_plan_path tells which way the last call went.
+ */
+enum { COFFE_COV_AUTO = 0, COFFE_COV_ROWS = 1, COFFE_COV_CONTRACT = 2 };
+int coffe_cov_plan_set_path(coffe_cov_plan *p, int path);
+int coffe_cov_plan_path(const coffe_cov_plan *p);
 
 /*
  * The scaled FFTLog integrals of P and P^2 for nspec spectra (concatenated device
