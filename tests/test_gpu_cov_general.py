@@ -45,17 +45,20 @@ def test_two_sph_bessel_general_length(engine, l12):
     assert np.max(np.abs(res - ores)) <= 1e-11 * np.max(np.abs(ores)), np.max(np.abs(res - ores)) / np.max(np.abs(ores))
 
 
+@pytest.mark.parametrize("path", ["rows", "contract"])
 @pytest.mark.parametrize("N", [1792, 10000])
-def test_cov_integrals_general_length_vs_oracle(engine, N):
+def test_cov_integrals_general_length_vs_oracle(engine, N, path):
     import torch
     from coffe_amd import EngineError
     from coffe_amd.covariance import CovPlan
     k, pk = _fixture_spectrum()
     sep = np.arange(50, 350, 50) / H
     plan = CovPlan(engine, N, k[0], k[-1], LS, sep)
+    plan.set_path(path)
     print(f"cov integrals general N={N} rows={plan.nrows}", flush=True)
     kt, pt = torch.tensor(k, device="cuda"), torch.tensor(pk, device="cuda")
     got = plan.integrals(kt, pt, [len(k)]).cpu().numpy()
+    assert plan.path == path
     pairs = [(0, 2), (2, 2)] if N > 8192 else plan.pairs   # the oracle's 2D transform takes seconds at N = 10^4
     for (i, j) in pairs:
         q = plan.pairs.index((i, j))

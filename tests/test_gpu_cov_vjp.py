@@ -1,6 +1,7 @@
-"""Vector-Jacobian product of the covariance integrals (coffe_cov_integrals_vjp,
-cov_kernels.hip: the row functionals, row transforms and diagonal transposed, then
-the Akima spline's adjoint) against central finite differences of the forward
+"""Vector-Jacobian product of the covariance integrals (coffe_cov_integrals_vjp: as
+contractions over k, cov_contract.hip, and as the row functionals and row transforms
+transposed, cov_kernels.hip, then the diagonal's and the Akima spline's adjoint) against
+central finite differences of the forward
 integrals: for a random cotangent G and smooth random directions v of P,
 <gpk, v> = (<G, I(P + h v)> - <G, I(P - h v)>) / 2h, h = 1e-5, to 1e-7 of
 sum |gpk v|, on the fixture's spectrum.
@@ -21,6 +22,20 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 H = 0.67
+both_paths = pytest.mark.parametrize("path", ["rows", "contract"])
+
+
+def _plan(path, *args):
+    """a plan that takes `path` in its calls; the tests end with _close, which checks that it did"""
+    from coffe_amd.covariance import CovPlan
+    plan = CovPlan(*args)
+    plan.set_path(path)
+    return plan
+
+
+def _close(plan, path):
+    assert plan.path == path
+    plan.close()
 
 
 def _directions(ks, n, rng):
@@ -58,33 +73,33 @@ def _check(plan, ks_list, ps_list, rng, step=1e-5, tol=1e-7):
     return gpk
 
 
-def test_cov_vjp_single_spectrum(engine):
+@both_paths
+def test_cov_vjp_single_spectrum(engine, path):
     """The fixture's spectrum, N = 1024, l = 0, 2, 4 (6 pairs), 6 separations."""
     import os
-    from coffe_amd.covariance import CovPlan
     gold = os.path.join(os.path.dirname(__file__), "golden")
     k, pk = np.loadtxt(os.path.join(gold, "PkL_CLASS.dat")).T
     k, pk = k * H, pk / H ** 3
     sep = np.arange(50, 350, 50) / H
-    plan = CovPlan(engine, 1024, k[0], k[-1], [0, 2, 4], sep)
+    plan = _plan(path, engine, 1024, k[0], k[-1], [0, 2, 4], sep)
     print(f"cov vjp: N=1024 rows={plan.nrows}", flush=True)
     _check(plan, [k], [pk], np.random.default_rng(5))
-    plan.close()
+    _close(plan, path)
 
 
-def test_cov_vjp_batch(engine):
+@both_paths
+def test_cov_vjp_batch(engine, path):
     """Three spectra of different lengths in one call, N = 1000 (radix-10 passes),
     l = 0, 2: the homogeneity identity per spectrum, central differences along affine
     directions per spectrum, and the gradient of each spectrum depends on its own
     cotangent only."""
     import torch
-    from coffe_amd.covariance import CovPlan
     from tests.synth import batch_spectra
     specs = batch_spectra(3, seed=4, lengths=(1024, 2048))
     kmin = max(s[0][0] for s in specs)
     kmax = min(s[0][-1] for s in specs)
     sep = np.array([30.0, 47.0, 90.0, 150.0, 260.0])
-    plan = CovPlan(engine, 1000, kmin, kmax, [0, 2], sep)
+    plan = _plan(path, engine, 1000, kmin, kmax, [0, 2], sep)
     ks = [s[0] for s in specs]
     ps = [s[1] for s in specs]
     print(f"cov vjp: batch of 3, N=1000 rows={plan.nrows}", flush=True)
@@ -126,16 +141,16 @@ def test_cov_vjp_batch(engine):
     for s in (0, 2):
         np.testing.assert_allclose(g_part[o[s]:o[s + 1]], g_full[o[s]:o[s + 1]], rtol=0,
                                    atol=1e-12 * np.max(np.abs(g_full[o[s]:o[s + 1]])))
-    plan.close()
+    _close(plan, path)
 
 
-def test_cov_vjp_dense_shuffled_separations(engine):
+@both_paths
+def test_cov_vjp_dense_shuffled_separations(engine, path):
     """48 separations 10-200 Mpc/h (several per grid cell, so the row windows of the
     functionals are not monotone in the separation) given in a shuffled order, N = 2048:
     the homogeneity identity, and the gradient equals the one of the sorted plan with
     the cotangent permuted alike."""
     import torch
-    from coffe_amd.covariance import CovPlan
     from tests.synth import spectrum
     k_np, p_np = spectrum(4096)
     sep = np.linspace(10.0, 200.0, 48) / H
@@ -143,8 +158,8 @@ def test_cov_vjp_dense_shuffled_separations(engine):
     dev = dict(device="cuda", dtype=torch.float64)
     k = torch.tensor(k_np, **dev)
     p = torch.tensor(p_np, **dev)
-    ps = CovPlan(engine, 2048, k_np[0], k_np[-1], [0, 2], sep)
-    pu = CovPlan(engine, 2048, k_np[0], k_np[-1], [0, 2], sep[perm])
+    ps = _plan(path, engine, 2048, k_np[0], k_np[-1], [0, 2], sep)
+    pu = _plan(path, engine, 2048, k_np[0], k_np[-1], [0, 2], sep[perm])
     print(f"cov vjp: 48 shuffled seps, N=2048 rows={ps.nrows}", flush=True)
     G = torch.tensor(np.random.default_rng(2).standard_normal((1, 2, ps.npair, ps.R, ps.R)), **dev)
     Gu = G[:, :, :, perm][:, :, :, :, perm].contiguous()
@@ -156,8 +171,8 @@ def test_cov_vjp_dense_shuffled_separations(engine):
     rhs = (Gu[0, 0] * Iu[0, 0]).sum().item() + 2 * (Gu[0, 1] * Iu[0, 1]).sum().item()
     ref = (torch.abs(Gu[0, 0] * Iu[0, 0]).sum() + 2 * torch.abs(Gu[0, 1] * Iu[0, 1]).sum()).item()
     assert abs(lhs - rhs) <= 1e-12 * ref, (lhs, rhs)
-    ps.close()
-    pu.close()
+    _close(ps, path)
+    _close(pu, path)
 
 
 def _euler_and_affine(plan, k_np, p_np, seed, h=1e-3, affine_tol=1e-9):
@@ -190,29 +205,29 @@ def _euler_and_affine(plan, k_np, p_np, seed, h=1e-3, affine_tol=1e-9):
         assert abs(an - fd) <= affine_tol * scale, (trial, an, fd, scale)
 
 
-def test_cov_vjp_n8000(engine):
+@both_paths
+def test_cov_vjp_n8000(engine, path):
     """The adjoint at the covariance's default length N = 8000 (radix-10 transforms, about
     1200 rows), l = 0, 2, 4, 16 separations 10-200 Mpc/h, the fixture spectrum."""
     import os
-    from coffe_amd.covariance import CovPlan
     gold = os.path.join(os.path.dirname(__file__), "golden")
     k, pk = np.loadtxt(os.path.join(gold, "PkL_CLASS.dat")).T
     k, pk = k * H, pk / H ** 3
     sep = np.linspace(10.0, 200.0, 16) / H
-    plan = CovPlan(engine, 8000, k[0], k[-1], [0, 2, 4], sep)
+    plan = _plan(path, engine, 8000, k[0], k[-1], [0, 2, 4], sep)
     print(f"cov vjp: N=8000 rows={plan.nrows}", flush=True)
     _euler_and_affine(plan, k, pk, 21)
-    plan.close()
+    _close(plan, path)
 
 
-def test_cov_vjp_more_than_256_separations(engine):
-    """300 separations (the transposed column functionals run over them in chunks of 256,
-    so the second chunk is exercised), N = 512, l = 0, 2."""
-    from coffe_amd.covariance import CovPlan
+@both_paths
+def test_cov_vjp_more_than_256_separations(engine, path):
+    """300 separations (the rows' transposed column functionals run over them in chunks of 256,
+    so the second chunk is exercised; the contraction's waves take 64), N = 512, l = 0, 2."""
     from tests.synth import spectrum
     k_np, p_np = spectrum(2048)
     sep = np.linspace(10.0, 250.0, 300) / H
-    plan = CovPlan(engine, 512, k_np[0], k_np[-1], [0, 2], sep)
+    plan = _plan(path, engine, 512, k_np[0], k_np[-1], [0, 2], sep)
     print(f"cov vjp: 300 seps, N=512 rows={plan.nrows}", flush=True)
     _euler_and_affine(plan, k_np, p_np, 31)
-    plan.close()
+    _close(plan, path)

@@ -56,13 +56,15 @@ def _scaled(raw, l1, l2, power):
     return raw * (2 * l1 + 1) * (2 * l2 + 1) * (2.0 if power == 1 else 1.0) / np.pi / np.pi
 
 
+@pytest.mark.parametrize("path", ["rows", "contract"])
 @pytest.mark.parametrize("N", [1024])
-def test_cov_integrals_vs_oracle(engine, N):
+def test_cov_integrals_vs_oracle(engine, N, path):
     import torch
     from coffe_amd.covariance import CovPlan
     k, pk = _fixture_spectrum()
     sep = np.arange(50, 350, 50) / H
     plan = CovPlan(engine, N, k[0], k[-1], LS, sep)
+    plan.set_path(path)
     print(f"cov integrals N={N} rows={plan.nrows}", flush=True)
     got = plan.integrals(torch.tensor(k, device="cuda"), torch.tensor(pk, device="cuda"), [len(k)]).cpu().numpy()
     for q, (i, j) in enumerate(plan.pairs):
@@ -73,7 +75,8 @@ def test_cov_integrals_vs_oracle(engine, N):
     plan.close()
 
 
-def test_cov_integrals_batch_vs_oracle(engine):
+@pytest.mark.parametrize("path", ["rows", "contract"])
+def test_cov_integrals_batch_vs_oracle(engine, path):
     import torch
     from coffe_amd.covariance import CovPlan
     from tests.synth import batch_spectra
@@ -82,6 +85,7 @@ def test_cov_integrals_batch_vs_oracle(engine):
     kmax = min(s[0][-1] for s in specs)
     sep = np.array([30.0, 47.0, 90.0, 150.0, 260.0])
     plan = CovPlan(engine, 512, kmin, kmax, [0, 2], sep)
+    plan.set_path(path)
     k = torch.tensor(np.concatenate([s[0] for s in specs]), device="cuda")
     p = torch.tensor(np.concatenate([s[1] for s in specs]), device="cuda")
     got = plan.integrals(k, p, [len(s[0]) for s in specs]).cpu().numpy()
@@ -200,7 +204,8 @@ def test_cov_vs_reference_fixtures(engine):
     assert worst < 2e-3
 
 
-def test_cov_integrals_n8000_vs_oracle(engine):
+@pytest.mark.parametrize("path", ["rows", "contract"])
+def test_cov_integrals_n8000_vs_oracle(engine, path):
     """The covariance's default transform length (covariance_integration_bins = 8000, the
     bench's configuration) against the oracle's generic N x N transform and bicubic:
     the fixture spectrum, 16 separations 10-200 Mpc/h, pairs (0, 2) and (4, 4), P and P^2,
@@ -210,6 +215,7 @@ def test_cov_integrals_n8000_vs_oracle(engine):
     k, pk = _fixture_spectrum()
     sep = np.linspace(10.0, 200.0, 16) / H
     plan = CovPlan(engine, 8000, k[0], k[-1], LS, sep)
+    plan.set_path(path)
     print(f"cov integrals N=8000 rows={plan.nrows}", flush=True)
     got = plan.integrals(torch.tensor(k, device="cuda"), torch.tensor(pk, device="cuda"), [len(k)]).cpu().numpy()
     plan.close()
