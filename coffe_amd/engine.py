@@ -26,6 +26,15 @@ def _need(t, shape, name):
         raise ValueError(f"{name}: shape {tuple(t.shape)} != {tuple(shape)}")
 
 
+def _raw_stream(device):
+    """The handle of torch's current stream on the device (0: the default stream)."""
+    import torch
+    global _raw_stream   # torch's own from the second call on
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+        (lambda d: torch.cuda.current_stream(d).cuda_stream)
+    return _raw_stream(device)
+
+
 class Engine:
     """One engine per device (stream + cache of spectrum-independent grid tables)."""
 
@@ -35,7 +44,7 @@ class Engine:
         check(self.L.coffe_engine_create(device, ctypes.byref(h)), "coffe_engine_create")
         self.h = h
         self.device = device
-        self._ext = None
+        self._switch = None
 
     def empty(self, *shapes):
         """New float64 tensors on the device, for a call that gets no stream.  With torch on its
@@ -44,19 +53,32 @@ class Engine:
         that stream's, so that the allocator hands their memory to no other stream while
         the engine still writes it."""
         import torch
-        if torch._C._cuda_getCurrentRawStream(self.device):
+        if _raw_stream(self.device):
             return [torch.empty(s, dtype=torch.float64, device=self.device) for s in shapes]
-        # the two switches by the stream's ids: half the time of the stream context manager
-        to, own = torch._C._cuda_setStream, self._ext
-        if own is None:
-            ext = torch.cuda.ExternalStream(self.L.coffe_engine_stream(self.h), device=self.device)
-            cur = torch.cuda.default_stream(self.device)
-            own = self._ext = (ext.stream_id, cur.stream_id, ext.device_index, ext.device_type)
-        to(stream_id=own[0], device_index=own[2], device_type=own[3])
+        fast = self._switch
+        if fast is None:
+            fast = self._switch = self._own_stream()
+        # the context manager also puts back another current device
+        if not fast or fast[1]() != self.device:
+            with torch.cuda.stream(self._ext):
+                return [torch.empty(s, dtype=torch.float64, device=self.device) for s in shapes]
+        to, _, own, default, index, kind = fast
+        to(stream_id=own, device_index=index, device_type=kind)
         try:
             return [torch.empty(s, dtype=torch.float64, device=self.device) for s in shapes]
         finally:
-            to(stream_id=own[1], device_index=own[2], device_type=own[3])
+            to(stream_id=default, device_index=index, device_type=kind)
+
+    def _own_stream(self):
+        """The engine's stream as torch's (_ext), and torch's switch of the current stream by ids with its
+        arguments, half the time of the context manager (() where torch has none)."""
+        import torch
+        self._ext = torch.cuda.ExternalStream(self.L.coffe_engine_stream(self.h), device=self.device)
+        to, device = getattr(torch._C, "_cuda_setStream", None), getattr(torch._C, "_cuda_getDevice", None)
+        if not to or not device:
+            return ()
+        return (to, device, self._ext.stream_id, torch.cuda.default_stream(self.device).stream_id, self._ext.device_index,
+                self._ext.device_type)
 
     def close(self):
         if self.h:
@@ -124,8 +146,7 @@ class Batch:
         _need(out, self._oshape, "out")
 
     def _stream(self):
-        import torch
-        return torch._C._cuda_getCurrentRawStream(self.engine.device)
+        return _raw_stream(self.engine.device)
 
     def _outputs(self, want, stream):
         """The outputs of `want` ((tensor or None, shape) each), allocated where the caller gave none."""

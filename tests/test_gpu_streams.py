@@ -72,3 +72,26 @@ def test_overlapping_passes_of_two_engines():
             assert float((g - w).norm()) <= 1e-12 * float(w.norm())
     for s in sets:
         s[0].close()
+
+
+def test_outputs_by_the_context_manager():
+    """the same outputs where the stream is switched by torch's context manager: allocated as the engine's, and
+    the caller's stream and device stay current"""
+    import torch
+    from coffe_amd.engine import Batch, Engine
+    k, p = spectrum(512)
+    kt, pt = torch.tensor(k, device="cuda"), torch.tensor(p, device="cuda")
+    eng = Engine(0)
+    b = Batch(eng, [512], [512], [k[0]], [k[-1]], [(0, 0)], np.array([30.0, 60.0]), 1, 1)
+    want = b.forward(kt, pt)[0].clone()
+    by_ids, eng._switch = eng._switch, ()
+    first = b.forward(kt, pt)[0]
+    ptr = first.data_ptr()
+    assert torch.equal(first, want)
+    del first
+    eng._switch = by_ids
+    again = b.forward(kt, pt)[0]   # the block of the engine's pool that the other way gave back
+    assert again.data_ptr() == ptr and torch.equal(again, want)
+    assert torch.cuda.current_device() == 0 and torch.cuda.current_stream() == torch.cuda.default_stream()
+    b.close()
+    eng.close()
