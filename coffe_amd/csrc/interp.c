@@ -5,6 +5,7 @@
  * (common.c:524-576, 704-710).  Out-of-range points give NaN.
  */
 #include <math.h>
+#include <stdlib.h>
 
 #include "coffe_engine.h"
 
@@ -28,29 +29,54 @@ static double slope(size_t n, const double *x, const double *y, long i)
     return (i == -1 || i == last + 1) ? 2.0 * m0 - m1 : 3.0 * m0 - 2.0 * m1;
 }
 
-/* the coefficients are made for the queries' intervals only: the API reads a few hundred values of
-   tables of 10^4 nodes */
+/* b, c, d of the interval between nodes of slopes m[2] (m[0] ... m[4]: the slopes of the intervals two before
+   to two after it) */
+static void coefs(const double *m, double h, double *b, double *c, double *d)
+{
+    const double ne = fabs(m[3] - m[2]) + fabs(m[1] - m[0]);
+    *b = m[2];
+    *c = *d = 0.0;
+    if (ne == 0.0) return;
+    const double nn = fabs(m[4] - m[3]) + fabs(m[2] - m[1]);
+    const double al = fabs(m[1] - m[0]) / ne;
+    const double tn = nn == 0.0 ? m[2] : (1.0 - fabs(m[2] - m[1]) / nn) * m[2] + fabs(m[2] - m[1]) / nn * m[3];
+    *b = (1.0 - al) * m[1] + al * m[2];
+    *c = (3.0 * m[2] - 2.0 * *b - tn) / h;
+    *d = (*b + tn - 2.0 * m[2]) / (h * h);
+}
+
+/*
+ * The coefficients of every interval beforehand where a third as many values as nodes are asked for, else
+ * those of the queries' intervals only (the API reads a few hundred values of tables of 10^4
+ * nodes): the same values.  A node costs 7 ns beforehand, a query 20 more without: 1000 queries of 6
+ * nodes 4.7 against 18 us, 100 of 10043 nodes 72 against 3.
+ */
 int coffe_akima_eval(size_t n, const double *x, const double *y, size_t nq, const double *xq, double *out)
 {
     if (n < 5 || !x || !y || (nq && (!xq || !out))) return COFFE_EINVAL;
+    double *tab = nq >= n / 3 ? (double *)malloc(sizeof(double) * (4 * n + 3)) : NULL;   /* NULL will do as well */
+    if (tab) {
+        double *bcd = tab + n + 3;
+        for (long i = -2; i <= (long)n; ++i) tab[i + 2] = slope(n, x, y, i);
+        for (size_t i = 0; i + 1 < n; ++i) coefs(tab + i, x[i + 1] - x[i], bcd + 3 * i, bcd + 3 * i + 1, bcd + 3 * i + 2);
+        for (size_t q = 0; q < nq; ++q) {
+            const double v = xq[q];
+            if (!(v >= x[0] && v <= x[n - 1])) { out[q] = NAN; continue; }
+            const size_t i = bsearch_lo(x, v, 0, n - 1);
+            const double dx = v - x[i], *k = bcd + 3 * i;
+            out[q] = y[i] + dx * (k[0] + dx * (k[1] + k[2] * dx));
+        }
+        free(tab);
+        return COFFE_OK;
+    }
     for (size_t q = 0; q < nq; ++q) {
         const double v = xq[q];
         if (!(v >= x[0] && v <= x[n - 1])) { out[q] = NAN; continue; }
         const long i = (long)bsearch_lo(x, v, 0, n - 1);
-        double m[5];   /* the slopes of intervals i - 2 ... i + 2 */
-        for (int j = 0; j < 5; ++j) m[j] = slope(n, x, y, i - 2 + j);
-        const double ne = fabs(m[3] - m[2]) + fabs(m[1] - m[0]);
-        double b = m[2], c = 0.0, d = 0.0;
-        if (ne != 0.0) {
-            const double h = x[i + 1] - x[i];
-            const double nn = fabs(m[4] - m[3]) + fabs(m[2] - m[1]);
-            const double al = fabs(m[1] - m[0]) / ne;
-            const double tn = nn == 0.0 ? m[2] : (1.0 - fabs(m[2] - m[1]) / nn) * m[2] + fabs(m[2] - m[1]) / nn * m[3];
-            b = (1.0 - al) * m[1] + al * m[2];
-            c = (3.0 * m[2] - 2.0 * b - tn) / h;
-            d = (b + tn - 2.0 * m[2]) / (h * h);
-        }
         const double dx = v - x[i];
+        double m[5], b, c, d;   /* m: the slopes of intervals i - 2 ... i + 2 */
+        for (int j = 0; j < 5; ++j) m[j] = slope(n, x, y, i - 2 + j);
+        coefs(m, x[i + 1] - x[i], &b, &c, &d);
         out[q] = y[i] + dx * (b + dx * (c + d * dx));
     }
     return COFFE_OK;
