@@ -1778,16 +1778,19 @@ int coffe_integral_tables(int ntab, const int *n, const int *l, size_t N, const 
     if (!e) return COFFE_ENODEVICE;
     hipSetDevice(e->device);
     ce_grid *g = NULL;
-    int st = grid_get(e, (int)N, kmin, kmax, kmin, 1.0, ntab, td, &g);
-    if (st != COFFE_OK || g->rp.npass == 0) {
-        /* lengths outside the LDS kernels, or more than two biases: table by table */
-        if (st != COFFE_OK && st != COFFE_EUNSUPPORTED) return st;
+    ce_radix_plan rp;
+    /* lengths outside the LDS kernels, or more than two biases: table by table (a grid of all of them would
+       stay on the engine unused) */
+    int st = N > 16384 ? COFFE_EUNSUPPORTED : ce_radix_schedule((int)N / 2, &rp);
+    if (st == COFFE_OK) st = grid_get(e, (int)N, kmin, kmax, kmin, 1.0, ntab, td, &g);
+    if (st == COFFE_EUNSUPPORTED) {
         for (int t = 0; t < ntab; ++t) {
             st = coffe_integral_table(n[t], l[t], N, k, pk, nin, kmin, kmax, out_x, out_y + (N + nodes) * (size_t)t);
             if (st != COFFE_OK) return st;
         }
         return COFFE_OK;
     }
+    if (st != COFFE_OK) return st;
     const int M = (int)N / 2;
     const int64_t n_in1 = (int64_t)nin, n_fft1 = (int64_t)N;
     const int len = chunk_len(n_in1, n_fft1, chunk_points(1, &n_in1, &n_fft1));

@@ -41,3 +41,19 @@ def test_refused_as_one_at_a_time(engine):
                 call(*args)
             codes.append(err.value.code)
         assert codes[0] == codes[1], args
+
+
+def test_no_grid_of_all_tables_where_they_go_one_by_one(engine):
+    """at a length outside the LDS kernels the tables go one at a time, with their own grids: the joint call
+    adds nothing to the device memory that those calls have taken"""
+    import torch
+    from coffe_amd.engine import integral_table, integral_tables
+    k, p = spectrum(300)
+    tables, N = TABLES[:3], 300000
+    want = [integral_table(*t, k, p, N)[1] for t in tables]
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    got = integral_tables(tables, k, p, N)
+    assert free - torch.cuda.mem_get_info()[0] < 1 << 20
+    for t, w in zip(tables, want):
+        assert np.array_equal(got[t][1], w)
