@@ -304,46 +304,6 @@ static void grid_to_dev(const ce_grid *g, ce_grid_dev *d)
 
 /* ---- engine ----------------------------------------------------------------- */
 
-/*
- * Streams of engines that are gone, for the next ones: callers keep memory by the stream it was used
- * on (torch's allocator: the outputs of Engine.empty), and what a dropped stream leaves in such a
- * pool no other stream gets.  At most IDLE_STREAMS; idle, since their engines waited for them.
- */
-#define IDLE_STREAMS 8
-static struct {
-    hipStream_t stream;
-    int device;
-} g_idle[IDLE_STREAMS];
-static int g_nidle = 0;
-static pthread_mutex_t g_idle_lock = PTHREAD_MUTEX_INITIALIZER;
-
-/* a stream on the current device, the last one given back first */
-static int stream_take(int device, hipStream_t *s)
-{
-    pthread_mutex_lock(&g_idle_lock);
-    for (int i = g_nidle - 1; i >= 0; --i)
-        if (g_idle[i].device == device) {
-            *s = g_idle[i].stream;
-            memmove(&g_idle[i], &g_idle[i + 1], sizeof(g_idle[0]) * (size_t)(--g_nidle - i));
-            pthread_mutex_unlock(&g_idle_lock);
-            return COFFE_OK;
-        }
-    pthread_mutex_unlock(&g_idle_lock);
-    return hip_ok(hipStreamCreate(s));
-}
-
-static void stream_give(int device, hipStream_t s)
-{
-    pthread_mutex_lock(&g_idle_lock);
-    const int kept = hipStreamQuery(s) == hipSuccess && g_nidle < IDLE_STREAMS;
-    if (kept) {
-        g_idle[g_nidle].stream = s;
-        g_idle[g_nidle++].device = device;
-    }
-    pthread_mutex_unlock(&g_idle_lock);
-    if (!kept) hipStreamDestroy(s);
-}
-
 int coffe_engine_create(int device, coffe_engine **out)
 {
     if (!out) return COFFE_EINVAL;
@@ -360,14 +320,14 @@ int coffe_engine_create(int device, coffe_engine **out)
         if (v == 256 || v == 512 || v == 1024) e->threads = v;
     }
     pthread_mutex_init(&e->lock, NULL);
-    if (hipSetDevice(device) != hipSuccess || stream_take(device, &e->stream) != COFFE_OK) {
+    if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&e->stream) != hipSuccess) {
         free(e);
         return COFFE_EDEVICE;
     }
     if (hipEventCreateWithFlags(&e->ev_scratch, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&e->ev_stage[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&e->ev_stage[1], hipEventDisableTiming) != hipSuccess) {
-        stream_give(device, e->stream);
+        hipStreamDestroy(e->stream);
         free(e);
         return COFFE_EDEVICE;
     }
@@ -391,7 +351,7 @@ void coffe_engine_destroy(coffe_engine *e)
         hipEventDestroy(e->ev_stage[i]);
     }
     hipEventDestroy(e->ev_scratch);
-    stream_give(e->device, e->stream);
+    hipStreamDestroy(e->stream);
     pthread_mutex_destroy(&e->lock);
     free(e);
 }
