@@ -27,10 +27,11 @@
 //
 // Operand loads: an instruction reads 16 rows x 4 contracted elements, one per lane (row q =
 // lane % 16, elements by g = lane / 16), and rows of an (m, t) array are far apart, which costs the
-// L1 an access per lane (measured 54 per load instruction; k_cov_few was bound by them: 207
-// against 80 us).  The contracted index may run in any order, so the tables and the diagonals
-// are stored as fragments: 16 x 16 blocks in the order [half][lane][2], lane (q, g) holding
-// t = 4 g ... 4 g + 3 of its row in two 16-byte loads that read 1 KB each.
+// L1 an access per lane (k_cov_few was bound by them: 214 us, 130 with fragments; k_cov_many's
+// loads take 16 accesses now, the least for 1 KB).  The contracted index may run in any order, so
+// the tables and the diagonals are stored as fragments: 16 x 16 blocks in the order
+// [half][lane][2], lane (q, g) holding t = 4 g ... 4 g + 3 of its row in two 16-byte loads that
+// read 1 KB each.  The transposes read plain rows (k_cov_unfold) with their lanes along t.
 #include <hip/hip_runtime.h>
 
 #include <utility>

@@ -13,8 +13,9 @@
 //   - single: the two mixed separations are closest at x = chi1 c / chi2 and chi2 c /
 //     chi1; [0, 1] is cut there (and halfway between), each piece mapped by x = centre
 //     +- s sinh(u) about its nearer centre (s the ridge width), u Gauss-Legendre.
-// Every lookup is an Akima interpolation of raw nodes (ce::akima_general) and the
-// renormalisation grid a GSL-style bicubic, as the reference's splines.
+// Every lookup is the Akima interpolation of the raw nodes (as ce::akima_general; the interval's
+// coefficients are made once per call, k_intg_coef) and the renormalisation grid a GSL-style
+// bicubic, as the reference's splines.
 
 #include <hip/hip_runtime.h>
 

@@ -51,7 +51,10 @@ class Engine:
         default stream such a call runs on the engine's own stream (which the default
         stream's work waits for and which waits for it); the tensors are then allocated as
         that stream's, so that the allocator hands their memory to no other stream while
-        the engine still writes it."""
+        the engine still writes it.  (What the allocator keeps for a closed engine's stream it gives
+        back in torch.cuda.empty_cache(), or before it runs out of memory.  Keeping the streams
+        for the next engines instead cost their overlap: streams are spread over the hardware
+        queues when they are made, and reused ones met on one.)"""
         import torch
         if _raw_stream(self.device):
             return [torch.empty(s, dtype=torch.float64, device=self.device) for s in shapes]
