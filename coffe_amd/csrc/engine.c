@@ -943,7 +943,7 @@ static int scratch_reserve(coffe_engine *e, size_t bytes, hipStream_t s)
     hipFree(e->d_scratch);
     e->d_scratch = NULL;
     e->scratch_bytes = 0;
-    if (injected_failure() || hipMalloc(&e->d_scratch, bytes) != hipSuccess) { e->d_scratch = NULL; return COFFE_ENOMEM; }
+    if (dev_alloc(&e->d_scratch, bytes) != COFFE_OK) return COFFE_ENOMEM;
     e->scratch_bytes = bytes;
     return COFFE_OK;
 }
@@ -1795,8 +1795,13 @@ int coffe_integral_tables(int ntab, const int *n, const int *l, size_t N, const 
         hipHostFree(e->h_down);
         e->h_down = NULL;
         e->down_bytes = 0;
-        if (injected_failure() || hipHostMalloc(&e->h_down, down, hipHostMallocDefault) != hipSuccess) st = COFFE_ENOMEM;
-        else e->down_bytes = down;
+        if (injected_failure() || hipHostMalloc(&e->h_down, down, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            e->h_down = NULL;
+            st = COFFE_ENOMEM;
+        } else {
+            e->down_bytes = down;
+        }
     }
     if (st == COFFE_OK) {
         char *d = (char *)e->d_scratch;
