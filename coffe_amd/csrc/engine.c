@@ -382,7 +382,7 @@ coffe_engine *coffe_engine_default(void)
 
 struct coffe_batch {
     coffe_engine *e;
-    int nspec, ntab, nsep, nz, nl, nq, nunit, ngrid, nchunk, nadj;
+    int nspec, ntab, nsep, nz, nl, nq, nunit, ngrid, nchunk, adj0, nadj;
     int max_M, max_N, threads;
     int64_t total_in;
     ce_grid **grids;
@@ -392,7 +392,7 @@ struct coffe_batch {
     ce_grid_dev *d_grids;
     ce_table_desc *d_tabs;
     ce_unit_dev *d_units;
-    ce_chunk_dev *d_chunks; /* the resample chunks, then those of k_spline_adj */
+    ce_chunk_dev *d_chunks; /* the resample chunks; those of k_spline_adj from adj0 on (0: the same) */
     int32_t *d_ranges; /* resample index ranges per chunk (4 each), from the prepare stage */
     int32_t *d_packs;  /* table workgroups: first unit, unit count, groups, 0 */
     int npack, lt_off;
@@ -633,9 +633,10 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
                 ++c;
             }
         }
-        b->nadj = 0;
-        for (c = 0; c < b->nchunk && st == COFFE_OK;) {
-            ce_chunk_dev *q = &chunks[b->nchunk + b->nadj++];
+        b->adj0 = merge > 1 ? b->nchunk : 0;
+        b->nadj = merge > 1 ? 0 : b->nchunk;
+        for (c = 0; merge > 1 && c < b->nchunk && st == COFFE_OK;) {
+            ce_chunk_dev *q = &chunks[b->adj0 + b->nadj++];
             *q = chunks[c];
             const int m = adj_merged(q->b - q->a, merge);
             while (++c < b->nchunk && chunks[c].a != 0 && c < q->id + m) {
@@ -658,7 +659,7 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_grids, sizeof(ce_grid_dev) * (size_t)b->ngrid);
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_tabs, sizeof(ce_table_desc) * (size_t)ntab);
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_units, sizeof(ce_unit_dev) * (size_t)b->nunit);
-    if (st == COFFE_OK) st = dev_alloc((void **)&b->d_chunks, sizeof(ce_chunk_dev) * (size_t)(b->nchunk + b->nadj));
+    if (st == COFFE_OK) st = dev_alloc((void **)&b->d_chunks, sizeof(ce_chunk_dev) * (size_t)(b->adj0 + b->nadj));
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_ranges, 4 * sizeof(int32_t) * (size_t)b->nchunk);
     if (st == COFFE_OK) st = hip_ok(hipMemset(b->d_ranges, 0, 4 * sizeof(int32_t) * (size_t)b->nchunk));
     if (st == COFFE_OK) st = dev_alloc((void **)&b->d_sidx, sizeof(int32_t) * (size_t)b->ngrid * (size_t)nsep);
@@ -735,7 +736,7 @@ int coffe_batch_create(coffe_engine *e, int nspec, const int64_t *n_in, const in
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_grids, hg, sizeof(ce_grid_dev) * (size_t)b->ngrid, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_tabs, tabs, sizeof(ce_table_desc) * (size_t)ntab, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_units, units, sizeof(ce_unit_dev) * (size_t)b->nunit, hipMemcpyHostToDevice, s));
-    if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_chunks, chunks, sizeof(ce_chunk_dev) * (size_t)(b->nchunk + b->nadj),
+    if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_chunks, chunks, sizeof(ce_chunk_dev) * (size_t)(b->adj0 + b->nadj),
                                                       hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_sidx, sidx, sizeof(int32_t) * (size_t)b->ngrid * (size_t)nsep, hipMemcpyHostToDevice, s));
     if (st == COFFE_OK) st = hip_ok(hipMemcpyAsync(b->d_sep, sep, sizeof(double) * (size_t)nsep, hipMemcpyHostToDevice, s));
@@ -783,7 +784,7 @@ int coffe_batch_adj_c2r(coffe_batch *b, void *stream)
 int coffe_batch_spline_adj(coffe_batch *b, const double *d_k, double *d_gpk, void *stream)
 {
     if (!b || !d_k || !d_gpk) return COFFE_EINVAL;
-    return ce_launch_spline_adj(pick_stream(b, stream), b->nadj, b->d_chunks + b->nchunk, b->d_spec, b->d_grids, d_k,
+    return ce_launch_spline_adj(pick_stream(b, stream), b->nadj, b->d_chunks + b->adj0, b->d_spec, b->d_grids, d_k,
                                 b->d_ws, d_gpk, b->d_ranges)
                ? COFFE_EDEVICE
                : COFFE_OK;
@@ -827,7 +828,7 @@ int coffe_batch_prepare_adj(coffe_batch *b, const double *d_k, const double *d_p
     if (ce_launch_adj_c2r(s, b->nspec, b->d_spec, b->d_grids, b->d_tabs, b->ntab, b->nq, b->d_ws, b->d_xb,
                           b->threads, b->max_M, NULL, NULL, NULL, 0, 0, 0))
         return COFFE_EDEVICE;
-    return ce_launch_spline_adj(s, b->nadj, b->d_chunks + b->nchunk, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk,
+    return ce_launch_spline_adj(s, b->nadj, b->d_chunks + b->adj0, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk,
                                 b->d_ranges)
                ? COFFE_EDEVICE
                : COFFE_OK;
@@ -865,7 +866,7 @@ int coffe_batch_vjp(coffe_batch *b, const double *d_k, const double *d_pk, const
     if (ce_launch_adj_c2r(s, b->nspec, b->d_spec, b->d_grids, b->d_tabs, b->ntab, b->nq, b->d_ws, b->d_xb,
                           b->threads, b->max_M, d_A, itab, d_out, b->nz, b->nl, b->nsep))
         return COFFE_EDEVICE;
-    return ce_launch_spline_adj(s, b->nadj, b->d_chunks + b->nchunk, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk,
+    return ce_launch_spline_adj(s, b->nadj, b->d_chunks + b->adj0, b->d_spec, b->d_grids, d_k, b->d_ws, d_gpk,
                                 b->d_ranges)
                ? COFFE_EDEVICE
                : COFFE_OK;
